@@ -18,9 +18,10 @@
 //    Output X[J][k][a] (a fastest).  Workgroups of one vector are placed on
 //    one XCD so that the two reads of every packed element (as row and as
 //    transposed column) share that XCD's L2.
-//  * SYRK: a workgroup owns one TMxTM tile (A >= B) of K and a slice of the
+//  * SYRK: a workgroup owns one tile (A >= B) of K and a slice of the
 //    vectors; it contracts over (J, k in the density's bank columns) with
-//    v_mfma_f64_16x16x4f64 and writes an FP64 partial tile.  A final
+//    MFMA (FP64: k_syrk64, operands straight from memory into registers) and
+//    writes an FP64 partial tile.  A final
 //    deterministic reduction sums the slices into LT storage.
 #include <type_traits>
 
@@ -70,6 +71,22 @@ struct SyrkSets {
   int nsplit[kMaxSets];
   int item0[kMaxSets + 1];
   int64_t kbase[kMaxSets];
+};
+
+// The same for the FP64 SYRK (k_syrk64): 64x64 tiles only, the off-diagonal and
+// the diagonal tiles sliced separately (nsf / nsd slices), because a diagonal
+// tile costs 10 MFMAs per step where an off-diagonal one costs 16.  Set d owns
+// the blocks item0[d] .. item0[d+1]-1 (multiples of 8: block b runs on XCD
+// b % 8) and the partial tiles at kf[d] (off-diagonal) and kd[d] (diagonal).
+constexpr int kT64 = 64;
+constexpr int kSlot64 = kT64 * kT64;
+struct Syrk64Sets {
+  int n;
+  int off[kMaxSets];
+  int opad[kMaxSets];
+  int nsf[kMaxSets], nsd[kMaxSets];
+  int item0[kMaxSets + 1];
+  int64_t kf[kMaxSets], kd[kMaxSets];
 };
 
 __device__ inline int find_set(const SyrkSets &sets, int b) {
@@ -571,6 +588,193 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
       }
 }
 
+// ---- FP64 SYRK -------------------------------------------------------------
+// Workgroup = (one 64x64 tile A >= B of K, one slice of the chunk's vectors);
+// its four waves share the tile and take the slice's 4-row contraction steps
+// in turn (wave w: steps w, w+4, ...), each accumulating the whole tile, and
+// are summed through LDS once at the end.  A step is four rows of X (one
+// vector, four bank columns: opad is a multiple of 4); lane l = 16 g + m loads
+// columns 32 i + 2 m, 2 m + 1 (i = 0, 1) of row g of both tile sides, 16 bytes
+// each, and these ARE the MFMA operands: tile (i, c) holds the columns
+// 32 i + 2 m + c.  So no LDS, no barrier and no address arithmetic sits
+// between the loads and the MFMAs: per step 4 loads and 16 MFMAs of 64 cycles,
+// kSyrkD steps of loads in flight per wave, two waves per SIMD.
+// Bound by the matrix cores and the clock they leave: at n=1200 nchol=6000
+// nocc=150 they are busy 88% of the cycles and the clock settles near 2.1 GHz
+// (63 TFLOP/s executed; the card's own large FP64 product reaches 70).  The
+// LDS-staged 128x128 tile it replaces ran the same shape in 27.3 ms (now 21.8)
+// and n=536 nchol=2510 nocc=98 in 2.18 ms (now 1.26): whole 128-wide diagonal
+// and edge tiles, whose idle waves held their workgroup's slots, cost a third.
+// SH: the tile row holds rows in its first 32 columns only (ragged n); DG:
+// diagonal tile, its 10 lower MFMA tiles ((i, 0) x (i, 1) is the transpose of
+// (i, 1) x (i, 0) and is read from there).
+constexpr int kSyrkD = 4;
+
+// Slot layout of a partial tile: MFMA tile q = 4 (2 i + c) + 2 i' + c', result
+// register r, lane: position 256 q + 64 r + lane.
+__device__ __forceinline__ int slot64_pos(int al, int bl) {
+  const int m = (al >> 1) & 15;  // row index inside MFMA tile (i, c)
+  const int q = 4 * (2 * (al >> 5) + (al & 1)) + 2 * (bl >> 5) + (bl & 1);
+  return 256 * q + 64 * (m >> 2) + 16 * (m & 3) + ((bl >> 1) & 15);
+}
+
+template <bool SH, bool DG>
+__device__ __forceinline__ void syrk64_tile(const double *__restrict__ X, int n_pad, int ldc, int off,
+                                            int q4, int64_t ja, int nst, int A, int B, double *__restrict__ kp,
+                                            double (*__restrict__ red)[4][4][64]) {
+  constexpr int HA = SH ? 1 : 2, HB = (SH && DG) ? 1 : 2;  // 32-column halves of the two sides
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  v4d acc[2 * HA][2 * HB];
+#pragma unroll
+  for (int i = 0; i < 2 * HA; ++i)
+#pragma unroll
+    for (int j = 0; j < 2 * HB; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
+  auto used = [](int i, int j) { return !DG || (i >> 1) > (j >> 1) || ((i >> 1) == (j >> 1) && i >= j); };
+  // steps of this wave and the row pointer of its next load (uniform)
+  const int ns = nst > w ? (nst - w + 3) / 4 : 0;
+  if (ns > 0) {
+    int kk = w % q4, left = ns;
+    const int64_t row4 = 4 * int64_t(n_pad);
+    const double *p = X + ((ja + w / q4) * ldc + off) * int64_t(n_pad) + kk * row4;
+    const int64_t wrap = (int64_t(ldc) - 4 * q4) * n_pad;  // from one vector's bank columns to the next's
+    const uint32_t la = uint32_t((lane >> 4) * n_pad + A * kT64 + 2 * (lane & 15)) * 8u;
+    const uint32_t lb = uint32_t((lane >> 4) * n_pad + B * kT64 + 2 * (lane & 15)) * 8u;
+    v2d ra[kSyrkD][HA], rb[kSyrkD][DG ? 1 : 2];
+    // every call issues the same loads; past the last step the pointer stays
+    auto load = [&](v2d(&a)[HA], v2d(&b)[DG ? 1 : 2]) __attribute__((always_inline)) {
+      const char *c = reinterpret_cast<const char *>(p);
+#pragma unroll
+      for (int i = 0; i < HA; ++i) a[i] = *reinterpret_cast<const v2d *>(c + la + 256 * i);
+      if constexpr (!DG) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) b[i] = *reinterpret_cast<const v2d *>(c + lb + 256 * i);
+      }
+      if (--left > 0) {
+        p += 4 * row4;
+        kk += 4;
+        while (kk >= q4) {
+          kk -= q4;
+          p += wrap;
+        }
+      }
+    };
+    auto mul = [&](const v2d(&a)[HA], const v2d(&b)[DG ? 1 : 2]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 2 * HA; ++i)
+#pragma unroll
+        for (int j = 0; j < 2 * HB; ++j)
+          if (used(i, j)) {
+            double bv;
+            if constexpr (DG) bv = a[j >> 1][j & 1];
+            else bv = b[j >> 1][j & 1];
+            acc[i][j] = F64::mma(a[i >> 1][i & 1], bv, acc[i][j]);
+          }
+    };
+#pragma unroll
+    for (int s = 0; s < kSyrkD; ++s) load(ra[s], rb[s]);
+    int t = 0;
+    for (; t + kSyrkD <= ns; t += kSyrkD) {
+#pragma unroll
+      for (int s = 0; s < kSyrkD; ++s) {
+        mul(ra[s], rb[s]);
+        __builtin_amdgcn_sched_barrier(0);
+        load(ra[s], rb[s]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < kSyrkD - 1; ++s)
+      if (t + s < ns) mul(ra[s], rb[s]);
+  }
+  // sum of the four waves in wave order: MFMA tiles four at a time through
+  // LDS, wave w finishing the w-th of them
+  constexpr int NT = 4 * HA * HB;
+#pragma unroll
+  for (int q0 = 0; q0 < NT; q0 += 4) {
+    if (q0) __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = (q0 + u) / (2 * HB), j = (q0 + u) % (2 * HB);
+      if (used(i, j)) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[w][u][r][lane] = acc[i][j][r];
+      }
+    }
+    __syncthreads();
+    const int i = (q0 + w) / (2 * HB), j = (q0 + w) % (2 * HB);
+    if (used(i, j)) {
+      double *__restrict__ out = kp + 256 * (4 * i + j) + lane;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        double v = red[0][w][r][lane];
+#pragma unroll
+        for (int u = 1; u < 4; ++u) v += red[u][w][r][lane];
+        out[64 * r] = v;
+      }
+    }
+  }
+}
+
+__global__ __launch_bounds__(kThreads, 2) void k_syrk64(const double *__restrict__ X, int n, int n_pad,
+                                                     int ldc, int64_t jc, int T, const Syrk64Sets sets,
+                                                     double *__restrict__ kpart, int chunk, const Screen sc) {
+  __shared__ double red[4][4][4][64];
+  int set = 0;
+  while (set + 1 < sets.n && int(blockIdx.x) >= sets.item0[set + 1]) ++set;
+  const int local = blockIdx.x - sets.item0[set], x = local & 7, li = local >> 3;
+  const int nf = T * (T - 1) / 2;
+  const int nsf = sets.nsf[set], nsd = sets.nsd[set];
+  // XCD x takes the x-th eighth of the diagonal items (first: their slices are
+  // the longer ones) and of the off-diagonal ones, both slice by slice, so the
+  // tiles that read the same rows of X run on one XCD
+  const int nd8 = (nsd * T + 7) / 8, nf8 = (nsf * nf + 7) / 8;
+  const bool diag = li < nd8;
+  const int l = diag ? x * nd8 + li : x * nf8 + (li - nd8);
+  if (l >= (diag ? nsd * T : nsf * nf)) return;
+  int A, B, s, ns;
+  double *kp;
+  if (diag) {
+    s = l / T;
+    A = B = l - s * T;
+    ns = nsd;
+    kp = kpart + sets.kd[set] + (int64_t(chunk) * nsd * T + l) * kSlot64;
+  } else {
+    s = l / nf;
+    const int t = l - s * nf;
+    ns = nsf;
+    A = int((sqrt(8.0 * t + 1.0) + 1.0) * 0.5);
+    while (A * (A - 1) / 2 > t) --A;
+    while (A * (A + 1) / 2 <= t) ++A;
+    B = t - A * (A - 1) / 2;
+    kp = kpart + sets.kf[set] + (int64_t(chunk) * nsf * nf + l) * kSlot64;
+  }
+  const int64_t jper = (jc + ns - 1) / ns;
+  const int64_t ja = s * jper, jz = min(jc, ja + jper);
+  const int q4 = sets.opad[set] / 4;
+  const int nst = int(jz > ja ? jz - ja : 0) * q4;  // < 2^29, checked on the host
+  if (sc.xn2 && nst > 0) {  // screened: |K_ab| of this slice <= sum_J ||X^J_A||_F ||X^J_B||_F
+    double bound = 0.0;
+    for (int64_t J = ja; J < jz; ++J) {
+      const double *__restrict__ r = sc.xn2 + (int64_t(set) * jc + J) * sc.nstrip;
+      bound += sqrt(r[A] * r[B]);
+    }
+    if (bound < sc.tau) {
+      for (int e = threadIdx.x; e < kSlot64; e += kThreads) kp[e] = 0.0;
+      if (threadIdx.x == 0) atomicAdd(sc.cnt, 1ull);
+      return;
+    }
+  }
+  const bool half = n - A * kT64 <= 32;
+  const int off = sets.off[set];
+  if (diag) {
+    if (half) syrk64_tile<true, true>(X, n_pad, ldc, off, q4, ja, nst, A, B, kp, red);
+    else syrk64_tile<false, true>(X, n_pad, ldc, off, q4, ja, nst, A, B, kp, red);
+  } else {
+    if (half) syrk64_tile<true, false>(X, n_pad, ldc, off, q4, ja, nst, A, B, kp, red);
+    else syrk64_tile<false, false>(X, n_pad, ldc, off, q4, ja, nst, A, B, kp, red);
+  }
+}
+
 // ---- screening norms -------------------------------------------------------
 __device__ inline double block_sum256(double x, double *red) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -999,38 +1203,74 @@ __global__ __launch_bounds__(kThreads) void k_syrk_b3(
       }
 }
 
-// klt[d*ldk + a*(a+1)/2 + b] = sum_s kpart[kbase[d] + (s*ntiles + tile(a,b))*TM*TM
-//                                           + (a%TM)*TM + b%TM],  s over (chunk, slice)
-// grid = (n rows a, nsets), block 256.
-__global__ void k_reduce_k(const double *__restrict__ kpart_all, int n, int tm, int ntiles,
-                           const SyrkSets sets, int nchunk, double *__restrict__ klt,
-                           int64_t ldk) {
-  const int a = blockIdx.x, d = blockIdx.y;
-  const int A = a / tm, al = a % tm;
-  const int nsplit = sets.nsplit[d] * nchunk;  // slots (chunk, slice), chunk-major
-  const double *__restrict__ kpart = kpart_all + sets.kbase[d];
-  double *__restrict__ out = klt + d * ldk + tri0(a);
-  for (int b = threadIdx.x; b <= a; b += blockDim.x) {
-    if (nsplit == 0) {
-      out[b] = 0.0;
-      continue;
-    }
-    const int B = b / tm, bl = b % tm;
-    const int64_t t = int64_t(A) * (A + 1) / 2 + B;
-    const double *__restrict__ src = kpart + t * tm * tm + al * tm + bl;
-    const int64_t stride = int64_t(ntiles) * tm * tm;
-    double s = 0.0;
-    int k = 0;
-    for (; k + 8 <= nsplit; k += 8) {  // eight loads in flight, summed in slot order
-      double v[8];
+// Sum of every fourth value, from the q-th, of cnt values `stride` apart, eight
+// loads in flight, in a fixed order.
+__device__ __forceinline__ double strided_sum(const double *__restrict__ src, int64_t stride, int cnt, int q) {
+  double s = 0.0;
+  int k = q;
+  for (; k + 28 < cnt; k += 32) {
+    double v[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = src[(k + u) * stride];
+    for (int u = 0; u < 8; ++u) v[u] = src[(k + 4 * u) * stride];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) s += v[u];
-    }
-    for (; k < nsplit; ++k) s += src[k * stride];
-    out[b] = s;
+    for (int u = 0; u < 8; ++u) s += v[u];
   }
+  for (; k < cnt; k += 4) s += src[k * stride];
+  return s;
+}
+
+// klt[d*ldk + a*(a+1)/2 + b] = sum over the partial tiles of (a, b): the FP64
+// chunks' (k_syrk64, nchunk64 of them, slots of sets64) and the reduced-
+// precision chunks' (nchunk of them, slots of sets, row-major TM x TM tiles).
+// grid = (n rows a, column blocks of 64, nsets), block 256: thread (q, column)
+// sums every fourth slot, so that a small K, which has few rows to run side by
+// side, is not one long chain of loads per element.
+__global__ __launch_bounds__(kThreads) void k_reduce_k(const double *__restrict__ kpart64, const Syrk64Sets sets64,
+                                                      int nchunk64, const double *__restrict__ kpart_all, int tm,
+                                                      const SyrkSets sets, int nchunk, int n,
+                                                      double *__restrict__ klt, int64_t ldk) {
+  __shared__ double red[3][64];
+  const int a = blockIdx.x, d = blockIdx.z;
+  const int cb = threadIdx.x & 63, q = threadIdx.x >> 6;
+  const int b = blockIdx.y * 64 + cb;
+  if (int(blockIdx.y) * 64 > a) return;
+  double s = 0.0;
+  if (b <= a) {
+    if (nchunk64 > 0) {
+      const int T = (n + kT64 - 1) / kT64;
+      const int A = a / kT64, B = b / kT64;
+      int al = a % kT64, bl = b % kT64;
+      const double *src;
+      int64_t stride;
+      int cnt;
+      if (A == B) {
+        if ((al >> 5) == (bl >> 5) && !(al & 1) && (bl & 1)) {  // stored as its transpose
+          const int t = al;
+          al = bl;
+          bl = t;
+        }
+        cnt = sets64.nsd[d] * nchunk64;
+        stride = int64_t(T) * kSlot64;
+        src = kpart64 + sets64.kd[d] + int64_t(A) * kSlot64;
+      } else {
+        const int nf = T * (T - 1) / 2;
+        cnt = sets64.nsf[d] * nchunk64;
+        stride = int64_t(nf) * kSlot64;
+        src = kpart64 + sets64.kf[d] + (int64_t(A) * (A - 1) / 2 + B) * kSlot64;
+      }
+      s = strided_sum(src + slot64_pos(al, bl), stride, cnt, q);
+    }
+    if (nchunk > 0) {
+      const int ntile1 = (n + tm - 1) / tm, ntiles = ntile1 * (ntile1 + 1) / 2;
+      const int A = a / tm, B = b / tm;
+      const double *src = kpart_all + sets.kbase[d] + (int64_t(A) * (A + 1) / 2 + B) * tm * tm +
+                          int64_t(a % tm) * tm + b % tm;
+      s += strided_sum(src, int64_t(ntiles) * tm * tm, sets.nsplit[d] * nchunk, q);
+    }
+  }
+  if (q > 0) red[q - 1][cb] = s;
+  __syncthreads();
+  if (q == 0 && b <= a) klt[d * ldk + tri0(a) + b] = ((s + red[0][cb]) + red[1][cb]) + red[2][cb];
 }
 
 template <class P, int OT, int TA, int BK>
@@ -1106,14 +1346,22 @@ void ht_dispatch(Context *c, int ot, const typename P::T *L, const typename P::T
   }
 }
 
-template <class P>
-void syrk_launch(Context *c, int tm, int items, const typename P::T *X, int ldc, int64_t jn,
-                 int ntiles, const SyrkSets &sets, double *kpart, int chunk) {
+void syrk_launch64(Context *c, const double *X, int ldc, int64_t jn, const Syrk64Sets &sets, double *kpart,
+                   int chunk) {
+  const int T = int(ceil_div(c->n, kT64));
+  hipLaunchKernelGGL(k_syrk64, dim3(unsigned(sets.item0[sets.n])), dim3(kThreads), 0, c->stream, X, c->n, c->n_pad,
+                     ldc, jn, T, sets, kpart, chunk, c->scr);
+  if (c->scr.xn2)
+    for (int d = 0; d < sets.n; ++d) c->k_items += int64_t(sets.nsd[d]) * T + int64_t(sets.nsf[d]) * T * (T - 1) / 2;
+}
+
+void syrk_launch32(Context *c, int tm, int items, const float *X, int ldc, int64_t jn, int ntiles,
+                   const SyrkSets &sets, double *kpart, int chunk) {
   if (tm == 128)
-    hipLaunchKernelGGL((k_syrk<P, 128, 16>), dim3(unsigned(items)), dim3(kThreads), 0, c->stream, X,
+    hipLaunchKernelGGL((k_syrk<F32, 128, 16>), dim3(unsigned(items)), dim3(kThreads), 0, c->stream, X,
                        c->n_pad, ldc, jn, ntiles, sets, kpart, chunk, c->scr);
   else
-    hipLaunchKernelGGL((k_syrk<P, 64, 32>), dim3(unsigned(items)), dim3(kThreads), 0, c->stream, X,
+    hipLaunchKernelGGL((k_syrk<F32, 64, 32>), dim3(unsigned(items)), dim3(kThreads), 0, c->stream, X,
                        c->n_pad, ldc, jn, ntiles, sets, kpart, chunk, c->scr);
   if (c->scr.xn2) c->k_items += items;
 }
@@ -1237,6 +1485,48 @@ int ensure_l32(Context *c) {
   return hip_check(c, hipGetLastError(), "L to FP32");
 }
 
+// Slices of the FP64 SYRK (k_syrk64) for chunks of jc vectors: fills sets and
+// returns the doubles its partial tiles take over nchunk chunks.
+// Workgroups per launch: whole rounds of two per CU, as many (up to 64) as leave
+// each of a workgroup's four waves about 160 steps (a step is four rows, 16
+// MFMAs); a diagonal tile (10 MFMAs per step) gets 10/16 of the slices.  The
+// tiles of one slice drift apart as they run, and once they are further apart
+// than the XCD's L2 holds, each fetches X from HBM by itself; short slices bound
+// the drift until the partial tiles' traffic takes over.  Measured (workgroups
+// per launch: 1024, 4096, 16384, 32768): n=512 nchol=2048 nocc=64 0.58, 0.61,
+// 0.73, 0.95 ms; n=800 nchol=3600 nocc=150 6.5, 6.1, 5.7, 5.8 ms; n=1200
+// nchol=6000 nocc=150 22.9, 21.4, 22.4, 21.5 ms.
+int64_t plan_syrk64(const Context *c, int32_t nk, const int32_t *nocc, const std::vector<int> &off,
+                    const std::vector<int> &opad, int64_t jc, int64_t work, int64_t nchunk, Syrk64Sets *out) {
+  Syrk64Sets &s = *out;
+  s.n = nk;
+  const int64_t T = ceil_div(c->n, kT64), nf = T * (T - 1) / 2;
+  const int64_t units = 16 * nf + 10 * T;  // MFMAs of one step over all tiles
+  const int64_t slots = 2 * int64_t(c->ncu), steps = jc * work / 4;
+  const int64_t rounds = std::min<int64_t>(64, std::max<int64_t>(1, steps * units / (16 * 4 * 160 * slots)));
+  const int64_t target = c->split_target ? c->split_target : slots * rounds;
+  int64_t kb = 0;
+  for (int d = 0; d < nk; ++d) {
+    s.off[d] = off[size_t(d)];
+    s.opad[d] = std::max(opad[size_t(d)], 4);
+    s.nsf[d] = s.nsd[d] = 0;
+    if (nocc[d] > 0) {
+      const int64_t own = target * opad[size_t(d)];
+      // at least 4 steps per wave, at most one slice per vector
+      const int64_t most = std::max<int64_t>(1, std::min<int64_t>(jc, jc * opad[size_t(d)] / 64));
+      auto clip = [&](int64_t v) { return int(std::max<int64_t>(1, std::min<int64_t>(v, most))); };
+      s.nsf[d] = clip(own * 16 / (work * units));
+      s.nsd[d] = clip(own * 10 / (work * units));
+    }
+    s.kf[d] = kb;
+    kb += s.nsf[d] * nchunk * nf * kSlot64;
+    s.kd[d] = kb;
+    kb += s.nsd[d] * nchunk * T * kSlot64;
+    s.item0[d + 1] = s.item0[d] + int(8 * (ceil_div(s.nsd[d] * T, 8) + ceil_div(s.nsf[d] * nf, 8)));
+  }
+  return kb;
+}
+
 // A run of vectors [j0, j1) computed in one precision.
 struct Segment {
   int64_t j0, j1;
@@ -1282,26 +1572,28 @@ int exchange_segments(Context *c, int32_t nk, const int32_t *nocc, const double 
   const int64_t elem = use[MJK_PREC_FP64] ? 8 : 4;
   const int64_t xvec_bytes = elem * ldc * n_pad;
   int64_t jc = std::max<int64_t>(1, std::min<int64_t>(c->nchol, c->x_budget / xvec_bytes));
-  int64_t nchunk = 0;
+  int64_t nchunk = 0, nchunk64 = 0;  // chunks in reduced precision, in FP64
   for (const Segment &s : segs)
-    if (s.j1 > s.j0) nchunk += ceil_div(s.j1 - s.j0, jc);
+    if (s.j1 > s.j0) (s.prec == MJK_PREC_FP64 ? nchunk64 : nchunk) += ceil_div(s.j1 - s.j0, jc);
   if (jc * ldc >= (int64_t(1) << 31))
     return set_error(c, MJK_ERR_ARG, "exchange: chunk contraction length exceeds 2^31");
   if ((rc = ensure(c, c->w->x, size_t(xvec_bytes) * jc))) return rc;
 
   // ---- SYRK tiling and slices (one launch per chunk covers every density)
+  int64_t work = 0;  // contraction rows per vector over all densities
+  for (int d = 0; d < nk; ++d)
+    if (nocc[d] > 0) work += opad[size_t(d)];
+  Syrk64Sets sets64{};
+  int64_t kb64 = nchunk64 ? plan_syrk64(c, nk, nocc, off, opad, jc, work, nchunk64, &sets64) : 0;
   int tm = c->tile_syrk ? c->tile_syrk : (n_pad >= 512 && n_pad % 128 == 0 ? 128 : 64);
   if (n_pad % tm) tm = 64;
-  const int ntile1 = n_pad / tm;
+  const int ntile1 = int(ceil_div(n, tm));
   const int ntiles = ntile1 * (ntile1 + 1) / 2;
   SyrkSets sets{};
   sets.n = nk;
   int64_t kb = 0;
   sets.item0[0] = 0;
-  // slices per density in proportion to its contraction length (opad rows per vector)
-  int64_t work = 0;
-  for (int d = 0; d < nk; ++d)
-    if (nocc[d] > 0) work += opad[size_t(d)];
+  // slices per density in proportion to its contraction length (opad rows per vector).
   // Workgroups per launch: at most the target, rounded down, so that a target of
   // whole resident rounds (k_syrk keeps two workgroups per CU) leaves no handful
   // of items to a round of its own.  Default: the most rounds (1, 2, 4 or 8) that
@@ -1322,8 +1614,8 @@ int exchange_segments(Context *c, int32_t nk, const int32_t *nocc, const double 
     sets.item0[d + 1] = sets.item0[d] + sets.nsplit[d] * ntiles;
   }
   const int items = sets.item0[nk];
-  if ((rc = ensure(c, c->w->kpart, sizeof(double) * size_t(std::max<int64_t>(kb, 1))))) return rc;
-  double *kpart = static_cast<double *>(c->w->kpart.ptr);
+  if ((rc = ensure(c, c->w->kpart, sizeof(double) * size_t(std::max<int64_t>(kb64 + kb, 1))))) return rc;
+  double *kpart64 = static_cast<double *>(c->w->kpart.ptr), *kpart = kpart64 + kb64;
 
   // ---- screening set-up (norms of L strips, of the orbital sets, counters)
   const bool screen = tau > 0.0 || thr_x > 0.0;
@@ -1370,9 +1662,9 @@ int exchange_segments(Context *c, int32_t nk, const int32_t *nocc, const double 
     }
   }
 
-  int64_t slot = 0;  // running chunk index over all segments
+  int64_t slot = 0, slot64 = 0;  // running chunk indices
   for (const Segment &s : segs) {
-    for (int64_t j0 = s.j0; j0 < s.j1; j0 += jc, ++slot) {
+    for (int64_t j0 = s.j0; j0 < s.j1; j0 += jc, ++(s.prec == MJK_PREC_FP64 ? slot64 : slot)) {
       const int64_t jn = std::min(jc, s.j1 - j0);
       phase_begin(c);
       switch (s.prec) {
@@ -1413,12 +1705,11 @@ int exchange_segments(Context *c, int32_t nk, const int32_t *nocc, const double 
       phase_begin(c);
       switch (s.prec) {
         case MJK_PREC_FP64:
-          syrk_launch<F64>(c, tm, items, static_cast<const double *>(c->w->x.ptr), ldc, jn, ntiles,
-                           sets, kpart, int(slot));
+          syrk_launch64(c, static_cast<const double *>(c->w->x.ptr), ldc, jn, sets64, kpart64, int(slot64));
           break;
         case MJK_PREC_FP32:
-          syrk_launch<F32>(c, tm, items, static_cast<const float *>(c->w->x.ptr), ldc, jn, ntiles,
-                           sets, kpart, int(slot));
+          syrk_launch32(c, tm, items, static_cast<const float *>(c->w->x.ptr), ldc, jn, ntiles,
+                        sets, kpart, int(slot));
           break;
         default:
           syrk_launch_b3(c, tm, items, static_cast<const float *>(c->w->x.ptr), ldc, jn, ntiles,
@@ -1428,8 +1719,8 @@ int exchange_segments(Context *c, int32_t nk, const int32_t *nocc, const double 
     }
   }
   phase_begin(c);
-  hipLaunchKernelGGL(k_reduce_k, dim3(unsigned(n), unsigned(nk)), dim3(256), 0, c->stream, kpart, n,
-                     tm, ntiles, sets, int(nchunk), klt, ldk);
+  hipLaunchKernelGGL(k_reduce_k, dim3(unsigned(n), unsigned(ceil_div(n, 64)), unsigned(nk)), dim3(kThreads), 0,
+                     c->stream, kpart64, sets64, int(nchunk64), kpart, tm, sets, int(nchunk), n, klt, ldk);
   phase_end(c, MJK_PHASE_REDUCE);
   return hip_check(c, hipGetLastError(), "exchange launch");
 }

@@ -39,7 +39,7 @@ extern "C" int mjk_autotune(mjk_context *c, int32_t nk, const int32_t *nocc,
   c->tile_syrk = c->split_target = c->ht_ta = 0;
   if ((rc = exchange(c, nk, nocc, corb, klt, ldk, precision))) goto done;
   for (int tm : tms) {
-    if (c->n_pad % tm) continue;
+    if (c->n_pad % tm || (precision == MJK_PREC_FP64 && tm != 64)) continue;  // the FP64 SYRK has one tile
     for (int sp : splits) {
       for (int ta : tas) {
         c->tile_syrk = tm;
