@@ -615,7 +615,7 @@ int coulomb_exchange_run(Context *c, const double *dlt, int64_t ldd, double *jlt
     return exchange(c, nk, nocc, corb, klt, ldk, MJK_PREC_FP64);
   }
   const int64_t M = c->nchol;
-  const int ntmax = c->n_pad / 64;  // AO tiles of the narrowest half-transform tile
+  const int ntmax = int(ceil_div(c->n, 16));  // at most one wave per 16 columns
   if ((rc = ensure(c, c->w->vpart, sizeof(double) * size_t(ntmax) * M)) ||
       (rc = ensure(c, c->w->v, sizeof(double) * M)))
     return rc;

@@ -9,14 +9,12 @@
 //  * All orbital sets of one call are concatenated into one "orbital bank"
 //    Cb[b][k] (AO row b, orbital column k; every set starts at a multiple of 4
 //    columns, padded with zeros), so ONE pass over L serves every density.
-//  * Half-transform: a workgroup owns (vector J, 64-wide AO tile a0) and all
-//    bank rows k.  It walks b in chunks of BK, unpacks the packed-triangle
-//    block L^J[b0:b0+BK, a0:a0+64] into a square LDS tile (mirroring across
-//    the diagonal; the reference's 1/2 on diagonal pairs added twice is the
-//    same as taking the diagonal once), stages Cb[b0:b0+BK, :] in LDS and
-//    runs v_mfma_f64_16x16x4f64 with wave w owning AO columns 16w..16w+15.
-//    Output X[J][k][a] (a fastest).  Workgroups of one vector are placed on
-//    one XCD so that the two reads of every packed element (as row and as
+//  * Half-transform X[J][k][a] (a fastest): FP64 k_ht64, L from memory into MFMA
+//    registers; FP32 k_ht, a workgroup per (vector J, AO tile) that unpacks the
+//    packed-triangle block L^J[b0:b0+BK, tile] into a square LDS tile (mirroring
+//    across the diagonal; the reference's 1/2 on diagonal pairs added twice is
+//    the same as taking the diagonal once).  Workgroups of one vector are placed
+//    on one XCD so that the two reads of every packed element (as row and as
 //    transposed column) share that XCD's L2.
 //  * SYRK: a workgroup owns one tile (A >= B) of K and a slice of the
 //    vectors; it contracts over (J, k in the density's bank columns) with
@@ -127,7 +125,7 @@ __global__ void k_to_f32(const double *__restrict__ src, float *__restrict__ dst
     dst[i] = float(src[i]);
 }
 
-// ---- half-transform ------------------------------------------------------
+// ---- FP32 half-transform -------------------------------------------------
 // grid.x = round_up(ceil(jc/NJ) * ntile_a, 8), block = 256.  Workgroup (jr,
 // a-tile of TA columns) computes, for the NJ vectors J = NJ*jr + q < jc,
 // X[(J*LDC + k)*n_pad + a] = sum_b Cb[b*LDC + k] L^J_ab for all LDC = 16*OT
@@ -135,19 +133,13 @@ __global__ void k_to_f32(const double *__restrict__ src, float *__restrict__ dst
 // (TA/64 MFMA column tiles) and all OT row tiles; each orbital fragment read
 // from LDS feeds the MFMAs of all NJ vectors.  The next b-chunk is fetched
 // into registers while the current one is multiplied out of LDS.
-// FV: the workgroup also sums L^J_ba D_ba over the staged elements with b >= a
-// (only "row-major" chunks hold such elements; each packed element is staged
-// there by exactly one workgroup) into fv.vpart[tile * fv.m + j0 + J] -- the
-// Coulomb pass V = L^T D without a read of L of its own, and the folded
-// density read for half of the chunks only.
-template <class P, int OT, int TA, int BK, int NJ, bool FV>
+template <class P, int OT, int TA, int BK, int NJ>
 __global__ __launch_bounds__(kThreads) void k_ht(
     const typename P::T *__restrict__ L, int64_t ldl, int n, int n_pad,
     const typename P::T *__restrict__ Cb, int64_t j0, int64_t jc, int ntile_a, int64_t nblocks,
-    typename P::T *__restrict__ X, const Screen sc, const FuseV fv) {
+    typename P::T *__restrict__ X, const Screen sc) {
   typedef typename P::T T;
   typedef typename P::Acc Acc;
-  static_assert(!FV || std::is_same<T, double>::value, "fused Coulomb pass is FP64 only");
   constexpr int LDC = 16 * OT;
   // Wave layout.  Narrow banks: wave w owns AO columns w*TA/4 .. (w+1)*TA/4-1
   // and all OT row tiles.  Wide banks (one vector, even OT >= 6, TA = 64): 2 x 2
@@ -207,9 +199,6 @@ __global__ __launch_bounds__(kThreads) void k_ht(
     for (int t = 0; t < OTW; ++t)
 #pragma unroll
       for (int j = 0; j < NB; ++j) acc[q][t][j] = Acc{0, 0, 0, 0};
-  T vp[NJ];  // FV: this thread's share of sum_ab L^J_ab P_ab
-#pragma unroll
-  for (int q = 0; q < NJ; ++q) vp[q] = T(0);
 
   if (a0 < n) {
     // orbital bank rows are contiguous: 16-byte pieces where the tile divides
@@ -218,8 +207,6 @@ __global__ __launch_bounds__(kThreads) void k_ht(
     constexpr int CV = CN / VW;
     VT rc[CV];
     T rl[NJ][LN];
-    T rd[FV ? LN : 1];  // FV: density elements of the staged L elements
-    uint32_t vok = 0;   // FV: bit i: element i lies in the matrix with b >= a
     // bit i: element i lies inside the matrix.  The mask is applied when the
     // chunk is stashed, so the loads stay in flight across the multiply of
     // the current chunk (a select right after the load would wait for it).
@@ -236,8 +223,8 @@ __global__ __launch_bounds__(kThreads) void k_ht(
     constexpr int DA = kThreads / BK, DB = kThreads / TA;
     static_assert(kThreads % BK == 0 && kThreads % TA == 0, "element walk");
     // The chunk kinds differ only in the packed index of each element: the
-    // branches form the indices, and one load sequence after them fills rl
-    // (and rd).  Loads issued inside the branches left their registers to be
+    // branches form the indices, and one load sequence after them fills rl.
+    // Loads issued inside the branches left their registers to be
     // merged by copies at the join, and a copy of a register whose load is in
     // flight waits for the whole memory queue: the chunk after next was then
     // waited for right after its loads were issued.
@@ -259,7 +246,6 @@ __global__ __launch_bounds__(kThreads) void k_ht(
           a += uint32_t(DA);
         }
         lok = LN == 32 ? ~0u : (1u << LN) - 1u;
-        if constexpr (FV) vok = 0u;
       } else if (inside && b0 >= a0 + TA) {  // packed row b = b0 + tid/TA + DB i at column a0 + tid%TA
         uint32_t b = uint32_t(b0 + tid / TA);
         uint32_t x = tri0u(b) + uint32_t(a0 + tid % TA);
@@ -270,7 +256,6 @@ __global__ __launch_bounds__(kThreads) void k_ht(
           b += uint32_t(DB);
         }
         lok = LN == 32 ? ~0u : (1u << LN) - 1u;
-        if constexpr (FV) vok = lok;
       } else {
 #pragma unroll
         for (int i = 0; i < LN; ++i) {
@@ -281,17 +266,12 @@ __global__ __launch_bounds__(kThreads) void k_ht(
           const int hi = b >= a ? b : a, lo = b >= a ? a : b;
           idx[i] = ok ? tri0u(uint32_t(hi)) + uint32_t(lo) : 0u;  // branch-free masked load
           lok = ok ? (lok | (1u << i)) : (lok & ~(1u << i));
-          if constexpr (FV) vok = (!colmajor && ok && b >= a) ? (vok | (1u << i)) : (vok & ~(1u << i));
         }
       }
 #pragma unroll
       for (int i = 0; i < LN; ++i)
 #pragma unroll
         for (int q = 0; q < NJ; ++q) rl[q][i] = Lq[q][idx[i]];
-      if constexpr (FV) {  // column chunks hold no b >= a element: one cached address, masked by vok
-#pragma unroll
-        for (int i = 0; i < LN; ++i) rd[i] = fv.p[colmajor ? 0u : idx[i]];
-      }
     };
     auto stash = [&](int b0, int buf) {
       const bool colmajor = b0 + BK <= a0;
@@ -305,13 +285,6 @@ __global__ __launch_bounds__(kThreads) void k_ht(
 #pragma unroll
         for (int q = 0; q < NJ; ++q)
           sL[buf][q][bb * SLD + aa] = ((lok >> i) & 1u) ? rl[q][i] : T(0);
-        if constexpr (FV) {
-          if (!colmajor) {
-            const T d = ((vok >> i) & 1u) ? rd[i] : T(0);
-#pragma unroll
-            for (int q = 0; q < NJ; ++q) vp[q] += rl[q][i] * d;
-          }
-        }
       }
     };
     // Double-buffered LDS: chunk c is multiplied out of buffer c&1 while
@@ -354,25 +327,6 @@ __global__ __launch_bounds__(kThreads) void k_ht(
       __syncthreads();
     }
   }
-  if constexpr (FV) {  // workgroup sum in a fixed order: wave butterflies, then waves 0..3
-    __shared__ double sV[NJ][kThreads / 64];
-#pragma unroll
-    for (int q = 0; q < NJ; ++q) {
-      double v = vp[q];
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-      if (lane == 0) sV[q][w] = v;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < NJ; ++q)
-      if (tid == q && live[q]) {
-        double v = 0.0;
-#pragma unroll
-        for (int k = 0; k < kThreads / 64; ++k) v += sV[q][k];
-        fv.vpart[int64_t(lb % ntile_a) * fv.m + j0 + NJ * jr + q] = v;
-      }
-  }
 #pragma unroll
   for (int q = 0; q < NJ; ++q) {
     if (!live[q]) continue;
@@ -386,6 +340,365 @@ __global__ __launch_bounds__(kThreads) void k_ht(
         for (int r = 0; r < 4; ++r)
           xj[int64_t(16 * (t0 + t) + P::row(lane, r)) * n_pad + a] = acc[q][t][j][r];
     }
+  }
+}
+
+// ---- FP64 half-transform ------------------------------------------------------
+// Wave item = (vector J, up to NB blocks of 16 AO columns a); the wave forms all
+// OT 16-row orbital tiles of its columns and walks b in 16-row chunks.  No other
+// wave needs its elements of L^J for this product, so L goes from memory into
+// the wave's registers with no staging shared between waves; only the bank
+// chunk, which the workgroup's four waves share, is staged in LDS (one barrier
+// per chunk).  Every load instruction covers 128-byte runs of packed rows:
+//  * below the diagonal block (b >= a) packed row b holds a contiguous and lane
+//    l = 16 g + m loads L(b, a) at b = 16 c + 4 g + s, a = a0 + 16 j + m: these
+//    are the MFMA operands of the four steps s (the bank rows in the same
+//    order), and step s of chunk c + 1 is loaded into the registers of step s
+//    of chunk c as soon as that is multiplied;
+//  * above it (b < a) packed row a holds b contiguous: lane l loads
+//    b = 16 c + m of row a = a0 + 16 j + 4 q + g (q = 0..3) and each 16 x 16
+//    block is turned through a wave-private LDS tile (loads that follow the
+//    operand layout there touch one cache line per lane, four times over:
+//    the L1 request rate bound the kernel);
+//  * the diagonal chunks gather element by element.
+// Orbital tile pair (i, h) holds the bank columns 32 i + 2 m + h, so one 16-byte
+// LDS read gives two A fragments.  Indices past n are clamped to n - 1 (always
+// inside the packed row) and the values zeroed where that can happen.
+// FV: sum_{b >= a} L_ba D_ba of the wave's columns into *vout.
+// Bound by the matrix cores (busy 74-85% of the cycles) at the clock they leave
+// (2.1-2.3 GHz); where few orbitals share an element, by the L traffic too (each
+// packed element is read twice, 3.7 TB/s at n=512 nocc=64).  With the V work:
+// n=1200 nchol=6000 nocc=150 55.3 -> 43.3 ms (65 TFLOP/s executed), n=536
+// nchol=2510 nocc=98 3.7 -> 2.8 ms, n=512 nchol=2048 nocc=64 1.40 -> 1.34 ms,
+// n=187 nchol=905 nocc=23 0.116 -> 0.084 ms, against staging square tiles of L
+// in LDS (its transposing stores, their waits and 5 VALU operations per MFMA
+// stood between the MFMAs).
+constexpr int kHtB = 16;       // contraction rows per chunk
+constexpr int kHtS = 17;       // row stride of a turned block
+
+template <int OT, int NBV, bool FV>
+__device__ __forceinline__ void ht64_wave(const double *__restrict__ Lj, int n, int nch, int n_pad,
+                                          const double *__restrict__ Cb, int a0, double *__restrict__ xj,
+                                          const double *__restrict__ dens, double *__restrict__ vout,
+                                          double (*__restrict__ sC)[kHtB * 16 * OT], double *__restrict__ sT) {
+  constexpr int LDC = 16 * OT;
+  constexpr int HP = OT / 2;                 // pairs of orbital tiles; an odd last tile stands alone
+  constexpr int NB1 = NBV > 0 ? NBV : 1;
+  constexpr int CN = kHtB * LDC / 2 / kThreads;  // 16-byte pieces of a bank chunk per thread ...
+  constexpr int CR = kHtB * LDC / 2 % kThreads;  // ... and those of a last, partial round
+  const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
+  v4d acc[OT][NB1];
+#pragma unroll
+  for (int t = 0; t < OT; ++t)
+#pragma unroll
+    for (int j = 0; j < NBV; ++j) acc[t][j] = v4d{0.0, 0.0, 0.0, 0.0};
+  double vp = 0.0;
+  // bank chunk: global -> registers -> LDS, the layout unchanged
+  v2d rc[CN + (CR ? 1 : 0)];
+  auto fetch_c = [&](int c) __attribute__((always_inline)) {
+    const double *__restrict__ src = Cb + int64_t(c) * kHtB * LDC;
+#pragma unroll
+    for (int i = 0; i < CN; ++i) rc[i] = *reinterpret_cast<const v2d *>(src + 2 * (tid + kThreads * i));
+    if constexpr (CR > 0)
+      rc[CN] = *reinterpret_cast<const v2d *>(src + 2 * (tid < CR ? tid + kThreads * CN : 0));
+  };
+  auto stash_c = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < CN; ++i) *reinterpret_cast<v2d *>(&sC[buf][2 * (tid + kThreads * i)]) = rc[i];
+    if constexpr (CR > 0)
+      if (tid < CR) *reinterpret_cast<v2d *>(&sC[buf][2 * (tid + kThreads * CN)]) = rc[CN];
+  };
+  const int ncol = a0 / kHtB;  // chunks wholly above the diagonal block
+  double rl[4][NB1];
+  double rd[2][NB1];  // FV: density values of two steps in flight
+  // General loads, for the chunks outside the two long runs below.  The lane's
+  // parts of the packed indices are hidden from the loop-invariant code motion,
+  // which would keep an index per load in registers.
+  auto load_low = [&](int c, int s) __attribute__((always_inline)) {  // c >= ncol
+    const int b0 = c * kHtB;
+    int mm = m, gg = g;
+    asm volatile("" : "+v"(mm), "+v"(gg));
+    const uint32_t b = uint32_t(min(b0 + 4 * gg + s, n - 1));
+    const uint32_t tb = tri0u(b);
+    uint32_t x[NB1];
+#pragma unroll
+    for (int j = 0; j < NBV; ++j) {
+      const uint32_t a = uint32_t(min(a0 + 16 * j + mm, n - 1));
+      x[j] = b >= a ? tb + a : tri0u(a) + b;
+    }
+#pragma unroll
+    for (int j = 0; j < NBV; ++j) rl[s][j] = Lj[x[j]];
+  };
+  auto load_col = [&](int c, int s) __attribute__((always_inline)) {  // c < ncol
+    int mm = m, gg = g;
+    asm volatile("" : "+v"(mm), "+v"(gg));
+#pragma unroll
+    for (int j = 0; j < NBV; ++j)
+      rl[s][j] = Lj[tri0u(uint32_t(min(a0 + 16 * j + 4 * s + gg, n - 1))) + uint32_t(c * kHtB + mm)];
+  };
+  // density of the step's elements with b >= a (the others: one cached address)
+  auto load_d = [&](int c, int s) __attribute__((always_inline)) {
+    if constexpr (FV) {
+      int mm = m, gg = g;
+      asm volatile("" : "+v"(mm), "+v"(gg));
+      const int b = min(c * kHtB + 4 * gg + s, n - 1);
+      const uint32_t tb = tri0u(uint32_t(b)) + uint32_t(a0 + mm);
+#pragma unroll
+      for (int j = 0; j < NBV; ++j) rd[s & 1][j] = dens[a0 + 16 * j + mm <= b ? tb + 16u * j : 0u];
+    }
+  };
+  // A fragments of one step, each pair replaced by the next step's once used
+  v2d cf[HP > 0 ? HP : 1];
+  double co = 0.0;
+  auto load_cp = [&](int buf, int s, int i) __attribute__((always_inline)) {
+    cf[i] = *reinterpret_cast<const v2d *>(&sC[buf][(4 * g + s) * LDC + 32 * i + 2 * m]);
+  };
+  auto load_co = [&](int buf, int s) __attribute__((always_inline)) {
+    if constexpr (OT % 2 == 1) co = sC[buf][(4 * g + s) * LDC + 16 * (OT - 1) + m];
+  };
+  auto step = [&](int buf, int s, const double(&x)[NB1]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < HP; ++i) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int j = 0; j < NBV; ++j) acc[2 * i + h][j] = F64::mma(cf[i][h], x[j], acc[2 * i + h][j]);
+      if (s < 3) load_cp(buf, s + 1, i);
+    }
+    if constexpr (OT % 2 == 1) {
+#pragma unroll
+      for (int j = 0; j < NBV; ++j) acc[OT - 1][j] = F64::mma(co, x[j], acc[OT - 1][j]);
+      if (s < 3) load_co(buf, s + 1);
+    }
+  };
+  auto first_c = [&](int buf) __attribute__((always_inline)) {
+    if constexpr (NBV > 0) {
+#pragma unroll
+      for (int i = 0; i < HP; ++i) load_cp(buf, 0, i);
+      load_co(buf, 0);
+    }
+  };
+
+  auto next_c = [&](int c) __attribute__((always_inline)) {  // end of chunk c
+    stash_c((c & 1) ^ 1);
+    fetch_c(min(c + 2, nch - 1));
+    __syncthreads();
+  };
+  fetch_c(0);
+  stash_c(0);
+  fetch_c(min(1, nch - 1));
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    if (ncol > 0) load_col(0, s);
+    else load_low(0, s);
+  }
+  __syncthreads();
+  int c = 0;
+  // ---- chunks above the diagonal block (b < a): blocks turned through LDS;
+  // the next chunk is loaded as soon as this one is in LDS
+  auto upper = [&](int c, auto load) __attribute__((always_inline)) {
+    const int cur = c & 1;
+    first_c(cur);
+    if constexpr (NBV > 0) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int j = 0; j < NBV; ++j) sT[(16 * j + 4 * s + g) * kHtS + m] = rl[s][j];
+      __builtin_amdgcn_sched_barrier(0);
+      load();
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_wave_barrier();
+      double xs[2][NB1];
+      auto turn = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < NBV; ++j) xs[s & 1][j] = sT[(16 * j + m) * kHtS + 4 * g + s];
+      };
+      turn(0);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        if (s < 3) turn(s + 1);
+        step(cur, s, xs[s & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+    next_c(c);
+  };
+  // byte offsets of the long runs are 32-bit: below 2^29 packed elements
+  const bool small = uint32_t(n) < 32768u;
+  if (small) {
+    // chunk c + 1 of every row is 128 bytes after chunk c: one offset per load,
+    // kept, and a uniform pointer that moves
+    uint32_t off[4][NB1];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int j = 0; j < NBV; ++j) off[s][j] = 8u * (tri0u(uint32_t(min(a0 + 16 * j + 4 * s + g, n - 1))) + uint32_t(m));
+    const char *__restrict__ p = reinterpret_cast<const char *>(Lj);
+#pragma unroll 1
+    for (; c + 1 < ncol; ++c) {
+      p += 8 * kHtB;
+      upper(c, [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int j = 0; j < NBV; ++j) rl[s][j] = *reinterpret_cast<const double *>(p + off[s][j]);
+      });
+    }
+  }
+#pragma unroll 1
+  for (; c + 1 < ncol; ++c)
+    upper(c, [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) load_col(c + 1, s);
+    });
+  if (c < ncol) {
+    upper(c, [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) load_low(c + 1, s);
+    });
+    ++c;
+  }
+  // ---- diagonal block and below
+  auto lower = [&](int c) __attribute__((always_inline)) {
+    const int cur = c & 1, cn = min(c + 1, nch - 1);
+    first_c(cur);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      if constexpr (NBV > 0) {
+        // masks by selects into temporaries: a branch that rewrote the loaded
+        // registers made the compiler copy them while their loads were in flight
+        const int b = c * kHtB + 4 * g + s;
+        double x[NB1];
+#pragma unroll
+        for (int j = 0; j < NBV; ++j) x[j] = b < n ? rl[s][j] : 0.0;
+        if constexpr (FV) {
+#pragma unroll
+          for (int j = 0; j < NBV; ++j) vp += x[j] * (b >= a0 + 16 * j + m ? rd[s & 1][j] : 0.0);
+          asm volatile("" : "+v"(vp));  // summed here: sunk to the end of the chunk, the operands would stay live
+          __builtin_amdgcn_sched_barrier(0);
+          load_d(s < 2 ? c : cn, (s + 2) & 3);
+        }
+        step(cur, s, x);
+        __builtin_amdgcn_sched_barrier(0);
+        load_low(cn, s);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    next_c(c);
+  };
+  load_d(c, 0);
+  load_d(c, 1);
+  const int cd = min(ncol + NBV, nch);            // past the diagonal chunks
+  const int cr = n % kHtB == 0 ? nch - 1 : nch - 2;  // the next chunk has all its rows inside up to here
+#pragma unroll 1
+  for (; c < cd; ++c) lower(c);
+  if (NBV > 0 && small && c < cr) {
+    // chunks below the diagonal block whose next chunk needs no clamp: the
+    // offset of row 16 c + 4 g + s of the next chunk steps by its row distance
+    const char *__restrict__ lp = reinterpret_cast<const char *>(Lj);
+    const char *__restrict__ dp = reinterpret_cast<const char *>(dens);
+    uint32_t off[4], inc[4];  // this chunk's rows; bytes to the next chunk's: 8 (16 b + 136)
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const uint32_t b = uint32_t(c * kHtB + 4 * g + s);
+      off[s] = 8u * (tri0u(b) + uint32_t(a0 + m));
+      inc[s] = 8u * (16u * b + 136u);
+    }
+#pragma unroll 1
+    for (; c < cr; ++c) {
+      const int cur = c & 1;
+      first_c(cur);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        double x[NB1];
+#pragma unroll
+        for (int j = 0; j < NBV; ++j) x[j] = rl[s][j];
+        if constexpr (FV) {
+#pragma unroll
+          for (int j = 0; j < NBV; ++j) vp += x[j] * rd[s & 1][j];
+          asm volatile("" : "+v"(vp));
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int j = 0; j < NBV; ++j)
+            rd[s & 1][j] = *reinterpret_cast<const double *>(dp + off[(s + 2) & 3] + 128 * j);
+        }
+        step(cur, s, x);
+        __builtin_amdgcn_sched_barrier(0);
+        off[s] += inc[s];
+        inc[s] += 8u * 256u;
+#pragma unroll
+        for (int j = 0; j < NBV; ++j) rl[s][j] = *reinterpret_cast<const double *>(lp + off[s] + 128 * j);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      next_c(c);
+    }
+  }
+#pragma unroll 1
+  for (; c < nch; ++c) lower(c);
+  if constexpr (FV) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) vp += __shfl_xor(vp, o);
+    if (NBV > 0 && lane == 0) *vout = vp;
+  }
+#pragma unroll
+  for (int j = 0; j < NBV; ++j) {
+    const int a = a0 + 16 * j + m;
+#pragma unroll
+    for (int t = 0; t < OT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 4 * r + g;
+        const int k = t < 2 * HP ? 32 * (t >> 1) + 2 * row + (t & 1) : 16 * t + row;
+        xj[int64_t(k) * n_pad + a] = a < n ? acc[t][j][r] : 0.0;  // clamped columns
+      }
+  }
+}
+
+// grid.x = round_up(ceil(jc * W / 4), 8): four wave items per workgroup, item =
+// J * W + t over the W = ceil(nblk / nb) waves of a vector (nblk = ceil(n / 16)
+// column blocks, nb <= NB of them per wave).
+template <int OT, int NB, bool FV>
+__global__ __launch_bounds__(kThreads, 2) void k_ht64(const double *__restrict__ L, int64_t ldl, int n, int n_pad,
+                                                   const double *__restrict__ Cb, int64_t j0, int64_t jc, int W,
+                                                   int nb, int64_t nblocks, double *__restrict__ X,
+                                                   const Screen sc, const FuseV fv) {
+  static_assert(NB <= 4, "tail widths");
+  __shared__ __attribute__((aligned(16))) double sC[2][kHtB * 16 * OT];
+  __shared__ __attribute__((aligned(16))) double sT[4][NB * 16 * kHtS];
+  const int64_t lb = xcd_logical(nblocks);
+  if (lb < 0) return;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t item = 4 * lb + w;
+  const bool live = item < jc * W;
+  const int64_t J = live ? item / W : jc - 1;
+  const int t = live ? int(item - J * W) : 0;
+  const int nblk = (n + 15) / 16, nch = nblk;
+  const int a0 = 16 * nb * t;
+  int nbv = live ? min(nb, nblk - nb * t) : 0;
+  const double *__restrict__ Lj = L + (j0 + J) * ldl;
+  double *__restrict__ xj = X + J * (16 * OT) * int64_t(n_pad);
+  if (sc.lnorm && live) {  // screened: ||X tile||_F <= ||L^J[:, strips of the tile]||_F max_d ||C_d||_F
+    double s2 = 0.0;
+    for (int st = a0 / 64; st <= (a0 + 16 * nbv - 1) / 64; ++st) {
+      const double v = sc.lnorm[(j0 + J) * sc.nstrip + st];
+      s2 += v * v;
+    }
+    if (sqrt(s2) * sc.cmax[0] < sc.thr_x) {
+      for (int e = threadIdx.x & 63; e < 16 * OT * 16 * nbv; e += 64)
+        xj[int64_t(e / (16 * nbv)) * n_pad + a0 + e % (16 * nbv)] = 0.0;
+      if ((threadIdx.x & 63) == 0) atomicAdd(sc.cnt + 1, 1ull);
+      nbv = 0;
+    }
+  }
+  double *vout = FV ? fv.vpart + int64_t(t) * fv.m + j0 + J : nullptr;
+  // a wave without columns still stages its share of the bank and joins the barriers
+  switch (nbv) {
+    case 0: ht64_wave<OT, 0, FV>(Lj, n, nch, n_pad, Cb, a0, xj, fv.p, vout, sC, sT[w]); break;
+    case 1: ht64_wave<OT, 1, FV>(Lj, n, nch, n_pad, Cb, a0, xj, fv.p, vout, sC, sT[w]); break;
+    case 2: if constexpr (NB >= 2) ht64_wave<OT, 2, FV>(Lj, n, nch, n_pad, Cb, a0, xj, fv.p, vout, sC, sT[w]); break;
+    case 3: if constexpr (NB >= 3) ht64_wave<OT, 3, FV>(Lj, n, nch, n_pad, Cb, a0, xj, fv.p, vout, sC, sT[w]); break;
+    default: if constexpr (NB >= 4) ht64_wave<OT, 4, FV>(Lj, n, nch, n_pad, Cb, a0, xj, fv.p, vout, sC, sT[w]); break;
   }
 }
 
@@ -812,7 +1125,7 @@ __global__ __launch_bounds__(kThreads) void k_strip_norms(const double *__restri
 // xn2[(d*jn + J)*nstrip + st] = sum over the rows of set d and the 64 AOs of
 // strip st of X[J]^2.  grid = (jn, nstrip, nk), 256 threads.
 template <typename T>
-__global__ __launch_bounds__(kThreads) void k_xnorms(const T *__restrict__ X, int ldc, int n_pad,
+__global__ __launch_bounds__(kThreads) void k_xnorms(const T *__restrict__ X, int ldc, int n, int n_pad,
                                                      const SyrkSets sets, int nstrip,
                                                      double *__restrict__ xn2) {
   __shared__ double red[4];
@@ -821,6 +1134,7 @@ __global__ __launch_bounds__(kThreads) void k_xnorms(const T *__restrict__ X, in
   const int off = sets.off[d], opad = sets.opad[d];
   double s = 0.0;
   for (int e = threadIdx.x; e < opad * 64; e += kThreads) {
+    if (st * 64 + (e & 63) >= n) continue;  // columns past n need not be written
     const double v = double(X[(J * ldc + off + (e >> 6)) * int64_t(n_pad) + st * 64 + (e & 63)]);
     s += v * v;
   }
@@ -1273,76 +1587,95 @@ __global__ __launch_bounds__(kThreads) void k_reduce_k(const double *__restrict_
   if (q == 0 && b <= a) klt[d * ldk + tri0(a) + b] = ((s + red[0][cb]) + red[1][cb]) + red[2][cb];
 }
 
-template <class P, int OT, int TA, int BK>
-void launch_ht(Context *c, const typename P::T *L, const typename P::T *cb, int64_t j0, int64_t jc,
-               typename P::T *X) {
-  // two vectors per workgroup while the accumulators stay small (measured
-  // 5-6% faster at OT = 4: half the orbital-fragment LDS reads per MFMA), and
-  // at OT = 7 (4% faster; at OT = 5 and 6 it measured 3-7% slower: those keep
-  // one vector, 6 in the 2 x 2 wave layout)
+template <int OT, int TA, int BK>
+void launch_ht(Context *c, const float *L, const float *cb, int64_t j0, int64_t jc, float *X) {
+  // two vectors per workgroup while the accumulators stay small (half the
+  // orbital-fragment LDS reads per MFMA) and at OT = 7
   constexpr int NJ = (OT * (TA / 64) <= 4 || (TA == 64 && OT == 7)) ? 2 : 1;
   const int ntile_a = c->n_pad / TA;
   const int64_t nblocks = ceil_div(jc, NJ) * ntile_a;
   const int64_t grid = round_up(nblocks, 8);
-  if constexpr (std::is_same<P, F64>::value) {
-    if (c->fv.p) {  // fused Coulomb pass (never together with screening)
-      c->fv.ntile = ntile_a;
-      hipLaunchKernelGGL((k_ht<P, OT, TA, BK, NJ, true>), dim3(unsigned(grid)), dim3(kThreads), 0,
-                         c->stream, L, c->ldl, c->n, c->n_pad, cb, j0, jc, ntile_a, nblocks, X,
-                         Screen{}, c->fv);
-      return;
-    }
-  }
-  hipLaunchKernelGGL((k_ht<P, OT, TA, BK, NJ, false>), dim3(unsigned(grid)), dim3(kThreads), 0,
-                     c->stream, L, c->ldl, c->n, c->n_pad, cb, j0, jc, ntile_a, nblocks, X, c->scr,
-                     FuseV{});
+  hipLaunchKernelGGL((k_ht<F32, OT, TA, BK, NJ>), dim3(unsigned(grid)), dim3(kThreads), 0,
+                     c->stream, L, c->ldl, c->n, c->n_pad, cb, j0, jc, ntile_a, nblocks, X, c->scr);
   if (c->scr.lnorm) c->x_tiles += jc * ntile_a;
 }
 
-// AO tile width: FP64 defaults to 64 (more workgroups per CU); FP32 uses 128
-// while the accumulators fit (ot <= 6).  The context's ht_ta overrides
-// (autotuner).
-template <class P>
-inline int ht_tile(const Context *c, int ot) {
-  if (c->ht_ta == 64) return 64;
-  if (c->ht_ta == 128 && (ot <= 6 || std::is_same<P, F32>::value)) return 128;
-  if (std::is_same<P, F64>::value) return 64;
-  return ot <= 6 ? 128 : 64;
+// Column blocks per wave.  Few enough for three waves per SIMD up to five orbital
+// tiles (n=300 nocc=45: 0.32 ms with two blocks, 0.38 with four; n=512 nocc=64
+// 1.34 / 1.37 ms), two from there to ten tiles (n=536 nocc=98 2.81 ms, with one
+// block 2.91; n=1200 nocc=150 43.3 / 44.1 ms), one past that (registers).
+constexpr int ht64_nb(int ot) { return ot == 1 ? 4 : ot == 2 ? 3 : ot <= 10 ? 2 : 1; }
+
+template <int OT>
+void launch_ht64(Context *c, const double *cb, int64_t j0, int64_t jc, double *X) {
+  constexpr int NB = ht64_nb(OT);
+  const int64_t nblk = ceil_div(c->n, 16);
+  // fewer blocks per wave while the launch has less than two waves per SIMD
+  int nb = NB;
+  while (nb > 1 && jc * ceil_div(nblk, nb) < 8 * int64_t(c->ncu)) --nb;
+  const int W = int(ceil_div(nblk, nb));
+  const int64_t nblocks = ceil_div(jc * W, 4);
+  const dim3 grid(unsigned(round_up(nblocks, 8)));
+  if (c->fv.p) {  // fused Coulomb pass (never together with screening)
+    c->fv.ntile = W;
+    hipLaunchKernelGGL((k_ht64<OT, NB, true>), grid, dim3(kThreads), 0, c->stream, c->L, c->ldl, c->n, c->n_pad, cb,
+                       j0, jc, W, nb, nblocks, X, Screen{}, c->fv);
+    return;
+  }
+  hipLaunchKernelGGL((k_ht64<OT, NB, false>), grid, dim3(kThreads), 0, c->stream, c->L, c->ldl, c->n, c->n_pad, cb,
+                     j0, jc, W, nb, nblocks, X, c->scr, FuseV{});
+  if (c->scr.lnorm) c->x_tiles += jc * W;
 }
 
-// Wide banks: 128-wide AO tiles exist for FP32 only (the FP64 accumulators
-// of 8+ tiles at 128 columns would not fit the register file).
-template <class P, int OT>
-void launch_ht_w(Context *c, bool wide, const typename P::T *L, const typename P::T *cb,
-                 int64_t j0, int64_t jn, typename P::T *X) {
+void ht64_dispatch(Context *c, int ot, const double *cb, int64_t j0, int64_t jn, double *X) {
+  switch (ot) {
+    case 1: launch_ht64<1>(c, cb, j0, jn, X); break;
+    case 2: launch_ht64<2>(c, cb, j0, jn, X); break;
+    case 3: launch_ht64<3>(c, cb, j0, jn, X); break;
+    case 4: launch_ht64<4>(c, cb, j0, jn, X); break;
+    case 5: launch_ht64<5>(c, cb, j0, jn, X); break;
+    case 6: launch_ht64<6>(c, cb, j0, jn, X); break;
+    case 7: launch_ht64<7>(c, cb, j0, jn, X); break;
+    case 8: launch_ht64<8>(c, cb, j0, jn, X); break;
+    case 9: launch_ht64<9>(c, cb, j0, jn, X); break;
+    case 10: launch_ht64<10>(c, cb, j0, jn, X); break;
+    case 11: launch_ht64<11>(c, cb, j0, jn, X); break;
+    case 12: launch_ht64<12>(c, cb, j0, jn, X); break;
+    case 13: launch_ht64<13>(c, cb, j0, jn, X); break;
+    case 14: launch_ht64<14>(c, cb, j0, jn, X); break;
+    case 15: launch_ht64<15>(c, cb, j0, jn, X); break;
+    default: launch_ht64<16>(c, cb, j0, jn, X); break;
+  }
+}
+
+// FP32 AO tile width: 128 while the accumulators fit (ot <= 6), else 64; the
+// context's ht_ta overrides (autotuner).
+inline int ht_tile(const Context *c, int ot) { return c->ht_ta ? c->ht_ta : ot <= 6 ? 128 : 64; }
+
+template <int OT>
+void launch_ht_w(Context *c, bool wide, const float *L, const float *cb, int64_t j0, int64_t jn, float *X) {
   // 8-row chunks where the staging pieces divide, else 16 (odd OT)
   constexpr int BK = (8 * 16 * OT) % kThreads == 0 ? 8 : 16;
-  if constexpr (std::is_same<P, F32>::value) {
-    if (wide) return launch_ht<P, OT, 128, BK>(c, L, cb, j0, jn, X);
-  }
-  launch_ht<P, OT, 64, BK>(c, L, cb, j0, jn, X);
+  if (wide) return launch_ht<OT, 128, BK>(c, L, cb, j0, jn, X);
+  launch_ht<OT, 64, BK>(c, L, cb, j0, jn, X);
 }
 
-template <class P>
-void ht_dispatch(Context *c, int ot, const typename P::T *L, const typename P::T *cb, int64_t j0,
-                 int64_t jn, typename P::T *X) {
-  // BK = 8 where the staging pieces divide (16 for one or three tiles): small
-  // LDS buffers let more workgroups share a CU, hiding the load latency behind
-  // other workgroups' MFMAs (8% faster than BK = 16 at four tiles)
-  const bool wide = ht_tile<P>(c, ot) == 128;
+void ht32_dispatch(Context *c, int ot, const float *L, const float *cb, int64_t j0, int64_t jn, float *X) {
+  // BK = 8 where the staging pieces divide (16 for one or three tiles)
+  const bool wide = ht_tile(c, ot) == 128;
   switch (ot) {
-    case 1: wide ? launch_ht<P, 1, 128, 16>(c, L, cb, j0, jn, X) : launch_ht<P, 1, 64, 16>(c, L, cb, j0, jn, X); break;
-    case 2: wide ? launch_ht<P, 2, 128, 16>(c, L, cb, j0, jn, X) : launch_ht<P, 2, 64, 8>(c, L, cb, j0, jn, X); break;
-    case 3: wide ? launch_ht<P, 3, 128, 16>(c, L, cb, j0, jn, X) : launch_ht<P, 3, 64, 16>(c, L, cb, j0, jn, X); break;
-    case 4: wide ? launch_ht<P, 4, 128, 16>(c, L, cb, j0, jn, X) : launch_ht<P, 4, 64, 8>(c, L, cb, j0, jn, X); break;
-    case 5: wide ? launch_ht<P, 5, 128, 16>(c, L, cb, j0, jn, X) : launch_ht<P, 5, 64, 16>(c, L, cb, j0, jn, X); break;
-    case 6: wide ? launch_ht<P, 6, 128, 16>(c, L, cb, j0, jn, X) : launch_ht<P, 6, 64, 8>(c, L, cb, j0, jn, X); break;
-    case 7: launch_ht_w<P, 7>(c, wide, L, cb, j0, jn, X); break;
-    case 8: launch_ht_w<P, 8>(c, wide, L, cb, j0, jn, X); break;
-    case 10: launch_ht_w<P, 10>(c, wide, L, cb, j0, jn, X); break;
-    case 12: launch_ht_w<P, 12>(c, wide, L, cb, j0, jn, X); break;
-    case 14: launch_ht_w<P, 14>(c, wide, L, cb, j0, jn, X); break;
-    default: launch_ht_w<P, 16>(c, wide, L, cb, j0, jn, X); break;
+    case 1: wide ? launch_ht<1, 128, 16>(c, L, cb, j0, jn, X) : launch_ht<1, 64, 16>(c, L, cb, j0, jn, X); break;
+    case 2: wide ? launch_ht<2, 128, 16>(c, L, cb, j0, jn, X) : launch_ht<2, 64, 8>(c, L, cb, j0, jn, X); break;
+    case 3: wide ? launch_ht<3, 128, 16>(c, L, cb, j0, jn, X) : launch_ht<3, 64, 16>(c, L, cb, j0, jn, X); break;
+    case 4: wide ? launch_ht<4, 128, 16>(c, L, cb, j0, jn, X) : launch_ht<4, 64, 8>(c, L, cb, j0, jn, X); break;
+    case 5: wide ? launch_ht<5, 128, 16>(c, L, cb, j0, jn, X) : launch_ht<5, 64, 16>(c, L, cb, j0, jn, X); break;
+    case 6: wide ? launch_ht<6, 128, 16>(c, L, cb, j0, jn, X) : launch_ht<6, 64, 8>(c, L, cb, j0, jn, X); break;
+    case 7: launch_ht_w<7>(c, wide, L, cb, j0, jn, X); break;
+    case 8: launch_ht_w<8>(c, wide, L, cb, j0, jn, X); break;
+    case 10: launch_ht_w<10>(c, wide, L, cb, j0, jn, X); break;
+    case 12: launch_ht_w<12>(c, wide, L, cb, j0, jn, X); break;
+    case 14: launch_ht_w<14>(c, wide, L, cb, j0, jn, X); break;
+    default: launch_ht_w<16>(c, wide, L, cb, j0, jn, X); break;
   }
 }
 
@@ -1426,9 +1759,10 @@ int pack_bank_b3(Context *c, int32_t nk, const int32_t *nocc, const double *cons
   return MJK_OK;
 }
 
-// Layout of the bank for nk sets; returns MJK_OK and ot = 0 when empty.
+// Layout of the bank for nk sets; returns MJK_OK and ot = 0 when empty.  The
+// reduced-precision kernels exist for even widths above eight tiles only.
 int bank_layout(Context *c, int32_t nk, const int32_t *nocc, std::vector<int> &off,
-                std::vector<int> &opad, int *ot_out, int *tot_out) {
+                std::vector<int> &opad, bool fp64_only, int *ot_out, int *tot_out) {
   off.assign(size_t(nk), 0);
   opad.assign(size_t(nk), 0);
   int tot = 0;
@@ -1442,12 +1776,12 @@ int bank_layout(Context *c, int32_t nk, const int32_t *nocc, std::vector<int> &o
   *tot_out = tot;
   *ot_out = 0;
   if (tot == 0) return MJK_OK;
-  static const int kOT[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16};
-  for (int v : kOT)
-    if (16 * v >= tot) {
-      *ot_out = v;
-      return MJK_OK;
-    }
+  int ot = int(ceil_div(tot, 16));
+  if (!fp64_only && ot > 8) ot = int(round_up(ot, 2));
+  if (ot <= 16) {
+    *ot_out = ot;
+    return MJK_OK;
+  }
   return set_error(c, MJK_ERR_ARG, "more than 256 orbital columns in one call");
 }
 
@@ -1541,16 +1875,17 @@ int exchange_segments(Context *c, int32_t nk, const int32_t *nocc, const double 
   if (nk > kMaxSets) return set_error(c, MJK_ERR_ARG, "exchange: more than 16 orbital sets");
   std::vector<int> off, opad;
   int ot = 0, tot = 0;
-  if ((rc = bank_layout(c, nk, nocc, off, opad, &ot, &tot))) return rc;
+  bool use[3] = {false, false, false};
+  for (const Segment &s : segs)
+    if (s.j1 > s.j0) use[s.prec] = true;
+  if ((rc = bank_layout(c, nk, nocc, off, opad, !use[MJK_PREC_FP32] && !use[MJK_PREC_BF16X3], &ot, &tot)))
+    return rc;
   if (tot == 0) {  // no orbitals: K = 0
     for (int d = 0; d < nk; ++d)
       if ((rc = fill_zero(c, klt + d * ldk, sizeof(double) * c->np))) return rc;
     return MJK_OK;
   }
   const int ldc = 16 * ot;
-  bool use[3] = {false, false, false};
-  for (const Segment &s : segs)
-    if (s.j1 > s.j0) use[s.prec] = true;
   const bool zsave = c->zs.z != nullptr;
   if (zsave && (nk != 1 || nocc[0] != c->zs.nocc))
     return set_error(c, MJK_ERR_ARG, "exchange: Z output needs exactly one orbital set");
@@ -1669,11 +2004,11 @@ int exchange_segments(Context *c, int32_t nk, const int32_t *nocc, const double 
       phase_begin(c);
       switch (s.prec) {
         case MJK_PREC_FP64:
-          ht_dispatch<F64>(c, ot, c->L, static_cast<const double *>(c->w->cbank.ptr), j0, jn,
-                           static_cast<double *>(c->w->x.ptr));
+          ht64_dispatch(c, ot, static_cast<const double *>(c->w->cbank.ptr), j0, jn,
+                        static_cast<double *>(c->w->x.ptr));
           break;
         case MJK_PREC_FP32:
-          ht_dispatch<F32>(c, ot, L32, static_cast<const float *>(c->w->cb32.ptr), j0, jn,
+          ht32_dispatch(c, ot, L32, static_cast<const float *>(c->w->cb32.ptr), j0, jn,
                            static_cast<float *>(c->w->x.ptr));
           break;
         default: {
@@ -1695,11 +2030,11 @@ int exchange_segments(Context *c, int32_t nk, const int32_t *nocc, const double 
         if (s.prec == MJK_PREC_FP64)
           hipLaunchKernelGGL(k_xnorms<double>, dim3(unsigned(jn), unsigned(nstrip), unsigned(nk)),
                              dim3(kThreads), 0, c->stream, static_cast<const double *>(c->w->x.ptr),
-                             ldc, n_pad, sets, nstrip, xn2);
+                             ldc, n, n_pad, sets, nstrip, xn2);
         else
           hipLaunchKernelGGL(k_xnorms<float>, dim3(unsigned(jn), unsigned(nstrip), unsigned(nk)),
                              dim3(kThreads), 0, c->stream, static_cast<const float *>(c->w->x.ptr),
-                             ldc, n_pad, sets, nstrip, xn2);
+                             ldc, n, n_pad, sets, nstrip, xn2);
         c->scr.xn2 = xn2;
       }
       phase_begin(c);
@@ -1729,13 +2064,13 @@ int exchange_segments(Context *c, int32_t nk, const int32_t *nocc, const double 
 
 int pack_bank(Context *c, int32_t nk, const int32_t *nocc, const double *const *corb,
               std::vector<int> &off, std::vector<int> &opad, int *ot, int *tot) {
-  int rc = bank_layout(c, nk, nocc, off, opad, ot, tot);
+  int rc = bank_layout(c, nk, nocc, off, opad, true, ot, tot);
   if (rc || *tot == 0) return rc;
   return pack_bank_t<double>(c, nk, nocc, corb, off, 16 * *ot, c->w->cbank);
 }
 
 void ht_launch(Context *c, int ot, const double *cb, int64_t j0, int64_t jn, double *X) {
-  ht_dispatch<F64>(c, ot, c->L, cb, j0, jn, X);
+  ht64_dispatch(c, ot, cb, j0, jn, X);
 }
 
 int exchange(Context *c, int32_t nk, const int32_t *nocc, const double *const *corb, double *klt,

@@ -1,7 +1,8 @@
 // Autotuner of the exchange tiling: for the orbital sets of one call it times
-// every combination of SYRK tile (64, 128), SYRK workgroups per launch (1, 2, 4
-// or 8 rounds of two per CU) and half-transform AO tile (64, 128) with HIP
-// events and keeps the fastest in the context.  Every point runs once untimed
+// every combination of SYRK workgroups per launch (as planned, or 1, 2, 4 or 8
+// rounds of two per CU) and, in reduced precision, SYRK tile (64, 128) and
+// half-transform AO tile (64, 128) with HIP events and keeps the fastest in the
+// context.  Every point runs once untimed
 // (so a switch of tiling pays its workspace growth and cold caches outside the
 // clock) and is then timed kRuns times back to back; the median decides, so
 // one slow run (a clock ramp, another queue's work) cannot pick the tiling.
@@ -30,7 +31,8 @@ extern "C" int mjk_autotune(mjk_context *c, int32_t nk, const int32_t *nocc,
     if ((rc = hip_check(c, hipEventCreate(&e0[r]), "event")) == MJK_OK)
       rc = hip_check(c, hipEventCreate(&e1[r]), "event");
   const int tms[] = {64, 128};
-  const int splits[] = {2 * c->ncu, 4 * c->ncu, 8 * c->ncu, 16 * c->ncu};
+  const bool fp64 = precision == MJK_PREC_FP64;  // its kernels choose their own tiles
+  const int splits[] = {0, 2 * c->ncu, 4 * c->ncu, 8 * c->ncu, 16 * c->ncu};  // 0: the planned slices
   const int tas[] = {64, 128};
   float best = 1e30f;
   int bt = 0, bs = 0, ba = 0;
@@ -39,9 +41,10 @@ extern "C" int mjk_autotune(mjk_context *c, int32_t nk, const int32_t *nocc,
   c->tile_syrk = c->split_target = c->ht_ta = 0;
   if ((rc = exchange(c, nk, nocc, corb, klt, ldk, precision))) goto done;
   for (int tm : tms) {
-    if (c->n_pad % tm || (precision == MJK_PREC_FP64 && tm != 64)) continue;  // the FP64 SYRK has one tile
+    if (c->n_pad % tm || (fp64 && tm != 64)) continue;
     for (int sp : splits) {
       for (int ta : tas) {
+        if (fp64 && ta != 64) continue;
         c->tile_syrk = tm;
         c->split_target = sp;
         c->ht_ta = ta;
@@ -66,9 +69,9 @@ extern "C" int mjk_autotune(mjk_context *c, int32_t nk, const int32_t *nocc,
       }
     }
   }
-  c->tile_syrk = bt;
+  c->tile_syrk = fp64 ? 0 : bt;
   c->split_target = bs;
-  c->ht_ta = ba;
+  c->ht_ta = fp64 ? 0 : ba;
   if (best_ms) *best_ms = best;
 done:
   for (int r = 0; r < kRuns; ++r) {
