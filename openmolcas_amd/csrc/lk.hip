@@ -9,13 +9,24 @@
 // the half-transform X_k = L C_k (sqrt|SumAClk(b,k) SvShp(ab)| >= thrv), and
 // which K blocks (a >= b) receive X_k,a X_k,b^T (MLk(a) MLk(b) >= tau,
 // sqrt|Faa(a) Faa(b)| >= tau/MaxRed, Keep flags).  The same decisions are
-// made here; the arithmetic is tiled for the GPU:
-//   - the half-transform stages 64 x 64 tiles of the packed vector in LDS and
-//     each thread accumulates one AO row for four orbitals, the mask of a
-//     (orbital, shell a, shell b) triple evaluated once per b-shell run;
-//   - the K kernel owns a 64 x 64 tile of the lower triangle, stages the
-//     batch's X rows of both tile sides per orbital and skips orbitals whose
-//     mask is empty on the tile;
+// made here.  Between two evaluations of the shell lists (DoScreen) the batches
+// do not depend on each other, so a group of batches goes through each kernel
+// together; the decisions of one orbital become one bit of a 64-bit word, a word
+// per (shell, shell) and 64 orbitals, which a wave forms with one ballot:
+//   - the half-transform takes one shell a at a time, because for a fixed a the
+//     mask depends on (orbital, b) only and can be applied to the orbital
+//     operand: X_k(J, a) = sum_b [m C](k, b) L_J(a, b) is an MFMA product with
+//     columns (J, a in the shell); steps of four b no orbital needs are left out;
+//   - the K kernel forms S_k = sum_J X_k X_k^T of one orbital on a 32 x 32 tile
+//     by MFMA and adds it under the mask of (orbital, shell a, shell b),
+//     skipping orbitals whose mask is empty on the tile;
+// Measured on a chain of 48 atoms (n=240, nchol=1200 in 48 batches, 48 orbitals),
+// whole call: 33.2 -> 0.96 ms.  One batch at a time, each kernel had 10-144
+// workgroups of serial work (K 0.35 ms per batch, half-transform 0.14, lists
+// 0.06, norms 0.05); now per call 0.04, 0.18 (bound by its gathered loads of L,
+// one cache line per lane), 0.13 (masks, bound by their scalar loads), 0.11
+// (reads L once), K-block masks 0.09.  The MFMA sums run in the order of the
+// scalar loops they replace: the result is bit for bit the same.
 //   - decision quantities (diagonal, SvShp, SumAClk, Y, Faa) are evaluated
 //     without FMA contraction, in the reference's summation order where it
 //     has one, so the cuts fall where the reference's fall.
@@ -25,6 +36,7 @@
 // monotone, that set is exactly {s : MLk(s) max MLk >= tau} (SCF) or
 // {s : MLk(s) >= sqrt(tau)} (CASSCF), which is what the list kernel forms.
 #include <cmath>
+#include <limits>
 
 #include "mjk_internal.h"
 
@@ -32,30 +44,47 @@ namespace mjk {
 namespace {
 
 constexpr int kLkBatch = 25;  // Cho_LK_MaxVecPerBatch (src/fock_util/cho_lk_maxvecperbatch.F90:30)
-constexpr int kT = 64;        // AO tile
-constexpr int kKc = 16;       // orbitals per half-transform workgroup
 constexpr int kLkThreads = 256;
+constexpr int kLkGroup = 64;  // most batches that go through the kernels together
+constexpr int kHtCols = 48;   // columns (J, a) of one half-transform wave
+constexpr int kHtPanel = 1024;  // contraction indices b listed at a time
 
 __device__ __forceinline__ int64_t shp_idx(int a, int b) {
   return a >= b ? int64_t(a) * (a + 1) / 2 + b : int64_t(b) * (b + 1) / 2 + a;
 }
 
 // One or two densities: orbital counts, first global orbital index, device
-// orbital matrices (orbital-major), thresholds.
+// orbital matrices (orbital-major), thresholds.  Mask words: density d owns the
+// words q0[d] .. q0[d+1]-1, word q the orbitals 64 (q - q0[d]) .. of it.
 struct LkDens {
   int nd;
   int nocc[2];
   int k0[2];           // global orbital offset of density d
-  int nkc[2];          // half-transform chunks of density d
+  int q0[3];
   const double *c[2];  // C_d(b, k) at k + nocc[d]*b
-  double tau[2], thrv[2], xtau[2];
+  double tau[2], xtau[2];
+  double thrv2[2];     // least x with sqrt(x) >= thrv
+  double tk2[2];       // least x with sqrt(x) >= tau / MaxRed
   int ktot;            // sum of nocc
+  int nq;              // words
+};
+
+// The batches of one group.
+struct LkGroup {
+  int nb;
+  int64_t j0[kLkGroup];
+  int jnum[kLkGroup];
+  const uint8_t *present[kLkGroup];  // shell-pair occupancy of the batch's reduced set
 };
 
 __device__ __forceinline__ void dk_of(const LkDens &D, int g, int *d, int *k) {
   *d = (D.nd > 1 && g >= D.k0[1]) ? 1 : 0;
   *k = g - D.k0[*d];
 }
+__device__ __forceinline__ int d_of_word(const LkDens &D, int q) { return D.nd > 1 && q >= D.q0[1] ? 1 : 0; }
+// Row length and position of orbital k of density d in the arrays that hold one
+// value per (shell, orbital), orbital fastest, words aligned.
+__device__ __forceinline__ int kpos(const LkDens &D, int d, int k) { return 64 * D.q0[d] + k; }
 
 #pragma clang fp contract(off)
 
@@ -88,13 +117,50 @@ __global__ void k_lk_update_diag(const double *__restrict__ L, int64_t ldl, int6
 }
 
 // SvShp(ab) = max_J sum_{p in shell pair ab} L_J(p)^2 (CHO_GetShFull,
-// src/fock_util/cho_getshfull.F90:48-96): one wave per shell pair.
+// src/fock_util/cho_getshfull.F90:48-96).  Small shells (kSmallShell functions
+// at most): one lane per shell pair, a wave the pairs of one shell a with 64
+// shells b, whose packed elements are neighbours in the rows of a.  grid =
+// (shells a, ceil(nshell / 256), batches).
+constexpr int kSmallShell = 8;
 __global__ __launch_bounds__(kLkThreads) void k_lk_svshp(const double *__restrict__ L, int64_t ldl,
-                                                         int64_t j0, int jnum, int nshell,
+                                                         const LkGroup G, int nshell,
                                                          const int32_t *__restrict__ koff,
                                                          const int32_t *__restrict__ nbsh,
-                                                         double *__restrict__ sv) {
-  const int lane = threadIdx.x & 63;
+                                                         double *__restrict__ svall) {
+  constexpr int U = 5;  // vectors in flight
+  const int sa = blockIdx.x, sb = blockIdx.y * kLkThreads + threadIdx.x, bt = blockIdx.z;
+  if (sb > sa) return;
+  const int na = nbsh[sa], nb = nbsh[sb], a0 = koff[sa], b0 = koff[sb];
+  const double *__restrict__ base = L + G.j0[bt] * ldl;
+  const int jnum = G.jnum[bt];
+  double best = 0.0;
+  for (int j = 0; j < jnum; j += U) {
+    double s[U] = {};
+    for (int al = 0; al < na; ++al) {
+      const int64_t row = int64_t(a0 + al) * (a0 + al + 1) / 2 + b0;
+      const int nbe = sa == sb ? al + 1 : nb;
+      for (int bl = 0; bl < nbe; ++bl) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const double v = base[(j + u < jnum ? j + u : j) * ldl + row + bl];
+          s[u] = s[u] + v * v;
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) best = s[u] > best ? s[u] : best;  // max(SvShp(:,1), SvShp(:,2))
+  }
+  svall[bt * (int64_t(nshell) * (nshell + 1) / 2) + shp_idx(sa, sb)] = best;
+}
+
+// The same for shells of any size: one wave per shell pair.  grid = (pairs / 4,
+// batches).
+__global__ __launch_bounds__(kLkThreads) void k_lk_svshp_wave(const double *__restrict__ L, int64_t ldl,
+                                                              const LkGroup G, int nshell,
+                                                              const int32_t *__restrict__ koff,
+                                                              const int32_t *__restrict__ nbsh,
+                                                              double *__restrict__ svall) {
+  const int lane = threadIdx.x & 63, bt = blockIdx.y;
   const int64_t nshp = int64_t(nshell) * (nshell + 1) / 2;
   const int64_t p = int64_t(blockIdx.x) * (kLkThreads / 64) + (threadIdx.x >> 6);
   if (p >= nshp) return;
@@ -103,30 +169,22 @@ __global__ __launch_bounds__(kLkThreads) void k_lk_svshp(const double *__restric
   while (int64_t(sa + 1) * (sa + 2) / 2 <= p) ++sa;
   const int sb = int(p - int64_t(sa) * (sa + 1) / 2);
   const int na = nbsh[sa], nb = nbsh[sb], a0 = koff[sa], b0 = koff[sb];
-  const int ne = sa == sb ? na * (na + 1) / 2 : na * nb;
   double best = 0.0;
-  for (int j = 0; j < jnum; ++j) {
-    const double *row = L + (j0 + j) * ldl;
+  for (int j = 0; j < G.jnum[bt]; ++j) {
+    const double *__restrict__ row = L + (G.j0[bt] + j) * ldl;
     double s = 0.0;
-    for (int e = lane; e < ne; e += 64) {
-      int al, bl;
-      if (sa == sb) {
-        al = int((sqrt(8.0 * double(e) + 1.0) - 1.0) * 0.5);
-        while (al * (al + 1) / 2 > e) --al;
-        while ((al + 1) * (al + 2) / 2 <= e) ++al;
-        bl = e - al * (al + 1) / 2;
-      } else {
-        al = e % na;
-        bl = e / na;
+    for (int al = 0; al < na; ++al) {
+      const int64_t a = a0 + al;
+      const int nbe = sa == sb ? al + 1 : nb;
+      for (int bl = lane; bl < nbe; bl += 64) {
+        const double v = row[a * (a + 1) / 2 + b0 + bl];
+        s = s + v * v;
       }
-      const int64_t a = a0 + al, b = b0 + bl;
-      const double v = row[a * (a + 1) / 2 + b];
-      s = s + v * v;
     }
     for (int off = 32; off > 0; off >>= 1) s = s + __shfl_xor(s, off, 64);
-    best = s > best ? s : best;  // max(SvShp(:,1), SvShp(:,2))
+    best = s > best ? s : best;
   }
-  if (lane == 0) sv[p] = best;
+  if (lane == 0) svall[bt * nshp + p] = best;
 }
 
 // DH(a,b) = DH(b,a) = sqrt|D(ab)| (swap_tosqrt, src/fock_util/swap_tosqrt.F90:57-72).
@@ -139,7 +197,8 @@ __global__ void k_lk_diah(const double *__restrict__ diag, int n, double *__rest
   }
 }
 
-// SumAClk(s,k) = sum_{i in s} C(i,k)^2 (cho_lk_scf.F90:235-253).
+// SumAClk(s,k) = sum_{i in s} C(i,k)^2 (cho_lk_scf.F90:235-253), at
+// sumac[s * 64 nq + kpos].
 __global__ void k_lk_sumac(LkDens D, int nshell, const int32_t *__restrict__ koff,
                            const int32_t *__restrict__ nbsh, double *__restrict__ sumac) {
   int d, k;
@@ -152,295 +211,458 @@ __global__ void k_lk_sumac(LkDens D, int nshell, const int32_t *__restrict__ kof
       const double v = c[k + int64_t(no) * (koff[s] + i)];
       t = t + v * v;
     }
-    sumac[int64_t(blockIdx.x) * nshell + s] = t;
+    sumac[int64_t(s) * 64 * D.nq + kpos(D, d, k)] = t;
   }
 }
 
-// Per orbital (one workgroup each): when screening, Y = DH |C_k| (DGEMV 'N',
-// :584-590), MLk per shell, the listed shells; then, every batch, Keep and the
-// number of half-transformed shell pairs (:659-702).
-__global__ __launch_bounds__(kLkThreads) void k_lk_lists(
-    LkDens D, int n, int nshell, int doscreen, int cas_cut, const int32_t *__restrict__ koff,
+// Per orbital (one workgroup each): Y = DH |C_k| (DGEMV 'N', :584-590), MLk per
+// shell, the listed shells (:602-627).
+__global__ __launch_bounds__(kLkThreads) void k_lk_screen(
+    LkDens D, int n, int nshell, int cas_cut, const int32_t *__restrict__ koff,
     const int32_t *__restrict__ nbsh, const double *__restrict__ dh, double *__restrict__ ylk,
-    double *__restrict__ mlk, uint8_t *__restrict__ listed, const double *__restrict__ sumac,
-    const double *__restrict__ sv, const uint8_t *__restrict__ present, uint8_t *__restrict__ keep,
-    unsigned long long *__restrict__ stats) {
+    double *__restrict__ mlk, uint8_t *__restrict__ listed, unsigned long long *__restrict__ stats) {
+  constexpr int U = 16;  // rows of DH in flight
   __shared__ double red[kLkThreads / 64];
-  __shared__ unsigned long long cnt[2];
-  const int g = blockIdx.x;
-  int d, k;
-  dk_of(D, g, &d, &k);
-  const int64_t so = int64_t(g) * nshell;
-  if (threadIdx.x == 0) cnt[0] = cnt[1] = 0;
-  if (doscreen) {
-    const double *c = D.c[d];
-    const int no = D.nocc[d];
-    double *y = ylk + int64_t(g) * n;
-    for (int l = threadIdx.x; l < n; l += blockDim.x) {
-      double s = 0.0;
-      for (int m = 0; m < n; ++m) s = s + dh[int64_t(m) * n + l] * fabs(c[k + int64_t(no) * m]);
-      y[l] = s;
-    }
-    __syncthreads();
-    double mx = 0.0;
-    for (int s = threadIdx.x; s < nshell; s += blockDim.x) {
-      double ym = 0.0;
-      for (int i = 0; i < nbsh[s]; ++i) ym = fmax(ym, y[koff[s] + i]);
-      mlk[so + s] = ym;
-      mx = fmax(mx, ym);
-    }
-    for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
-    __syncthreads();
-    mx = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
-    unsigned long long nl = 0;
-    for (int s = threadIdx.x; s < nshell; s += blockDim.x) {
-      const double m = mlk[so + s];
-      const bool ok = cas_cut ? (m >= D.xtau[d]) : (m * mx >= D.tau[d]);
-      listed[so + s] = ok ? 1 : 0;
-      nl += ok;
-    }
-    if (nl) atomicAdd(&cnt[0], nl);
-  }
-  __syncthreads();
-  unsigned long long nh = 0;
-  const double *sa_c = sumac + so;
-  for (int sa = threadIdx.x; sa < nshell; sa += blockDim.x) {
-    int count = 0;
-    if (listed[so + sa])
-      for (int sb = 0; sb < nshell; ++sb) {
-        const int64_t p = shp_idx(sa, sb);
-        if (!present[p] || nbsh[sa] * nbsh[sb] <= 0) continue;
-        if (sqrt(fabs(sa_c[sb] * sv[p])) >= D.thrv[d]) ++count;
-      }
-    keep[so + sa] = count > 0 ? 1 : 0;
-    nh += count;
-  }
-  if (nh) atomicAdd(&cnt[1], nh);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    if (cnt[0]) atomicAdd(&stats[0], cnt[0]);
-    if (cnt[1]) atomicAdd(&stats[1], cnt[1]);
-  }
-}
-
-// Faa(a) = max_{i in a} |sum_J X(i,J)^2| for listed, kept shells (:713-743),
-// then the number of K blocks the pair cuts keep (:749-830).
-__global__ __launch_bounds__(kLkThreads) void k_lk_faa(
-    LkDens D, int n_pad, int jnum, int nshell, const int32_t *__restrict__ koff,
-    const int32_t *__restrict__ nbsh, const double *__restrict__ X, const uint8_t *__restrict__ listed,
-    const uint8_t *__restrict__ keep, const double *__restrict__ mlk, double *__restrict__ faa,
-    double maxred, unsigned long long *__restrict__ stats) {
   __shared__ unsigned long long cnt;
   const int g = blockIdx.x;
   int d, k;
   dk_of(D, g, &d, &k);
-  const int64_t so = int64_t(g) * nshell;
+  const int64_t ld = 64 * int64_t(D.nq);
+  const int kp = kpos(D, d, k);
   if (threadIdx.x == 0) cnt = 0;
-  const double *x = X + int64_t(g) * jnum * n_pad;
+  const double *c = D.c[d];
+  const int no = D.nocc[d];
+  double *y = ylk + int64_t(g) * n;
+  for (int l = threadIdx.x; l < n; l += blockDim.x) {
+    double s = 0.0;
+    int m = 0;
+    for (; m + U <= n; m += U) {
+      double v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = dh[int64_t(m + u) * n + l];
+#pragma unroll
+      for (int u = 0; u < U; ++u) s = s + v[u] * fabs(c[k + int64_t(no) * (m + u)]);
+    }
+    for (; m < n; ++m) s = s + dh[int64_t(m) * n + l] * fabs(c[k + int64_t(no) * m]);
+    y[l] = s;
+  }
+  __syncthreads();
+  double mx = 0.0;
+  for (int s = threadIdx.x; s < nshell; s += blockDim.x) {
+    double ym = 0.0;
+    for (int i = 0; i < nbsh[s]; ++i) ym = fmax(ym, y[koff[s] + i]);
+    mlk[s * ld + kp] = ym;
+    mx = fmax(mx, ym);
+  }
+  for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  mx = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+  unsigned long long nl = 0;
+  for (int s = threadIdx.x; s < nshell; s += blockDim.x) {
+    const double m = mlk[s * ld + kp];
+    const bool ok = cas_cut ? (m >= D.xtau[d]) : (m * mx >= D.tau[d]);
+    listed[s * ld + kp] = ok ? 1 : 0;
+    nl += ok;
+  }
+  if (nl) atomicAdd(&cnt, nl);
+  __syncthreads();
+  if (threadIdx.x == 0 && cnt) atomicAdd(&stats[0], cnt);
+}
+
+// The half-transform's masks: bit k of word mw[((bt nq + q) nshell + sa) nshell
+// + sb] = orbital k lists shell a and takes the pair (:659-702); kw[(bt nq + q)
+// nshell + sa] = Keep(a).  Rows of shells with no kept orbital are not written.
+// One lane per orbital.  grid = (shells a, batches * words).
+__global__ __launch_bounds__(kLkThreads) void k_lk_mask(
+    LkDens D, const LkGroup G, int nshell, const int32_t *__restrict__ nbsh,
+    const uint8_t *__restrict__ listed, const double *__restrict__ sumac, const double *__restrict__ svall,
+    unsigned long long *__restrict__ mw, unsigned long long *__restrict__ kw,
+    unsigned long long *__restrict__ stats) {
+  constexpr int U = 4;  // shells b in flight per wave
+  __shared__ unsigned long long keep[kLkThreads / 64], cnt[kLkThreads / 64];
+  const int sa = blockIdx.x, bt = blockIdx.y / D.nq, q = blockIdx.y % D.nq;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int d = d_of_word(D, q), k = 64 * (q - D.q0[d]) + lane;
+  const int64_t ld = 64 * int64_t(D.nq), col = 64 * int64_t(q) + lane;
+  const double *__restrict__ sv = svall + bt * (int64_t(nshell) * (nshell + 1) / 2);
+  const uint8_t *__restrict__ present = G.present[bt];
+  const double thr = D.thrv2[d];
+  const bool l = k < D.nocc[d] && listed[sa * ld + col] != 0;
+  unsigned long long kept = 0, n = 0;
+  if (__ballot(l) != 0 && nbsh[sa] > 0) {
+    unsigned long long *__restrict__ row = mw + ((int64_t(bt) * D.nq + q) * nshell + sa) * nshell;
+    for (int s0 = w * U; s0 < nshell; s0 += (kLkThreads / 64) * U) {
+      double x[U];
+      bool ok[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int sb = s0 + u < nshell ? s0 + u : nshell - 1;
+        const int64_t p = shp_idx(sa, sb);
+        ok[u] = l && present[p] != 0 && nbsh[sb] > 0;
+        x[u] = sumac[sb * ld + col] * sv[p];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (s0 + u >= nshell) break;
+        const unsigned long long b = __ballot(ok[u] && fabs(x[u]) >= thr);
+        kept |= b;
+        n += __popcll(b);
+        if (lane == 0) row[s0 + u] = b;
+      }
+    }
+  }
+  if (lane == 0) {
+    keep[w] = kept;
+    cnt[w] = n;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    kw[(int64_t(bt) * D.nq + q) * nshell + sa] = (keep[0] | keep[1]) | (keep[2] | keep[3]);
+    const unsigned long long t = (cnt[0] + cnt[1]) + (cnt[2] + cnt[3]);
+    if (t) atomicAdd(&stats[1], t);
+  }
+}
+
+// Faa(a) = max_{i in a} |sum_J X(i,J)^2| (:713-743) at faa[(bt nshell + s) 64 nq
+// + kpos], for the kept shells of each orbital.  grid = (orbitals, batches).
+__global__ __launch_bounds__(kLkThreads) void k_lk_faa(
+    LkDens D, const LkGroup G, int n_pad, int nshell, const int32_t *__restrict__ koff,
+    const int32_t *__restrict__ nbsh, const double *__restrict__ X, const unsigned long long *__restrict__ kw,
+    double *__restrict__ faa) {
+  const int g = blockIdx.x, bt = blockIdx.y, jnum = G.jnum[bt];
+  int d, k;
+  dk_of(D, g, &d, &k);
+  const int q = D.q0[d] + k / 64;
+  const int64_t ld = 64 * int64_t(D.nq);
+  const double *__restrict__ x = X + (int64_t(bt) * D.ktot + g) * kLkBatch * n_pad;
   for (int s = threadIdx.x; s < nshell; s += blockDim.x) {
     double t = 0.0;
-    if (listed[so + s] && keep[so + s])
+    if ((kw[(int64_t(bt) * D.nq + q) * nshell + s] >> (k & 63)) & 1ull)
       for (int i = 0; i < nbsh[s]; ++i) {
         double f = 0.0;
-        for (int j = 0; j < jnum; ++j) {
-          const double v = x[int64_t(j) * n_pad + koff[s] + i];
-          f = f + v * v;
-        }
+        double v[kLkBatch];
+#pragma unroll
+        for (int j = 0; j < kLkBatch; ++j) v[j] = x[int64_t(j < jnum ? j : 0) * n_pad + koff[s] + i];
+#pragma unroll
+        for (int j = 0; j < kLkBatch; ++j) f = j < jnum ? f + v[j] * v[j] : f;
         t = fmax(t, fabs(f));
       }
-    faa[so + s] = t;
+    faa[(int64_t(bt) * nshell + s) * ld + kpos(D, d, k)] = t;
   }
-  __syncthreads();
+}
+
+// The K blocks each orbital keeps (:749-830): word pw[(bt nq + q) nshp + pair].
+// grid = (shells a, batches * words).
+__global__ __launch_bounds__(kLkThreads) void k_lk_pairs(
+    LkDens D, int nshell, const unsigned long long *__restrict__ kw, const double *__restrict__ mlk,
+    const double *__restrict__ faa, unsigned long long *__restrict__ pw, unsigned long long *__restrict__ stats) {
+  constexpr int U = 4;
+  __shared__ unsigned long long cnt[kLkThreads / 64];
+  const int sa = blockIdx.x, bt = blockIdx.y / D.nq, q = blockIdx.y % D.nq;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int d = d_of_word(D, q);
+  const int64_t ld = 64 * int64_t(D.nq), col = 64 * int64_t(q) + lane;
   const int64_t nshp = int64_t(nshell) * (nshell + 1) / 2;
-  unsigned long long c = 0;
-  const double tau = D.tau[d], tk = D.tau[d] / maxred;
-  for (int64_t p = threadIdx.x; p < nshp; p += blockDim.x) {
-    int sa = int((sqrt(8.0 * double(p) + 1.0) - 1.0) * 0.5);
-    while (int64_t(sa) * (sa + 1) / 2 > p) --sa;
-    while (int64_t(sa + 1) * (sa + 2) / 2 <= p) ++sa;
-    const int sb = int(p - int64_t(sa) * (sa + 1) / 2);
-    if (!listed[so + sa] || !listed[so + sb] || !keep[so + sa] || !keep[so + sb]) continue;
-    if (mlk[so + sa] * mlk[so + sb] < tau) continue;
-    if (!(sqrt(fabs(faa[so + sa] * faa[so + sb])) >= tk)) continue;
-    ++c;
+  const unsigned long long *__restrict__ kb = kw + (int64_t(bt) * D.nq + q) * nshell;
+  const double *__restrict__ fb = faa + int64_t(bt) * nshell * ld;
+  unsigned long long *__restrict__ row = pw + (int64_t(bt) * D.nq + q) * nshp + int64_t(sa) * (sa + 1) / 2;
+  const unsigned long long ka = kb[sa];
+  const double tau = D.tau[d], tk = D.tk2[d];
+  unsigned long long n = 0;
+  if (ka == 0) {
+    for (int sb = threadIdx.x; sb <= sa; sb += kLkThreads) row[sb] = 0;
+  } else {
+    const bool la = (ka >> lane) & 1ull;
+    const double ma = la ? mlk[sa * ld + col] : 0.0, fa = la ? fb[sa * ld + col] : 0.0;
+    for (int s0 = w * U; s0 <= sa; s0 += (kLkThreads / 64) * U) {
+      unsigned long long k2[U];
+      double m[U], f[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int sb = s0 + u <= sa ? s0 + u : sa;
+        k2[u] = kb[sb];
+        m[u] = mlk[sb * ld + col];
+        f[u] = fb[sb * ld + col];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (s0 + u > sa) break;
+        const bool ok = la && ((k2[u] >> lane) & 1ull) && !(ma * m[u] < tau) && fabs(fa * f[u]) >= tk;
+        const unsigned long long b = __ballot(ok);
+        n += __popcll(b);
+        if (lane == 0) row[s0 + u] = b;
+      }
+    }
   }
-  if (c) atomicAdd(&cnt, c);
+  if (lane == 0) cnt[w] = n;
   __syncthreads();
-  if (threadIdx.x == 0 && cnt) atomicAdd(&stats[2], cnt);
+  if (threadIdx.x == 0) {
+    const unsigned long long t = (cnt[0] + cnt[1]) + (cnt[2] + cnt[3]);
+    if (t) atomicAdd(&stats[2], t);
+  }
 }
 
 #pragma clang fp contract(fast)
 
-// Masked half-transform of one vector: X(g, J, a) = sum_b m(g, sa, sb) L_J(a,b)
-// C(b, k) for the listed shells a of orbital g = (d, k), zero elsewhere.
-// Workgroup: 64 AOs a x 16 orbitals of one density, one vector J.
-__global__ __launch_bounds__(kLkThreads) void k_lk_ht(
-    LkDens D, const double *__restrict__ L, int64_t ldl, int64_t j0, int jnum, int n, int n_pad,
-    int nshell, const int32_t *__restrict__ shell, const double *__restrict__ sumac,
-    const double *__restrict__ sv, const uint8_t *__restrict__ present,
-    const uint8_t *__restrict__ listed, double *__restrict__ X) {
-  __shared__ double tl[kT][kT + 1];
-  __shared__ double tc[kT][kKc];
-  __shared__ int tsb[kT];
-  const int tid = threadIdx.x, al = tid & 63, kq = tid >> 6;
-  const int a0 = blockIdx.x * kT, jr = blockIdx.y;
-  int d = 0, ch = blockIdx.z;
-  if (D.nd > 1 && ch >= D.nkc[0]) {
-    d = 1;
-    ch -= D.nkc[0];
-  }
-  const int kbase = ch * kKc, no = D.nocc[d];
-  const double *c = D.c[d];
-  const double *row = L + (j0 + jr) * ldl;
-  const int a = a0 + al;
-  const int sa = a < n ? shell[a] : -1;
-  bool lst[4];
-  int kk[4];
-  bool mine = false;
-  for (int i = 0; i < 4; ++i) {
-    kk[i] = kbase + kq + 4 * i;
-    const int g = D.k0[d] + kk[i];
-    lst[i] = sa >= 0 && kk[i] < no && listed[int64_t(g) * nshell + sa];
-    mine |= lst[i];
-  }
-  double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  if (__syncthreads_or(mine)) {
-    for (int b0 = 0; b0 < n; b0 += kT) {
-      // stage L_J(a0.., b0..): packed rows are contiguous in the smaller index
-      if (a0 > b0) {
-        for (int e = tid; e < kT * kT; e += kLkThreads) {
-          const int r = e >> 6, cc = e & 63;
-          const int64_t aa = a0 + r, bb = b0 + cc;
-          tl[r][cc] = (aa < n) ? row[aa * (aa + 1) / 2 + bb] : 0.0;
-        }
-      } else if (a0 < b0) {
-        for (int e = tid; e < kT * kT; e += kLkThreads) {
-          const int r = e & 63, cc = e >> 6;
-          const int64_t aa = a0 + r, bb = b0 + cc;
-          tl[r][cc] = (bb < n) ? row[bb * (bb + 1) / 2 + aa] : 0.0;
-        }
-      } else {
-        for (int e = tid; e < kT * kT; e += kLkThreads) {
-          const int r = e >> 6, cc = e & 63;
-          if (cc > r) continue;
-          const int64_t aa = a0 + r, bb = b0 + cc;
-          const double v = (aa < n) ? row[aa * (aa + 1) / 2 + bb] : 0.0;
-          tl[r][cc] = v;
-          tl[cc][r] = v;
-        }
-      }
-      for (int e = tid; e < kT * kKc; e += kLkThreads) {
-        const int r = e / kKc, q = e % kKc;
-        const int64_t bb = b0 + r;
-        const int k = kbase + q;
-        tc[r][q] = (bb < n && k < no) ? c[k + int64_t(no) * bb] : 0.0;
-      }
-      if (tid < kT) tsb[tid] = (b0 + tid < n) ? shell[b0 + tid] : -1;
-      __syncthreads();
-      if (mine) {
-        int prev = -2;
-        bool m[4] = {false, false, false, false};
-        const int bend = min(kT, n - b0);
-        for (int cc = 0; cc < bend; ++cc) {
-          const int sb = tsb[cc];
-          if (sb != prev) {
-            prev = sb;
-            const int64_t p = shp_idx(sa, sb);
-            const bool pres = present[p] != 0;
-            const double svv = sv[p];
-            for (int i = 0; i < 4; ++i) {
-              const int g = D.k0[d] + kk[i];
-              m[i] = lst[i] && pres && sqrt(fabs(sumac[int64_t(g) * nshell + sb] * svv)) >= D.thrv[d];
-            }
-          }
-          const double l = tl[al][cc];
-          for (int i = 0; i < 4; ++i)
-            if (m[i]) acc[i] += l * tc[cc][kq + 4 * i];
-        }
-      }
-      __syncthreads();
-    }
-  }
-  if (a < n_pad)
-    for (int i = 0; i < 4; ++i)
-      if (kk[i] < no) X[(int64_t(D.k0[d] + kk[i]) * jnum + jr) * n_pad + a] = acc[i];
+__device__ inline v4d mfma64(double a, double b, v4d c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// K tile (A, B), A >= B, of the lower triangle: kacc[d](a,b) += sum over the
-// orbitals k of density d whose pair cuts keep (sa, sb) of sum_J X X.
-__global__ __launch_bounds__(kLkThreads) void k_lk_k(
-    LkDens D, const double *__restrict__ X, int jnum, int n, int n_pad, int nshell,
-    const int32_t *__restrict__ shell, const uint8_t *__restrict__ listed,
-    const uint8_t *__restrict__ keep, const double *__restrict__ mlk, const double *__restrict__ faa,
-    double maxred, double *__restrict__ kacc, int64_t ldk) {
-  __shared__ double xa[kLkBatch][kT];
-  __shared__ double xb[kLkBatch][kT];
-  // tile (ta, tb), ta >= tb, from the linear block index
-  const int64_t t = blockIdx.x;
-  int ta = int((sqrt(8.0 * double(t) + 1.0) - 1.0) * 0.5);
-  while (int64_t(ta) * (ta + 1) / 2 > t) --ta;
-  while (int64_t(ta + 1) * (ta + 2) / 2 <= t) ++ta;
-  const int tb = int(t - int64_t(ta) * (ta + 1) / 2);
-  const int tid = threadIdx.x, ti = tid & 15, tj = tid >> 4;
-  int ar[4], bc[4], sa[4], sb[4];
-  for (int i = 0; i < 4; ++i) {
-    ar[i] = ta * kT + ti * 4 + i;
-    bc[i] = tb * kT + tj * 4 + i;
-    sa[i] = ar[i] < n ? shell[ar[i]] : -1;
-    sb[i] = bc[i] < n ? shell[bc[i]] : -1;
+// Masked half-transform: X(bt, g, J, a) for one shell a, 64 orbitals (word q) and
+// kHtCols columns (J, a in the shell, a fastest).  One wave; per step of four b
+// it takes four A fragments (16 orbitals each, masked bit by bit) and three B
+// fragments (packed elements gathered, one column per lane).  The steps whose
+// mask words are all zero are left out.  X of orbitals that do not keep the
+// shell is not meaningful and never read through its mask.
+// grid = (shells a, column groups, batches * words).
+__global__ __launch_bounds__(64) void k_lk_ht(
+    LkDens D, const LkGroup G, const double *__restrict__ L, int64_t ldl, int n, int n_pad, int nshell,
+    const int32_t *__restrict__ shell, const int32_t *__restrict__ koff, const int32_t *__restrict__ nbsh,
+    const unsigned long long *__restrict__ mw, const unsigned long long *__restrict__ kw, double *__restrict__ X) {
+  __shared__ unsigned long long sw[kHtPanel];
+  __shared__ uint16_t steps[kHtPanel / 4];
+  const int sa = blockIdx.x, bt = blockIdx.z / D.nq, q = blockIdx.z % D.nq;
+  if (kw[(int64_t(bt) * D.nq + q) * nshell + sa] == 0) return;
+  const int na = nbsh[sa], nc = na * G.jnum[bt], col0 = blockIdx.y * kHtCols;
+  if (col0 >= nc) return;
+  const int lane = threadIdx.x, m = lane & 15, g = lane >> 4;
+  const int d = d_of_word(D, q), kb = 64 * (q - D.q0[d]), no = D.nocc[d];
+  const int nkt = min(4, (no - kb + 15) / 16), nct = min(3, (nc - col0 + 15) / 16);
+  const double *__restrict__ c = D.c[d];
+  const unsigned long long *__restrict__ row = mw + ((int64_t(bt) * D.nq + q) * nshell + sa) * nshell;
+  // this lane's columns: vector row pointer and AO
+  const double *__restrict__ lp[3];
+  int64_t xo[3];
+  int ca[3];
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const int col = min(col0 + 16 * j + m, nc - 1);
+    const int jl = col / na;
+    ca[j] = koff[sa] + (col - jl * na);
+    lp[j] = L + (G.j0[bt] + jl) * ldl;
+    xo[j] = int64_t(jl) * n_pad + ca[j];
   }
-  for (int d = 0; d < D.nd; ++d) {
-    double acc[4][4] = {};
-    const double tau = D.tau[d], tk = D.tau[d] / maxred;
-    for (int k = 0; k < D.nocc[d]; ++k) {
-      const int g = D.k0[d] + k;
-      const int64_t so = int64_t(g) * nshell;
-      bool m[4][4];
-      bool any = false;
-      for (int i = 0; i < 4; ++i)
-        for (int j = 0; j < 4; ++j) {
-          bool ok = sa[i] >= 0 && sb[j] >= 0 && ar[i] >= bc[j];
-          if (ok) {
-            const int s1 = sa[i], s2 = sb[j];
-            ok = listed[so + s1] && listed[so + s2] && keep[so + s1] && keep[so + s2] &&
-                 !(mlk[so + s1] * mlk[so + s2] < tau) &&
-                 sqrt(fabs(faa[so + s1] * faa[so + s2])) >= tk;
-          }
-          m[i][j] = ok;
-          any |= ok;
-        }
-      if (!__syncthreads_or(any)) continue;
-      const double *xg = X + int64_t(g) * jnum * n_pad;
-      for (int e = tid; e < jnum * kT; e += kLkThreads) {
-        const int j = e >> 6, cc = e & 63;
-        xa[j][cc] = (ta * kT + cc < n_pad) ? xg[int64_t(j) * n_pad + ta * kT + cc] : 0.0;
-        xb[j][cc] = (tb * kT + cc < n_pad) ? xg[int64_t(j) * n_pad + tb * kT + cc] : 0.0;
-      }
-      __syncthreads();
-      if (any) {
-        double s[4][4] = {};
-        for (int j = 0; j < jnum; ++j) {
-          double va[4], vb[4];
-          for (int i = 0; i < 4; ++i) {
-            va[i] = xa[j][ti * 4 + i];
-            vb[i] = xb[j][tj * 4 + i];
-          }
-          for (int i = 0; i < 4; ++i)
-            for (int q = 0; q < 4; ++q) s[i][q] += va[i] * vb[q];
-        }
-        for (int i = 0; i < 4; ++i)
-          for (int q = 0; q < 4; ++q)
-            if (m[i][q]) acc[i][q] += s[i][q];
-      }
-      __syncthreads();
+  int kc[4];  // this lane's orbitals, clamped (their mask bits are zero past nocc)
+#pragma unroll
+  for (int i = 0; i < 4; ++i) kc[i] = min(kb + 16 * i + m, no - 1);
+  v4d acc[4][3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
+  for (int p0 = 0; p0 < n; p0 += kHtPanel) {
+    const int pn = min(kHtPanel, n - p0);
+    __syncthreads();
+    for (int e = lane; e < kHtPanel; e += 64) sw[e] = e < pn ? row[shell[p0 + e]] : 0ull;
+    __syncthreads();
+    int nact = 0;
+    for (int t0 = 0; 4 * t0 < pn; t0 += 64) {
+      const int t = t0 + lane;
+      const bool on = 4 * t < pn && ((sw[4 * t] | sw[4 * t + 1]) | (sw[4 * t + 2] | sw[4 * t + 3])) != 0;
+      const unsigned long long b = __ballot(on);
+      if (on) steps[nact + __popcll(b & ((1ull << lane) - 1ull))] = uint16_t(t);
+      nact += __popcll(b);
     }
-    double *kd = kacc + int64_t(d) * ldk;
-    for (int i = 0; i < 4; ++i)
-      for (int q = 0; q < 4; ++q)
-        if (ar[i] < n && bc[q] < n && ar[i] >= bc[q])
-          kd[int64_t(ar[i]) * (ar[i] + 1) / 2 + bc[q]] += acc[i][q];
+    __syncthreads();
+    double ar[2][4], br[2][3];
+    unsigned long long wr[2];
+    auto load = [&](int i, int st) __attribute__((always_inline)) {
+      const int e = 4 * steps[i] + g, b = min(p0 + e, n - 1);
+      wr[st] = sw[e];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) ar[st][t] = c[kc[t] + int64_t(no) * b];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        const int hi = max(ca[j], b), lo = min(ca[j], b);
+        br[st][j] = lp[j][int64_t(hi) * (hi + 1) / 2 + lo];
+      }
+    };
+    auto mul = [&](int st) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        if (t >= nkt) break;
+        const double a = (wr[st] >> (16 * t + m)) & 1ull ? ar[st][t] : 0.0;
+        acc[t][0] = mfma64(a, br[st][0], acc[t][0]);
+        if (nct > 1) acc[t][1] = mfma64(a, br[st][1], acc[t][1]);
+        if (nct > 2) acc[t][2] = mfma64(a, br[st][2], acc[t][2]);
+      }
+    };
+    if (nact > 0) {
+      load(0, 0);
+      for (int i = 0; i < nact; i += 2) {
+        load(min(i + 1, nact - 1), 1);
+        mul(0);
+        if (i + 1 >= nact) break;
+        load(min(i + 2, nact - 1), 0);
+        mul(1);
+      }
+    }
   }
+  double *__restrict__ xg = X + (int64_t(bt) * D.ktot + D.k0[d]) * kLkBatch * n_pad;
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    if (col0 + 16 * j + m >= nc) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int k = kb + 16 * i + 4 * r + g;
+        if (k < no) xg[int64_t(k) * kLkBatch * n_pad + xo[j]] = acc[i][j][r];
+      }
+  }
+}
+
+// K of one batch on the 32 x 32 tile t of the lower triangle, density d: the sum
+// over the orbitals whose pair mask is set of S_k = sum_J X_k X_k^T, formed by
+// MFMA per orbital and added under the mask.  One wave; a step's operands are
+// reloaded with the next kept orbital's as soon as they are multiplied.  kpart[((bt nd + d) ntile
+// + t) 1024 + (2 it + jt) 256 + 64 r + lane].  grid = (tiles, nd, batches).
+__global__ __launch_bounds__(64) void k_lk_k(LkDens D, const LkGroup G, const double *__restrict__ X, int n,
+                                             int n_pad, int nshell, const int32_t *__restrict__ shell,
+                                             const unsigned long long *__restrict__ pw, double *__restrict__ kpart) {
+  constexpr int KS = (kLkBatch + 3) / 4;
+  const int t = blockIdx.x, d = blockIdx.y, bt = blockIdx.z, jnum = G.jnum[bt];
+  int ta = int((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
+  while (ta * (ta + 1) / 2 > t) --ta;
+  while ((ta + 1) * (ta + 2) / 2 <= t) ++ta;
+  const int tb = t - ta * (ta + 1) / 2;
+  const int lane = threadIdx.x, m = lane & 15, g = lane >> 4;
+  const int64_t nshp = int64_t(nshell) * (nshell + 1) / 2;
+  v4d acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
+  uint32_t pr[2][2][4];  // shell pair of each element, ~0: not in the lower triangle (at most 65535 shells)
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int a = 32 * ta + 16 * i + 4 * r + g, b = 32 * tb + 16 * j + m;
+        pr[i][j][r] = a < n && b <= a ? uint32_t(shp_idx(shell[a], shell[b])) : ~0u;
+      }
+  const bool upper = ta != tb;  // tile (0, 1) of a diagonal tile lies above the diagonal
+  uint32_t jo[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) jo[s] = uint32_t(min(4 * s + g, jnum - 1)) * uint32_t(n_pad) + uint32_t(m);
+  for (int q = D.q0[d]; q < D.q0[d + 1]; ++q) {
+    const unsigned long long *__restrict__ pq = pw + (int64_t(bt) * D.nq + q) * nshp;
+    unsigned long long mk[2][2][4], any = 0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          mk[i][j][r] = pr[i][j][r] != ~0u ? pq[pr[i][j][r]] : 0ull;
+          any |= mk[i][j][r];
+        }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) any |= __shfl_xor(any, o);
+    any = (uint64_t(__builtin_amdgcn_readfirstlane(int(any >> 32))) << 32) |
+          uint32_t(__builtin_amdgcn_readfirstlane(int(any)));
+    if (any == 0) continue;
+    const double *__restrict__ xq =
+        X + (int64_t(bt) * D.ktot + D.k0[d] + 64 * (q - D.q0[d])) * kLkBatch * int64_t(n_pad);
+    double ra[KS][2], rb[KS][2];
+    auto load = [&](const double *__restrict__ x, int s) __attribute__((always_inline)) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        ra[s][h] = x[jo[s] + 32 * ta + 16 * h];
+        rb[s][h] = x[jo[s] + 32 * tb + 16 * h];
+      }
+    };
+    int k = __builtin_ctzll(any);
+#pragma unroll
+    for (int s = 0; s < KS; ++s) load(xq + int64_t(k) * kLkBatch * n_pad, s);
+    for (;;) {
+      any &= any - 1;
+      const int kn = any ? __builtin_ctzll(any) : k;  // next kept orbital, or this one again
+      const double *__restrict__ xn = xq + int64_t(kn) * kLkBatch * n_pad;
+      v4d sm[2][2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) sm[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const bool in = 4 * s + g < jnum;
+        double a[2], b[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          a[h] = in ? ra[s][h] : 0.0;
+          b[h] = in ? rb[s][h] : 0.0;
+        }
+        sm[0][0] = mfma64(a[0], b[0], sm[0][0]);
+        if (upper) sm[0][1] = mfma64(a[0], b[1], sm[0][1]);
+        sm[1][0] = mfma64(a[1], b[0], sm[1][0]);
+        sm[1][1] = mfma64(a[1], b[1], sm[1][1]);
+        load(xn, s);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[i][j][r] += (mk[i][j][r] >> k) & 1ull ? sm[i][j][r] : 0.0;
+      if (any == 0) break;
+      k = kn;
+    }
+  }
+  double *__restrict__ out = kpart + ((int64_t(bt) * D.nd + d) * gridDim.x + t) * 1024 + lane;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) out[(2 * i + j) * 256 + 64 * r] = acc[i][j][r];
+}
+
+// klt(d) += the group's batches in order.  grid = (tiles, nd), block 256.
+__global__ __launch_bounds__(kLkThreads) void k_lk_reduce(const double *__restrict__ kpart, int nb, int nd, int n,
+                                                          double *__restrict__ klt, int64_t ldk) {
+  const int t = blockIdx.x, d = blockIdx.y;
+  int ta = int((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
+  while (ta * (ta + 1) / 2 > t) --ta;
+  while ((ta + 1) * (ta + 2) / 2 <= t) ++ta;
+  const int tb = t - ta * (ta + 1) / 2;
+  const double *__restrict__ src = kpart + (int64_t(d) * gridDim.x + t) * 1024;
+  const int64_t stride = int64_t(nd) * gridDim.x * 1024;
+  for (int e = threadIdx.x; e < 1024; e += kLkThreads) {
+    const int tile = e >> 8, r = (e >> 6) & 3, lane = e & 63;
+    const int a = 32 * ta + 16 * (tile >> 1) + 4 * r + (lane >> 4), b = 32 * tb + 16 * (tile & 1) + (lane & 15);
+    if (a >= n || b > a) continue;
+    const int64_t p = d * ldk + int64_t(a) * (a + 1) / 2 + b;
+    double s = klt[p];
+    int k = 0;
+    for (; k + 8 <= nb; k += 8) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = src[(k + u) * stride + e];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s += v[u];
+    }
+    for (; k < nb; ++k) s += src[k * stride + e];
+    klt[p] = s;
+  }
+}
+
+// Least double x >= 0 with sqrt(x) >= t (the rounded square root, as the device
+// evaluates it, is monotone): sqrt|x| >= t can then be tested without a root.
+double least_square(double t) {
+  if (!(t > 0.0)) return 0.0;
+  double x = t * t;
+  if (std::isinf(x)) x = std::numeric_limits<double>::max();
+  while (std::sqrt(x) >= t) {
+    const double y = std::nextafter(x, 0.0);
+    if (!(std::sqrt(y) >= t) || y == x) break;
+    x = y;
+  }
+  while (std::sqrt(x) < t && !std::isinf(x)) x = std::nextafter(x, std::numeric_limits<double>::infinity());
+  return x;
 }
 
 // Shell-pair occupancy of a reduced set (nnBstRSh > 0 of the reference).
@@ -519,106 +741,153 @@ int lk_exchange(Context *c, int32_t nd, const int32_t *nocc, const double *const
     if (runs[i].rs < 0 || runs[i - 1].rs < 0 || runs[i].rs <= runs[i - 1].rs)
       return set_error(c, MJK_ERR_STATE,
                        "LK screening: vectors must come reduced set by reduced set, in order");
+  const double maxred = double(K.maxred > 0 ? K.maxred : int(std::max<size_t>(c->rsets.size(), 1)));
   LkDens D{};
   D.nd = nd;
   int ktot = 0;
   for (int d = 0; d < nd; ++d) {
     D.nocc[d] = std::max(0, nocc[d]);
     D.k0[d] = ktot;
-    D.nkc[d] = int(ceil_div(D.nocc[d], kKc));
+    D.q0[d + 1] = D.q0[d] + int(ceil_div(D.nocc[d], 64));
     D.c[d] = corb[d];
     D.tau[d] = tau[d];
-    D.thrv[d] = thrv[d];
     D.xtau[d] = std::sqrt(tau[d]);  // xtau = sqrt(tau), cho_lk_casscf.F90:193-194
+    D.thrv2[d] = least_square(thrv[d]);
+    D.tk2[d] = least_square(tau[d] / maxred);
     ktot += D.nocc[d];
   }
   D.ktot = ktot;
+  D.nq = D.q0[nd];
   int rc;
   for (int d = 0; d < nd; ++d)
     if ((rc = fill_zero(c, klt + d * ldk, sizeof(double) * size_t(np)))) return rc;
   K.last_stats[0] = K.last_stats[1] = K.last_stats[2] = 0;
   K.last_batches = 0;
   if (ktot == 0 || runs.empty()) return MJK_OK;
-  const int64_t kt = std::max(ktot, 1);
-  const size_t flag_bytes = size_t(round_up(kt * ns, 4));  // fill_zero works in 4-byte words
-  if ((rc = ensure(c, K.diag, sizeof(double) * size_t(np))) ||
-      (rc = ensure(c, K.dh, sizeof(double) * size_t(n) * n)) ||
-      (rc = ensure(c, K.ylk, sizeof(double) * size_t(kt) * n)) ||
-      (rc = ensure(c, K.svshp, sizeof(double) * size_t(nshp))) ||
-      (rc = ensure(c, K.sumac, sizeof(double) * size_t(kt) * ns)) ||
-      (rc = ensure(c, K.mlk, sizeof(double) * size_t(kt) * ns)) ||
-      (rc = ensure(c, K.faa, sizeof(double) * size_t(kt) * ns)) ||
-      (rc = ensure(c, K.listed, flag_bytes)) || (rc = ensure(c, K.keep, flag_bytes)) ||
-      (rc = ensure(c, K.x, sizeof(double) * size_t(kt) * kLkBatch * n_pad)) ||
-      (rc = ensure(c, K.stats, 3 * sizeof(unsigned long long))))
-    return rc;
-  double *diag = static_cast<double *>(K.diag.ptr);
-  if ((rc = hip_check(c, hipMemcpyAsync(diag, K.diag0.ptr, sizeof(double) * size_t(np),
-                                        hipMemcpyDeviceToDevice, c->stream), "LK diagonal")) ||
-      (rc = fill_zero(c, K.stats.ptr, 3 * sizeof(unsigned long long))) ||
-      (rc = fill_zero(c, K.faa.ptr, sizeof(double) * size_t(kt) * ns)) ||
-      (rc = fill_zero(c, K.listed.ptr, flag_bytes)) ||
-      (rc = fill_zero(c, K.mlk.ptr, sizeof(double) * size_t(kt) * ns)))
-    return rc;
-  const int32_t *shell = static_cast<const int32_t *>(K.shell.ptr);
-  const int32_t *koff = static_cast<const int32_t *>(K.koff.ptr);
-  const int32_t *nbsh = static_cast<const int32_t *>(K.nbsh.ptr);
-  double *sv = static_cast<double *>(K.svshp.ptr), *sumac = static_cast<double *>(K.sumac.ptr);
-  double *mlk = static_cast<double *>(K.mlk.ptr), *faa = static_cast<double *>(K.faa.ptr);
-  uint8_t *listed = static_cast<uint8_t *>(K.listed.ptr), *keep = static_cast<uint8_t *>(K.keep.ptr);
-  double *X = static_cast<double *>(K.x.ptr);
-  auto *stats = static_cast<unsigned long long *>(K.stats.ptr);
-  const double maxred = double(K.maxred > 0 ? K.maxred : int(std::max<size_t>(c->rsets.size(), 1)));
-  hipLaunchKernelGGL(k_lk_sumac, dim3(unsigned(ktot)), dim3(kLkThreads), 0, c->stream, D, ns, koff,
-                     nbsh, sumac);
-  const unsigned gnp = unsigned(std::min<int64_t>(ceil_div(np, kLkThreads), 4096));
-  const int ntile = int(ceil_div(n, kT));
-  const unsigned nkt = unsigned(int64_t(ntile) * (ntile + 1) / 2);
-  // reduced sets JRED1..JRED2 of the vectors; the screening cadence counts
-  // every one of them, with or without vectors (:336-337,891-898)
-  const int jred1 = runs.front().rs, jred2 = runs.back().rs;
-  int kscreen = 1;
+  // the batches, and before which of them the shell lists are evaluated: the first
+  // one, and every nScreen reduced sets, counting each of JRED1..JRED2 with or
+  // without vectors (:336-337,374,831,891-898)
+  struct Batch { int64_t j0; int jnum; const uint8_t *present; bool screen; };
+  std::vector<Batch> batches;
+  int kscreen = 1, max_rows = 0;
   bool doscreen = true;
   size_t ri = 0;
-  for (int jred = jred1; jred <= jred2; ++jred) {
+  for (int jred = runs.front().rs; jred <= runs.back().rs; ++jred) {
     if (ri < runs.size() && runs[ri].rs == jred) {
       const Run &R = runs[ri++];
       const uint8_t *present = nullptr;
       if ((rc = lk_present(c, R.rs, &present))) return rc;
-      const int64_t nvec = std::min<int64_t>(kLkBatch, R.jn);  // :374
+      const int64_t nvec = std::min<int64_t>(kLkBatch, R.jn);
       for (int64_t b = 0; b < R.jn; b += nvec) {
-        const int64_t j0 = R.j0 + b;
-        const int jnum = int(std::min<int64_t>(nvec, R.jn - b));
-        if (K.estimate)
-          hipLaunchKernelGGL(k_lk_est_diag, dim3(gnp), dim3(kLkThreads), 0, c->stream, c->L, c->ldl,
-                             j0, jnum, np, diag);
-        hipLaunchKernelGGL(k_lk_svshp, dim3(unsigned(ceil_div(nshp, kLkThreads / 64))),
-                           dim3(kLkThreads), 0, c->stream, c->L, c->ldl, j0, jnum, ns, koff, nbsh, sv);
-        if (doscreen)
-          hipLaunchKernelGGL(k_lk_diah, dim3(unsigned(n)), dim3(kLkThreads), 0, c->stream, diag, n,
-                             static_cast<double *>(K.dh.ptr));
-        hipLaunchKernelGGL(k_lk_lists, dim3(unsigned(ktot)), dim3(kLkThreads), 0, c->stream, D, n, ns,
-                           int(doscreen), int(cas_cut), koff, nbsh,
-                           static_cast<const double *>(K.dh.ptr), static_cast<double *>(K.ylk.ptr),
-                           mlk, listed, sumac, sv, present, keep, stats);
-        hipLaunchKernelGGL(k_lk_ht, dim3(unsigned(ntile), unsigned(jnum), unsigned(D.nkc[0] + D.nkc[1])),
-                           dim3(kLkThreads), 0, c->stream, D, c->L, c->ldl, j0, jnum, n, n_pad, ns,
-                           shell, sumac, sv, present, listed, X);
-        hipLaunchKernelGGL(k_lk_faa, dim3(unsigned(ktot)), dim3(kLkThreads), 0, c->stream, D, n_pad,
-                           jnum, ns, koff, nbsh, X, listed, keep, mlk, faa, maxred, stats);
-        hipLaunchKernelGGL(k_lk_k, dim3(nkt), dim3(kLkThreads), 0, c->stream, D, X, jnum, n, n_pad, ns,
-                           shell, listed, keep, mlk, faa, maxred, klt, ldk);
-        if (K.update && c->lk_nscreen > 0)
-          hipLaunchKernelGGL(k_lk_update_diag, dim3(gnp), dim3(kLkThreads), 0, c->stream, c->L,
-                             c->ldl, j0, jnum, np, diag);
-        if ((rc = hip_check(c, hipGetLastError(), "LK batch launch"))) return rc;
-        doscreen = false;  // :831
-        ++K.last_batches;
+        batches.push_back({R.j0 + b, int(std::min<int64_t>(nvec, R.jn - b)), present, doscreen});
+        max_rows = std::max(max_rows, batches.back().jnum);
+        doscreen = false;
       }
     }
-    doscreen = kscreen == c->lk_nscreen;  // :891-898
+    doscreen = kscreen == c->lk_nscreen;
     if (!doscreen) ++kscreen;
     else kscreen = 1;
+  }
+  K.last_batches = int64_t(batches.size());
+  // Batches that go through the kernels together: as many as 1 GiB of per-batch
+  // buffers holds (X, masks, partial K), up to kLkGroup.
+  const int nt = int(ceil_div(n, 32)), ntile = nt * (nt + 1) / 2;
+  const int64_t ld = 64 * int64_t(D.nq);
+  const size_t bx = sizeof(double) * size_t(ktot) * kLkBatch * n_pad, bm = 8 * size_t(D.nq) * ns * ns,
+               bp = 8 * size_t(D.nq) * nshp, bk = sizeof(double) * 1024 * size_t(nd) * ntile,
+               bs = sizeof(double) * size_t(nshp), bf = sizeof(double) * size_t(ns) * ld,
+               bw = 8 * size_t(D.nq) * ns;
+  const int ng = int(std::max<size_t>(
+      1, std::min<size_t>({size_t(kLkGroup), batches.size(), (size_t(1) << 30) / (bx + bm + bp + bk + bs + bf + bw)})));
+  if (int64_t(ng) * D.nq > 65535 || ns > 65535)
+    return set_error(c, MJK_ERR_ARG, "LK screening: more shells or orbitals than the launch grid holds");
+  const size_t flag_bytes = size_t(ld) * ns;
+  if ((rc = ensure(c, K.diag, sizeof(double) * size_t(np))) ||
+      (rc = ensure(c, K.dh, sizeof(double) * size_t(n) * n)) ||
+      (rc = ensure(c, K.ylk, sizeof(double) * size_t(ktot) * n)) ||
+      (rc = ensure(c, K.svshp, bs * ng)) || (rc = ensure(c, K.sumac, sizeof(double) * size_t(ld) * ns)) ||
+      (rc = ensure(c, K.mlk, sizeof(double) * size_t(ld) * ns)) || (rc = ensure(c, K.faa, bf * ng)) ||
+      (rc = ensure(c, K.listed, flag_bytes)) || (rc = ensure(c, K.keep, bw * ng)) ||
+      (rc = ensure(c, K.mask, bm * ng)) || (rc = ensure(c, K.pairs, bp * ng)) ||
+      (rc = ensure(c, K.kacc, bk * ng)) || (rc = ensure(c, K.x, bx * ng)) ||
+      (rc = ensure(c, K.stats, 3 * sizeof(unsigned long long))))
+    return rc;
+  double *diag = static_cast<double *>(K.diag.ptr);
+  double *sv = static_cast<double *>(K.svshp.ptr), *sumac = static_cast<double *>(K.sumac.ptr);
+  double *mlk = static_cast<double *>(K.mlk.ptr), *faa = static_cast<double *>(K.faa.ptr);
+  double *X = static_cast<double *>(K.x.ptr), *kpart = static_cast<double *>(K.kacc.ptr);
+  uint8_t *listed = static_cast<uint8_t *>(K.listed.ptr);
+  typedef unsigned long long word;
+  word *keep = static_cast<word *>(K.keep.ptr), *mask = static_cast<word *>(K.mask.ptr);
+  word *pairs = static_cast<word *>(K.pairs.ptr), *stats = static_cast<word *>(K.stats.ptr);
+  // mlk, sumac and listed have entries past each density's orbitals: zero, and no
+  // mask bit is set for them
+  if ((rc = hip_check(c, hipMemcpyAsync(diag, K.diag0.ptr, sizeof(double) * size_t(np),
+                                        hipMemcpyDeviceToDevice, c->stream), "LK diagonal")) ||
+      (rc = fill_zero(c, stats, 3 * sizeof(word))) || (rc = fill_zero(c, listed, flag_bytes)) ||
+      (rc = fill_zero(c, mlk, sizeof(double) * size_t(ld) * ns)) ||
+      (rc = fill_zero(c, sumac, sizeof(double) * size_t(ld) * ns)) || (rc = fill_zero(c, faa, bf * ng)))
+    return rc;
+  const int32_t *shell = static_cast<const int32_t *>(K.shell.ptr);
+  const int32_t *koff = static_cast<const int32_t *>(K.koff.ptr);
+  const int32_t *nbsh = static_cast<const int32_t *>(K.nbsh.ptr);
+  hipLaunchKernelGGL(k_lk_sumac, dim3(unsigned(ktot)), dim3(kLkThreads), 0, c->stream, D, ns, koff,
+                     nbsh, sumac);
+  const unsigned gnp = unsigned(std::min<int64_t>(ceil_div(np, kLkThreads), 4096));
+  int max_shell = 1;
+  for (int32_t v : K.nbassh) max_shell = std::max(max_shell, int(v));
+  const unsigned cols = unsigned(ceil_div(int64_t(max_rows) * max_shell, kHtCols));
+  const bool update = K.update && c->lk_nscreen > 0;
+  for (size_t b0 = 0; b0 < batches.size();) {
+    LkGroup G{};
+    size_t b1 = b0;
+    int64_t jn = 0;
+    for (; b1 < batches.size() && int(b1 - b0) < ng && (b1 == b0 || !batches[b1].screen); ++b1) {
+      G.j0[b1 - b0] = batches[b1].j0;
+      G.jnum[b1 - b0] = batches[b1].jnum;
+      G.present[b1 - b0] = batches[b1].present;
+      jn += batches[b1].jnum;
+    }
+    G.nb = int(b1 - b0);
+    const unsigned nb = unsigned(G.nb), nbq = unsigned(G.nb * D.nq);
+    if (max_shell <= kSmallShell)
+      hipLaunchKernelGGL(k_lk_svshp, dim3(unsigned(ns), unsigned(ceil_div(ns, kLkThreads)), nb), dim3(kLkThreads), 0,
+                         c->stream, c->L, c->ldl, G, ns, koff, nbsh, sv);
+    else
+      hipLaunchKernelGGL(k_lk_svshp_wave, dim3(unsigned(ceil_div(nshp, kLkThreads / 64)), nb), dim3(kLkThreads), 0,
+                         c->stream, c->L, c->ldl, G, ns, koff, nbsh, sv);
+    if (batches[b0].screen) {
+      // Estimate: the diagonal of the batch the lists are evaluated before
+      if (K.estimate)
+        hipLaunchKernelGGL(k_lk_est_diag, dim3(gnp), dim3(kLkThreads), 0, c->stream, c->L, c->ldl,
+                           G.j0[0], G.jnum[0], np, diag);
+      hipLaunchKernelGGL(k_lk_diah, dim3(unsigned(n)), dim3(kLkThreads), 0, c->stream, diag, n,
+                         static_cast<double *>(K.dh.ptr));
+      hipLaunchKernelGGL(k_lk_screen, dim3(unsigned(ktot)), dim3(kLkThreads), 0, c->stream, D, n, ns,
+                         int(cas_cut), koff, nbsh, static_cast<const double *>(K.dh.ptr),
+                         static_cast<double *>(K.ylk.ptr), mlk, listed, stats);
+    }
+    hipLaunchKernelGGL(k_lk_mask, dim3(unsigned(ns), nbq), dim3(kLkThreads), 0, c->stream, D, G, ns, nbsh, listed,
+                       sumac, sv, mask, keep, stats);
+    hipLaunchKernelGGL(k_lk_ht, dim3(unsigned(ns), cols, nbq), dim3(64), 0, c->stream, D, G, c->L, c->ldl, n, n_pad,
+                       ns, shell, koff, nbsh, mask, keep, X);
+    hipLaunchKernelGGL(k_lk_faa, dim3(unsigned(ktot), nb), dim3(kLkThreads), 0, c->stream, D, G, n_pad, ns, koff,
+                       nbsh, X, keep, faa);
+    hipLaunchKernelGGL(k_lk_pairs, dim3(unsigned(ns), nbq), dim3(kLkThreads), 0, c->stream, D, ns, keep, mlk, faa,
+                       pairs, stats);
+    hipLaunchKernelGGL(k_lk_k, dim3(unsigned(ntile), unsigned(nd), nb), dim3(64), 0, c->stream, D, G, X, n, n_pad,
+                       ns, shell, pairs, kpart);
+    hipLaunchKernelGGL(k_lk_reduce, dim3(unsigned(ntile), unsigned(nd)), dim3(kLkThreads), 0, c->stream, kpart,
+                       G.nb, nd, n, klt, ldk);
+    // Update: only a later evaluation of the lists reads the diagonal, and with
+    // Estimate it is formed anew there
+    bool later = false;
+    for (size_t b = b1; b < batches.size(); ++b) later |= batches[b].screen;
+    if (update && later && !K.estimate)
+      hipLaunchKernelGGL(k_lk_update_diag, dim3(gnp), dim3(kLkThreads), 0, c->stream, c->L, c->ldl, G.j0[0],
+                         int(jn), np, diag);
+    if ((rc = hip_check(c, hipGetLastError(), "LK group launch"))) return rc;
+    b0 = b1;
   }
   unsigned long long h[3];
   if ((rc = hip_check(c, hipMemcpyAsync(h, stats, sizeof(h), hipMemcpyDeviceToHost, c->stream),

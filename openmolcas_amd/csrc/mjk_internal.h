@@ -94,12 +94,12 @@ struct LKState {
   DevBuf present_all;                     // every shell pair (vectors written in place)
   int64_t present_all_version = -1;
   // per call
-  DevBuf diag, dh, ylk, svshp, sumac, mlk, listed, keep, faa, x, kacc, stats;
+  DevBuf diag, dh, ylk, svshp, sumac, mlk, listed, keep, mask, pairs, faa, x, kacc, stats;
   long long last_stats[3] = {0, 0, 0};    // listed shells, half-transformed shell pairs, K blocks
   int64_t last_batches = 0;
   ~LKState() {
     for (DevBuf *b : {&shell, &koff, &nbsh, &diag0, &present_all, &diag, &dh, &ylk, &svshp, &sumac,
-                      &mlk, &listed, &keep, &faa, &x, &kacc, &stats})
+                      &mlk, &listed, &keep, &mask, &pairs, &faa, &x, &kacc, &stats})
       if (b->ptr) (void)hipFree(b->ptr);
     for (DevBuf &b : present)
       if (b.ptr) (void)hipFree(b.ptr);
