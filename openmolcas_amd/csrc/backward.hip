@@ -265,8 +265,7 @@ int gemm(Context *c, const GemmBatch &g0, int batch) {
   GemmBatch g = g0;
   // operands are addressed with 32-bit byte offsets inside one product
   constexpr int64_t kMaxElems = int64_t(1) << 28;
-  if (int64_t(g.m) * g.lda >= kMaxElems || int64_t(g.k) * g.ldb >= kMaxElems ||
-      int64_t(g.n) * g.ldb >= kMaxElems)
+  if (int64_t(g.m) * g.lda >= kMaxElems || int64_t(BT ? g.n : g.k) * g.ldb >= kMaxElems)
     return set_error(c, MJK_ERR_ARG, "gemm: operand of more than 2^28 elements");
   const int ti = (g.m + kTM - 1) / kTM, tj = (g.n + kTM - 1) / kTM;
   g.tiles = EPI == 1 ? ti * (ti + 1) / 2 : ti * tj;  // EPI == 1: square lower-triangle output
@@ -800,6 +799,25 @@ int zsym(Context *c, const TX *X, int64_t sx, const double *cb, int ldc, int noc
 }
 
 }  // namespace
+
+// O[i][j] = sum_k A[i][k] B[j][k], one launch per block of rows of A and of B
+// that the 32-bit offsets of the kernel reach.
+int gemm_nt(Context *c, const double *A, int64_t lda, const double *B, int64_t ldb, double *O, int64_t ldo,
+            int64_t m, int n, int k) {
+  constexpr int64_t kMost = (int64_t(1) << 28) - 1;
+  const int64_t mi = std::max<int64_t>(1, kMost / lda), mj = std::max<int64_t>(1, kMost / ldb);
+  for (int64_t i = 0; i < m; i += mi)
+    for (int64_t j = 0; j < n; j += mj) {
+      GemmBatch g{};
+      g.A = A + i * lda; g.lda = lda;
+      g.B = B + j * ldb; g.ldb = ldb;
+      g.O = O + i * ldo + j; g.ldo = ldo;
+      g.m = int(std::min(mi, m - i)); g.n = int(std::min<int64_t>(mj, n - j)); g.k = k; g.alpha = 1.0;
+      const int rc = gemm<true, 0>(c, g, 1);
+      if (rc) return rc;
+    }
+  return hip_check(c, hipGetLastError(), "gemm launch");
+}
 
 int z_from_x(Context *c, const void *X, bool x_f32, int ldc, int nocc, int64_t jn, double *z) {
   const double *cb = static_cast<const double *>(c->w->cbank.ptr);

@@ -20,6 +20,9 @@
 //   - the K kernel forms S_k = sum_J X_k X_k^T of one orbital on a 32 x 32 tile
 //     by MFMA and adds it under the mask of (orbital, shell a, shell b),
 //     skipping orbitals whose mask is empty on the tile;
+//   - decision quantities (diagonal, SvShp, SumAClk, Y, Faa) are evaluated
+//     without FMA contraction, in the reference's summation order where it
+//     has one, so the cuts fall where the reference's fall.
 // Measured on a chain of 48 atoms (n=240, nchol=1200 in 48 batches, 48 orbitals),
 // whole call: 33.2 -> 0.96 ms.  One batch at a time, each kernel had 10-144
 // workgroups of serial work (K 0.35 ms per batch, half-transform 0.14, lists
@@ -27,9 +30,6 @@
 // one cache line per lane), 0.13 (masks, bound by their scalar loads), 0.11
 // (reads L once), K-block masks 0.09.  The MFMA sums run in the order of the
 // scalar loops they replace: the result is bit for bit the same.
-//   - decision quantities (diagonal, SvShp, SumAClk, Y, Faa) are evaluated
-//     without FMA contraction, in the reference's summation order where it
-//     has one, so the cuts fall where the reference's fall.
 // The selection sort of the reference (:602-627) keeps the shells whose MLk
 // passes the cut, in decreasing MLk order, stopping at the first failure;
 // because the values along the sorted list do not increase and rounding is
@@ -534,7 +534,7 @@ __global__ __launch_bounds__(64) void k_lk_k(LkDens D, const LkGroup G, const do
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
-  uint32_t pr[2][2][4];  // shell pair of each element, ~0: not in the lower triangle (at most 65535 shells)
+  uint32_t pr[2][2][4];  // shell pair of each element, ~0: not in the lower triangle
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -797,10 +797,9 @@ int lk_exchange(Context *c, int32_t nd, const int32_t *nocc, const double *const
                bp = 8 * size_t(D.nq) * nshp, bk = sizeof(double) * 1024 * size_t(nd) * ntile,
                bs = sizeof(double) * size_t(nshp), bf = sizeof(double) * size_t(ns) * ld,
                bw = 8 * size_t(D.nq) * ns;
-  const int ng = int(std::max<size_t>(
-      1, std::min<size_t>({size_t(kLkGroup), batches.size(), (size_t(1) << 30) / (bx + bm + bp + bk + bs + bf + bw)})));
-  if (int64_t(ng) * D.nq > 65535 || ns > 65535)
-    return set_error(c, MJK_ERR_ARG, "LK screening: more shells or orbitals than the launch grid holds");
+  const int ng = int(std::max<size_t>(  // (batch, word) is one grid dimension
+      1, std::min<size_t>({size_t(kLkGroup), batches.size(), (size_t(1) << 30) / (bx + bm + bp + bk + bs + bf + bw),
+                           size_t(65535 / D.nq)})));
   const size_t flag_bytes = size_t(ld) * ns;
   if ((rc = ensure(c, K.diag, sizeof(double) * size_t(np))) ||
       (rc = ensure(c, K.dh, sizeof(double) * size_t(n) * n)) ||

@@ -220,6 +220,10 @@ void ht_launch(Context *c, int ot, const double *cb, int64_t j0, int64_t jn, dou
 // FP64 bank (cbank).  Writes z + J * nocc * nocc, nocc x nocc row-major.
 int z_from_x(Context *c, const void *X, bool x_f32, int ldc, int nocc, int64_t jn, double *z);
 
+// O[i][j] = sum_k A[i][k] B[j][k], FP64 (i < m, j < n; rows of lda, ldb, ldo).
+int gemm_nt(Context *c, const double *A, int64_t lda, const double *B, int64_t ldb, double *O, int64_t ldo,
+            int64_t m, int n, int k);
+
 // Exchange with tile screening (thresholds 0 = off): a K tile of a vector
 // slice is skipped when sum_J ||X^J_A||_F ||X^J_B||_F < tau, a half-transform
 // tile when ||L^J[:, tile]||_F max_d ||C_d||_F < thr_x.
