@@ -292,31 +292,31 @@ int grad_from_w(Context *c, int nocc, const double *W, int ldc, const double *v,
 // beta (C Z^J C^T)_ab) for the vectors J whose Z^J (nocc x nocc) has element
 // (k, l) at z + J sz + k ldz + l.
 struct GradRows {
-  const double *cb;  // orbital bank C[a][k]: n_pad rows of ldc, columns >= nocc zero
-  const float *cb32; // the same bank in FP32 (FP32 products only)
-  int ldc;
+  const void *ct;    // transposed orbital bank C^T[k][a], FP64 or FP32: 16 OC16 rows of n_pad,
+                     // zero for k >= nocc or a >= n
+  int n_pad;
   const double *z;
   int64_t sz;
   int ldz;
   int o;             // nocc
   const double *v;   // V[J]
-  const double *p;   // P, plain LT
+  const double *p;   // P, plain LT (null: 2 C C^T)
   double gv, beta;
   double *g;
   int64_t ldg;
   int32_t rowbytes;  // bytes of one packed triangle n (n + 1) / 2 (< 2^31)
-  int n, T;          // basis functions, row tiles of 64
-  int64_t items;     // T * vectors
+  int n, T;          // basis functions, strips of 32 rows
+  int64_t jn;        // vectors
+  int64_t items;     // strips x groups of four vectors
 };
-// Element index of a masked element in the packed triangle: byte offset
-// 2^31, past every row, so the buffer load returns 0 and the store is dropped
-// by the range check of the buffer resource (stride 0, rowbytes records).
-constexpr uint32_t kMasked = 0x10000000u;
+// Byte offset of a masked element in the packed triangle: past every row, so
+// the buffer load returns 0 and the store is dropped by the range check of the
+// buffer resource (stride 0, rowbytes records).
+constexpr uint32_t kMasked = 0x80000000u;
 constexpr int kRsrcWord3 = 0x00020000;  // buffer resource word 3 of this architecture family
-typedef int v2u __attribute__((ext_vector_type(2)));  // operand type of the 64-bit buffer builtins
-
-typedef double f4d __attribute__((ext_vector_type(4)));
-typedef float f4f __attribute__((ext_vector_type(4)));
+typedef int v2u __attribute__((ext_vector_type(2)));  // operand types of the buffer builtins
+typedef int v4u __attribute__((ext_vector_type(4)));
+typedef float v2f __attribute__((ext_vector_type(2)));
 
 // Arithmetic of k_grad_rows: FP64 MFMA, or FP32 MFMA (the split-precision
 // backward's tail vectors: contractions of at most 128 terms, FP64 output).
@@ -325,255 +325,263 @@ typedef float f4f __attribute__((ext_vector_type(4)));
 // 4(l/16) + r (FP32), column l%16.
 struct GR64 {
   typedef double T;
+  typedef v2d T2;
   typedef v4d Acc;
-  typedef f4d T4;
   __device__ static Acc mma(T a, T b, Acc c) { return mfma64(a, b, c); }
-  __device__ static int row(int lane, int r) { return 4 * r + (lane >> 4); }
-  __device__ static const T *bank(const GradRows &g) { return g.cb; }
+  static constexpr int kStep = 4;  // row(g, r) - row(g, r - 1)
+  __device__ static int row(int g, int r) { return 4 * r + g; }
 };
 struct GR32 {
   typedef float T;
+  typedef v2f T2;
   typedef v4f Acc;
-  typedef f4f T4;
   __device__ static Acc mma(T a, T b, Acc c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-  __device__ static int row(int lane, int r) { return 4 * (lane >> 4) + r; }
-  __device__ static const T *bank(const GradRows &g) { return g.cb32; }
+  static constexpr int kStep = 1;
+  __device__ static int row(int g, int r) { return 4 * g + r; }
 };
 
-// Work item (vector J, row tile I of 64 AOs).  Phase 1 forms W_I = C_I Z^J (64
-// x OC, OC = 16 OC16 >= nocc) with FP64 MFMA, both operands staged through LDS
-// in 16-column chunks, double-buffered; W_I goes to LDS.  Phase 2 walks the
-// column tiles j = 0..I: wave (wm, wn) forms its 32 x 32 quarter of W_I C_j^T
-// with the A operand from LDS and the C_j fragments read straight from the
-// bank, which every work item of the system reads and which stays in L2.  In a
-// 16-column chunk lane group g takes the contraction indices 4g..4g+3 in the
-// four MFMA steps (the A reads use the same order), so each fragment is one
-// 32-byte load; the fragments of the chunk after next are in flight while a
-// chunk is multiplied, and phase 2 needs no barrier.  Each finished block is
-// written packed with the V P term, all P values loaded before the first
-// store.  Within a vector the longest row tile runs first; consecutive items
-// run on one XCD.  W never goes through HBM (the two-GEMM form writes n x ldc
-// doubles per vector and reads them back once per column tile).
-template <int OC16, class R>
-__global__ __launch_bounds__(kThreads) void k_grad_rows(GradRows g) {
+// Work item = (four vectors J, one per wave; strip of 32 rows a).  Phase 1 forms
+// W^T = Z^T C^T of the strip (OC x 32, OC = 16 OC16 >= nocc): the transposed
+// product, because its result layout (column a on the lane, row l in the
+// register) is the A operand layout of phase 2, so W never leaves the
+// accumulators.  Phase 2 walks the column tiles of 32 up to the diagonal: A = W
+// from those registers, B = the tile's 32 columns of C^T, which the four waves
+// share in LDS (double-buffered, one barrier per tile).  Loads and stores retire
+// in one order, so a fragment loaded after a tile's stores is not there before
+// their acknowledgement: the next tile's columns are loaded to registers before
+// this tile's stores and no wait stands behind a store.  Lane l = 16 g + m takes
+// columns 2 m, 2 m + 1 at once (row and column tile (i, h): AO 32 t + 2 m + h).  The
+// tile is stored packed, two neighbours as 16 bytes, through a range-checked
+// buffer resource that drops elements past n; only the diagonal tile masks
+// element by element.  Contraction steps past nocc are left out.  The longest
+// strip of a group of vectors runs first; its strips run on one XCD (they share
+// the Z^J).
+// Bound by the matrix cores from about 90 orbitals (n=536 nchol=2510 nocc=98
+// 2.62 -> 1.98 ms, 56 TFLOP/s executed; n=600 nchol=2800 nocc=120 4.17 -> 3.11 ms),
+// below that and in FP32 by the scattered stores (2.0-2.6 TB/s of output; n=600
+// nchol=3000 nocc=75 2.83 -> 2.13 ms FP64, 2.07 -> 1.68 ms FP32; without them 0.4 ms
+// less; aligned or non-temporal stores do not help).  Before, one workgroup per
+// (J, 64 rows) kept W in LDS and read C AO-major: one L1 request per lane (74% of
+// the L1's cycles), and padding to 64 rows and 16 contraction indices.
+// HP: the density P is given.  Otherwise P = 2 C C^T, and gv V_J P + beta C Z C^T
+// = C (beta Z + 2 gv V_J 1) C^T takes the first term into phase 1 (FP64 only: the
+// V P term of an FP32 product stays in FP64, from P).
+template <int OC16, class R, bool HP>
+__global__ __launch_bounds__(kThreads, 2) void k_grad_rows(GradRows g) {
   typedef typename R::T T;
+  typedef typename R::T2 T2;
   typedef typename R::Acc Acc;
   constexpr int OC = 16 * OC16;
-  constexpr bool F32 = sizeof(T) == 4;
-  constexpr int WS = OC + 1;                                   // row stride of the phase-1 Z chunks
-  // Row stride of W_I.  FP32: a lane's four A values of a chunk are one
-  // 16-byte read; OC + 4 keeps rows 16-byte aligned and puts the 8 lanes of
-  // a read pass (rows r..r+7, 32 banks of 4 bytes) on 8 distinct 16-byte
-  // bank groups.  FP64 reads them one 8-byte value at a time (odd stride).
-  constexpr int WW = F32 ? OC + 4 : OC + 1;
-  constexpr int S1 = 2 * (kTM * (kBK + 1) + kBK * WS);         // phase-1 staging
-  constexpr int SW = kTM * WW;
-  __shared__ __attribute__((aligned(16))) T smem[S1 > SW ? S1 : SW];
-  typedef T RowA[kTM][kBK + 1];
-  typedef T RowB[kBK][WS];
-  RowA *sA = reinterpret_cast<RowA *>(smem);                   // [2]
-  RowB *sB = reinterpret_cast<RowB *>(smem + 2 * kTM * (kBK + 1));  // [2]
-  T(*sW)[WW] = reinterpret_cast<T(*)[WW]>(smem);               // aliases the staging
-
+  constexpr int V = 16 / int(sizeof(T));                 // elements of a 16-byte piece
+  constexpr int NP = OC * 32 / V;                        // pieces of a column tile
+  constexpr int PN = (NP + kThreads - 1) / kThreads;     // and per thread (the last one not for all)
+  typedef T VT __attribute__((ext_vector_type(V)));
+  __shared__ __attribute__((aligned(16))) T sB[2][OC * 32];
   const int64_t nblk = gridDim.x;  // multiple of 8
-  const int64_t l = (int64_t(blockIdx.x) & 7) * (nblk >> 3) + (int64_t(blockIdx.x) >> 3);
-  if (l >= g.items) return;
-  const int64_t J = l / g.T;
-  const int I = g.T - 1 - int(l - J * g.T);
-  const int i0 = I * kTM;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, gq = lane >> 4;
-  const T *__restrict__ cb = R::bank(g);
-  const int ldc = g.ldc, o = g.o;
+  const int64_t item = (int64_t(blockIdx.x) & 7) * (nblk >> 3) + (int64_t(blockIdx.x) >> 3);
+  if (item >= g.items) return;
+  const int64_t jr = item / g.T;
+  const int I = g.T - 1 - int(item - jr * g.T);
+  const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, gq = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int o = g.o, ldz = g.ldz, ldt = g.n_pad;
+  const T *__restrict__ ct = static_cast<const T *>(g.ct);
+  // a vector past the last repeats it, its stores dropped (a resource of no records)
+  const int64_t J = min(4 * jr + w, g.jn - 1);
   const double *__restrict__ zj = g.z + J * g.sz;
-  const int ldz = g.ldz;
+  const double vj = g.gv * g.v[J];
+  const __amdgpu_buffer_rsrc_t rg =
+      __builtin_amdgcn_make_buffer_rsrc(g.g + J * g.ldg, 0, 4 * jr + w < g.jn ? g.rowbytes : 0, kRsrcWord3);
+  const __amdgpu_buffer_rsrc_t rp =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(g.p), 0, g.rowbytes, kRsrcWord3);
 
-  // ---- phase 1: W_I = C_I Z^J; wave w owns rows 16w..16w+15, all OC columns
-  Acc acc1[OC16];
+  // column tile j of C^T: global -> registers -> LDS rows of 32
+  VT rs[PN];
+  auto fetch = [&](int j) __attribute__((always_inline)) {
 #pragma unroll
-  for (int t = 0; t < OC16; ++t) acc1[t] = Acc{0, 0, 0, 0};
-  T ra[4], rb[OC16];
-  uint32_t zok = 0;  // bit it: Z element it lies inside nocc x nocc (zeroed at stash time)
-  auto fetch1 = [&](int k0) {
-#pragma unroll
-    for (int it = 0; it < 4; ++it) {
-      const int e = tid + kThreads * it, r = e / kBK, kk = e % kBK;
-      ra[it] = cb[uint32_t(i0 + r) * uint32_t(ldc) + uint32_t(k0 + kk)];
-    }
-    zok = 0;
-#pragma unroll
-    for (int it = 0; it < OC16; ++it) {
-      const int e = tid + kThreads * it, kr = e / OC, cc = e % OC, k = k0 + kr;
-      const bool ok = k < o && cc < o;
-      rb[it] = T(zj[ok ? uint32_t(k) * uint32_t(ldz) + uint32_t(cc) : 0u]);
-      zok |= ok ? 1u << it : 0u;
+    for (int i = 0; i < PN; ++i) {
+      const int e = min(tid + kThreads * i, NP - 1);
+      rs[i] = *reinterpret_cast<const VT *>(ct + uint32_t(e / (32 / V)) * uint32_t(ldt) + uint32_t(32 * j + V * (e % (32 / V))));
     }
   };
-  auto stash1 = [&](int buf) {
+  auto stash = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int it = 0; it < 4; ++it) {
-      const int e = tid + kThreads * it;
-      sA[buf][e / kBK][e % kBK] = ra[it];
-    }
-#pragma unroll
-    for (int it = 0; it < OC16; ++it) {
-      const int e = tid + kThreads * it;
-      sB[buf][e / OC][e % OC] = ((zok >> it) & 1u) ? rb[it] : T(0);
-    }
+    for (int i = 0; i < PN; ++i)
+      if (kThreads * (i + 1) <= NP || tid + kThreads * i < NP)
+        *reinterpret_cast<VT *>(&sB[buf][V * (tid + kThreads * i)]) = rs[i];
   };
-  fetch1(0);
-  stash1(0);
-  if (OC16 > 1) fetch1(kBK);
-  __syncthreads();
-#pragma unroll 1
-  for (int c = 0; c < OC16; ++c) {
-    const int cur = c & 1;
-#pragma unroll
-    for (int ks = 0; ks < kBK / 4; ++ks) {
-      const T a = sA[cur][16 * w + (lane & 15)][4 * ks + gq];
-#pragma unroll
-      for (int t = 0; t < OC16; ++t) acc1[t] = R::mma(a, sB[cur][4 * ks + gq][16 * t + (lane & 15)], acc1[t]);
-    }
-    if (c + 1 < OC16) stash1(cur ^ 1);
-    if (c + 2 < OC16) fetch1((c + 2) * kBK);
-    __syncthreads();
-  }
-  // every wave is past its last read of the staging buffers: W_I replaces them
+  fetch(0);
+
+  // ---- phase 1: acc1[t][i] = rows l = 16 t .., columns a = 32 I + 2 m + i of W^T
+  Acc acc1[OC16][2];
 #pragma unroll
   for (int t = 0; t < OC16; ++t)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) sW[16 * w + R::row(lane, r)][16 * t + (lane & 15)] = acc1[t][r];
-  __syncthreads();
-
-  // ---- phase 2: the blocks W_I C_j^T, j = 0..I, as one stream of chunks.
-  // Every column tile is straight-line code (its OC16 chunks unrolled, the
-  // fragment stage of each chunk a compile-time constant) issuing the same
-  // global operations wherever it sits: the fragments of the chunk after
-  // next are loaded even past the last chunk (clamped to it, never used),
-  // and the epilogue stores every element, those above the diagonal or past
-  // n with an offset past the buffer's range, which the hardware drops.  The vector memory counter of this
-  // architecture counts loads and stores in one queue, so with a fixed count
-  // per tile the compiler's waits are exact: the epilogue waits for the
-  // tile's density values only, a chunk for its own fragments, and neither
-  // for the stores of the tile before (conditional stores made it drain the
-  // whole queue once per tile).
-  const int wm = w >> 1, wn = w & 1;
-  const int Q = (I + 1) * OC16;
-  const double vj = g.gv * g.v[J];
-  const double *__restrict__ P = g.p;
-  double *__restrict__ G = g.g + J * g.ldg;
-  const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc(G, 0, g.rowbytes, kRsrcWord3);
-  const __amdgpu_buffer_rsrc_t rp =
-      __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(P), 0, g.rowbytes, kRsrcWord3);
-  typedef typename R::T4 T4;
-  T4 bq[2][2];  // [stage][jj]: C_j fragments of the chunks in flight
-  auto loadB = [&](int q, T4 (&dst)[2]) __attribute__((always_inline)) {
-    q = q < Q ? q : Q - 1;
-    const int j = q / OC16, kc = q - j * OC16;
+    for (int i = 0; i < 2; ++i) acc1[t][i] = Acc{0, 0, 0, 0};
+  {
+    const int ns = (o + 3) / 4;  // steps of four contraction indices
+    T zr[2][OC16];
+    T2 cr[2];
+    const T *__restrict__ ca = ct + gq * int64_t(ldt) + 32 * I + 2 * m;
+    uint32_t zo[OC16];  // column l of this lane, clamped
 #pragma unroll
-    for (int jj = 0; jj < 2; ++jj) {
-      const uint32_t row = uint32_t(j * kTM + wn * 32 + jj * 16 + (lane & 15));
-      dst[jj] = *reinterpret_cast<const T4 *>(cb + row * uint32_t(ldc) + uint32_t(kc * kBK + 4 * gq));
+    for (int t = 0; t < OC16; ++t) zo[t] = uint32_t(min(16 * t + m, o - 1));
+    auto load = [&](int s, int st) __attribute__((always_inline)) {
+      s = min(s, ns - 1);
+      const uint32_t zrow = uint32_t(min(4 * s + gq, o - 1)) * uint32_t(ldz);
+      cr[st] = *reinterpret_cast<const T2 *>(ca + 4 * s * int64_t(ldt));
+#pragma unroll
+      for (int t = 0; t < OC16; ++t) zr[st][t] = T(zj[zrow + zo[t]]);
+    };
+    auto mul = [&](int s, int st) __attribute__((always_inline)) {
+      const int k = 4 * s + gq;
+#pragma unroll
+      for (int t = 0; t < OC16; ++t) {
+        T z = zr[st][t];
+        if constexpr (!HP) z = T(g.beta) * z + (k == 16 * t + m ? T(2.0 * vj) : T(0));
+        const T a = k < o && 16 * t + m < o ? z : T(0);
+        acc1[t][0] = R::mma(a, cr[st][0], acc1[t][0]);
+        acc1[t][1] = R::mma(a, cr[st][1], acc1[t][1]);
+      }
+    };
+    load(0, 0);
+    load(1, 1);
+    // two steps per trip (one past the last multiplies by zeros: a conditional
+    // step would give the accumulators a second set of registers)
+#pragma unroll 1
+    for (int s = 0; s < ns; s += 2) {
+      mul(s, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      load(s + 2, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      mul(s + 1, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      load(s + 3, 1);
+      __builtin_amdgcn_sched_barrier(0);
     }
-  };
-  Acc acc2[2][2];
+  }
+
+  // ---- phase 2
+  // steps of a tile's last chunk that hold an index below nocc: step s has the
+  // indices row(g, s), 4 s + g (FP64) or 4 g + s (FP32)
+  const int left = o - 16 * (OC16 - 1), tail = R::kStep == 4 ? (left + 3) / 4 : min(left, 4);
+  uint32_t ro[2][4];  // byte offset of this lane's first element in each of its rows
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int jj = 0; jj < 2; ++jj) acc2[i][jj] = Acc{0, 0, 0, 0};
-  // P values of the tile in progress, loaded at its start so the epilogue
-  // only stores
-  double pv[2][2][4];
-  uint32_t pi[2][2][4];
-  auto load_p = [&](int j) __attribute__((always_inline)) {
+    for (int r = 0; r < 4; ++r) {
+      const uint32_t a = uint32_t(32 * I + 2 * R::row(gq, r) + i);
+      ro[i][r] = a < uint32_t(g.n) ? (a * (a + 1u) / 2u + uint32_t(2 * m)) * 8u : kMasked;
+    }
+  Acc acc2[2][2];
+  // The contraction index of (step s, lane group) is the one phase 1 left in
+  // register s: row(gq, s) of the chunk.
+  auto chunks = [&](int buf) __attribute__((always_inline)) {
+    constexpr int D = OC16 < 8 || sizeof(T) == 4 ? 4 : 2;  // steps of fragments in flight (registers)
+    T2 bq[D];
+    auto load_b = [&](int u, T2 &dst) __attribute__((always_inline)) {
+      dst = *reinterpret_cast<const T2 *>(&sB[buf][(16 * (u / 4) + R::row(gq, u % 4)) * 32 + 2 * m]);
+    };
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int jj = 0; jj < 2; ++jj)
+      for (int h = 0; h < 2; ++h) acc2[i][h] = Acc{0, 0, 0, 0};
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const uint32_t gi = uint32_t(i0 + wm * 32 + i * 16 + R::row(lane, r));
-          const uint32_t gj = uint32_t(j * kTM + wn * 32 + jj * 16 + (lane & 15));
-          const bool ok = gi < uint32_t(g.n) && gi >= gj;
-          pi[i][jj][r] = (ok ? gi * (gi + 1u) / 2u + gj : kMasked) * 8u;  // byte offset
-          pv[i][jj][r] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rp, int(pi[i][jj][r]), 0, 0));
-        }
-  };
-  auto epilogue = [&](int j) __attribute__((always_inline)) {
+    for (int u = 0; u < D; ++u) load_b(u, bq[u]);
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const uint32_t gi = uint32_t(i0 + wm * 32 + i * 16 + R::row(lane, r));
-          const uint32_t gj = uint32_t(j * kTM + wn * 32 + jj * 16 + (lane & 15));
-          const double val = (gi == gj ? 1.0 : 2.0) * (vj * pv[i][jj][r] + g.beta * double(acc2[i][jj][r]));
-          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, val), rg, int(pi[i][jj][r]), 0, 0);
-        }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int jj = 0; jj < 2; ++jj) acc2[i][jj] = Acc{0, 0, 0, 0};
-  };
-  // Column tile j; PAR = parity of its first chunk in the stream (chunk q
-  // uses fragment stage q & 1 and refills it with chunk q + 2).
-  // The scheduler keeps each chunk to itself (sched_barrier): hoisting the
-  // loads and LDS reads of later chunks raised the register count to the
-  // point of one wave per SIMD.
-  auto tile = [&](int j, auto parity) __attribute__((always_inline)) {
-    constexpr int PAR = decltype(parity)::value;
-    load_p(j);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int kc = 0; kc < OC16; ++kc) {
-      const int S = (PAR + kc) & 1;
-      const T4 b0 = bq[S][0], b1 = bq[S][1];
-      loadB(j * OC16 + kc + 2, bq[S]);
-      T4 a4[2];
-      if constexpr (F32) {
+    for (int u = 0; u < 4 * OC16; ++u) {
+      if (u < 4 * (OC16 - 1) || u - 4 * (OC16 - 1) < tail) {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
-          a4[i] = *reinterpret_cast<const T4 *>(&sW[wm * 32 + i * 16 + (lane & 15)][kc * kBK + 4 * gq]);
-      }
 #pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        T af[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-          af[i] = F32 ? a4[i][ks] : sW[wm * 32 + i * 16 + (lane & 15)][kc * kBK + 4 * gq + ks];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          acc2[i][0] = R::mma(af[i], b0[ks], acc2[i][0]);
-          acc2[i][1] = R::mma(af[i], b1[ks], acc2[i][1]);
-        }
+          for (int h = 0; h < 2; ++h) acc2[i][h] = R::mma(acc1[u / 4][i][u % 4], bq[u % D][h], acc2[i][h]);
       }
       __builtin_amdgcn_sched_barrier(0);
+      if (u + D < 4 * OC16) load_b(u + D, bq[u % D]);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    epilogue(j);
-    __builtin_amdgcn_sched_barrier(0);
   };
-  // tile j starts at chunk j OC16: parity 0 for even j, OC16 & 1 for odd j.
-  // Tile 0 runs before the loop so that both ways into the loop end with an
-  // epilogue and the wait counts at the loop head stay exact.
-  loadB(0, bq[0]);
-  loadB(1, bq[1]);
-  tile(0, std::integral_constant<int, 0>{});
-  int j = 1;
-  for (; j + 1 <= I; j += 2) {
-    tile(j, std::integral_constant<int, OC16 & 1>{});
-    tile(j + 1, std::integral_constant<int, 0>{});
+  // element before the factor 2 off the diagonal
+  auto value = [&](int i, int h, int r, double p) __attribute__((always_inline)) {
+    const double x = double(acc2[i][h][r]);
+    if constexpr (HP) return vj * p + g.beta * x;
+    else return x;
+  };
+  stash(0);
+  __syncthreads();
+#pragma unroll 1
+  for (int j = 0; j < I; ++j) {  // tiles wholly below the diagonal
+    fetch(j + 1);
+    v4u pv[2][4];
+    constexpr bool kLate = OC16 >= 7 && sizeof(T) == 8;  // no registers for the densities beside the products
+    auto load_p = [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          pv[i][r] = __builtin_amdgcn_raw_buffer_load_b128(rp, int(ro[i][r] + 256u * uint32_t(j)), 0, 0);
+    };
+    if constexpr (HP && !kLate) load_p();
+    __builtin_amdgcn_sched_barrier(0);
+    chunks(j & 1);
+    __builtin_amdgcn_sched_barrier(0);
+    stash((j + 1) & 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (HP && kLate) load_p();
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        v2d p = {0.0, 0.0};
+        if constexpr (HP) p = __builtin_bit_cast(v2d, pv[i][r]);
+        v2d x;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) x[h] = 2.0 * value(i, h, r, p[h]);
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4u, x), rg, int(ro[i][r] + 256u * uint32_t(j)), 0, 0);
+      }
+    __syncthreads();
   }
-  if (j <= I) tile(j, std::integral_constant<int, OC16 & 1>{});
+  // the diagonal tile
+  auto po = [&](int i, int h, int r) __attribute__((always_inline)) {
+    return int(2 * R::row(gq, r) + i >= 2 * m + h ? ro[i][r] + 256u * uint32_t(I) + 8u * h : kMasked);
+  };
+  chunks(I & 1);
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const double f = 2 * R::row(gq, r) + i == 2 * m + h ? 1.0 : 2.0;
+        double p = 0.0;
+        if constexpr (HP) p = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(rp, po(i, h, r), 0, 0));
+        const double x = f * value(i, h, r, p);
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, x), rg, po(i, h, r), 0, 0);
+      }
+}
+
+// ct[k * n_pad + a] = T(cb[a * ldc + k]) for k < rows, 32 x 32 blocks through LDS.
+// grid = (n_pad / 32, ceil(rows / 32)), block 256.
+template <typename T>
+__global__ __launch_bounds__(kThreads) void k_bank_t(const double *__restrict__ cb, int ldc, int n_pad, int rows,
+                                                    T *__restrict__ ct) {
+  __shared__ double t[32][33];
+  const int a0 = blockIdx.x * 32, k0 = blockIdx.y * 32, x = threadIdx.x & 31, y = threadIdx.x >> 5;
+#pragma unroll
+  for (int i = y; i < 32; i += 8)
+    t[i][x] = k0 + x < ldc ? cb[int64_t(a0 + i) * ldc + k0 + x] : 0.0;
+  __syncthreads();
+#pragma unroll
+  for (int i = y; i < 32; i += 8)
+    if (k0 + i < rows) ct[int64_t(k0 + i) * n_pad + a0 + x] = T(t[x][i]);
 }
 
 template <int OC16>
-void launch_grad_rows(Context *c, const GradRows &g) {
-  if (g.cb32)
-    hipLaunchKernelGGL((k_grad_rows<OC16, GR32>), dim3(unsigned(round_up(g.items, 8))), dim3(kThreads), 0,
-                       c->stream, g);
-  else
-    hipLaunchKernelGGL((k_grad_rows<OC16, GR64>), dim3(unsigned(round_up(g.items, 8))), dim3(kThreads), 0,
-                       c->stream, g);
+void launch_grad_rows(Context *c, const GradRows &g, bool f32) {
+  const dim3 grid(unsigned(round_up(g.items, 8)));
+  if (f32) hipLaunchKernelGGL((k_grad_rows<OC16, GR32, true>), grid, dim3(kThreads), 0, c->stream, g);
+  else if (g.p) hipLaunchKernelGGL((k_grad_rows<OC16, GR64, true>), grid, dim3(kThreads), 0, c->stream, g);
+  else hipLaunchKernelGGL((k_grad_rows<OC16, GR64, false>), grid, dim3(kThreads), 0, c->stream, g);
 }
 
 // Whether the fused k_grad_rows takes this shape: nocc <= 128, 32-bit bank
@@ -584,20 +592,36 @@ bool grad_rows_fits(const Context *c, int nocc, int ldc) {
   return (nocc + 15) / 16 <= 8 && int64_t(c->n_pad) * ldc < (int64_t(1) << 28) && rowbytes < (int64_t(1) << 31);
 }
 
-// dL of the jn vectors from Z in one fused launch; returns MJK_ERR_ARG when
-// grad_rows_fits rejects the shape (the caller then forms W = C Z first).
-// cb32: the bank in FP32 for FP32 products, or null for FP64.
+// The transposed bank of k_grad_rows in FP64 or FP32 (workspaces gbt / gb32) from
+// the packed FP64 bank.
+int bank_t(Context *c, int nocc, int ldc, bool f32) {
+  const int rows = 16 * ((nocc + 15) / 16);
+  DevBuf &buf = f32 ? c->w->gb32 : c->w->gbt;
+  const int rc = ensure(c, buf, (f32 ? sizeof(float) : sizeof(double)) * size_t(rows) * c->n_pad);
+  if (rc) return rc;
+  const double *cb = static_cast<const double *>(c->w->cbank.ptr);
+  const dim3 grid(unsigned(c->n_pad / 32), unsigned(ceil_div(rows, 32)));
+  if (f32)
+    hipLaunchKernelGGL(k_bank_t<float>, grid, dim3(kThreads), 0, c->stream, cb, ldc, c->n_pad, rows,
+                       static_cast<float *>(buf.ptr));
+  else
+    hipLaunchKernelGGL(k_bank_t<double>, grid, dim3(kThreads), 0, c->stream, cb, ldc, c->n_pad, rows,
+                       static_cast<double *>(buf.ptr));
+  return hip_check(c, hipGetLastError(), "bank transpose launch");
+}
+
+// dL of the jn vectors from Z in one fused launch, with FP64 or FP32 products
+// (bank_t() of that precision first); returns MJK_ERR_ARG when grad_rows_fits
+// rejects the shape (the caller then forms W = C Z first).
 int grad_rows(Context *c, int nocc, int ldc, const double *z, int64_t sz, int ldz, const double *v,
-              const double *P, double alpha, double beta, double *dl, int64_t ldd, int64_t jn,
-              const float *cb32) {
+              const double *P, double alpha, double beta, double *dl, int64_t ldd, int64_t jn, bool f32) {
   const int oc16 = (nocc + 15) / 16;
   if (!grad_rows_fits(c, nocc, ldc)) return MJK_ERR_ARG;
   if (jn < 1) return MJK_OK;
   GradRows g{};
   g.rowbytes = int32_t(int64_t(c->n) * (c->n + 1) / 2 * int64_t(sizeof(double)));
-  g.cb = static_cast<const double *>(c->w->cbank.ptr);
-  g.cb32 = cb32;
-  g.ldc = ldc;
+  g.ct = f32 ? c->w->gb32.ptr : c->w->gbt.ptr;
+  g.n_pad = c->n_pad;
   g.z = z;
   g.sz = sz;
   g.ldz = ldz;
@@ -609,17 +633,18 @@ int grad_rows(Context *c, int nocc, int ldc, const double *z, int64_t sz, int ld
   g.g = dl;
   g.ldg = ldd;
   g.n = c->n;
-  g.T = int(ceil_div(c->n, kTM));
-  g.items = int64_t(g.T) * jn;
+  g.T = int(ceil_div(c->n, 32));
+  g.jn = jn;
+  g.items = int64_t(g.T) * ceil_div(jn, 4);
   switch (oc16) {
-    case 1: launch_grad_rows<1>(c, g); break;
-    case 2: launch_grad_rows<2>(c, g); break;
-    case 3: launch_grad_rows<3>(c, g); break;
-    case 4: launch_grad_rows<4>(c, g); break;
-    case 5: launch_grad_rows<5>(c, g); break;
-    case 6: launch_grad_rows<6>(c, g); break;
-    case 7: launch_grad_rows<7>(c, g); break;
-    default: launch_grad_rows<8>(c, g); break;
+    case 1: launch_grad_rows<1>(c, g, f32); break;
+    case 2: launch_grad_rows<2>(c, g, f32); break;
+    case 3: launch_grad_rows<3>(c, g, f32); break;
+    case 4: launch_grad_rows<4>(c, g, f32); break;
+    case 5: launch_grad_rows<5>(c, g, f32); break;
+    case 6: launch_grad_rows<6>(c, g, f32); break;
+    case 7: launch_grad_rows<7>(c, g, f32); break;
+    default: launch_grad_rows<8>(c, g, f32); break;
   }
   return MJK_OK;
 }
@@ -900,8 +925,12 @@ extern "C" int mjk_grad_vectors(mjk_context *c, int32_t nocc, const double *corb
   double *X = static_cast<double *>(c->w->x.ptr);
   double *Z = X + jc * ldc * int64_t(n_pad);
   double *W = Z + jc * ldc * int64_t(ldc);
-  const double *P = nullptr;  // caller's plain LT, or 2 C C^T
-  if ((rc = density_or(c, nocc, corb, p_lt, &P))) return rc;
+  const double *P = p_lt;  // caller's plain LT; without one the fused kernel needs none, the two-GEMM form 2 C C^T
+  if (grad_rows_fits(c, nocc, ldc)) {
+    if ((rc = bank_t(c, nocc, ldc, false))) return rc;
+  } else if ((rc = density_or(c, nocc, corb, p_lt, &P))) {
+    return rc;
+  }
   for (int64_t ch = 0; ch < nchunk; ++ch) {
     const int64_t j0 = ch * jc, jn = std::min(jc, M - j0);
     phase_begin(c);
@@ -923,7 +952,7 @@ extern "C" int mjk_grad_vectors(mjk_context *c, int32_t nocc, const double *corb
     }
     // dL[J] = s * (alpha V_J P + beta C Z[J] C^T), lower triangle, packed
     if (grad_rows(c, nocc, ldc, Z, int64_t(ldc) * ldc, ldc, v + j0, P, alpha, beta, dl + j0 * ldd,
-                  ldd, jn, nullptr) != MJK_OK) {  // nocc > 128: W = C Z first
+                  ldd, jn, false) != MJK_OK) {  // nocc > 128: W = C Z first
       g = GemmBatch{};
       g.A = cb; g.sA = 0; g.lda = ldc;
       g.B = Z; g.sB = int64_t(ldc) * ldc; g.ldb = ldc;
@@ -938,11 +967,6 @@ extern "C" int mjk_grad_vectors(mjk_context *c, int32_t nocc, const double *corb
 }
 
 namespace {
-__global__ void k_bank_f32(const double *__restrict__ src, float *__restrict__ dst, int64_t cnt) {
-  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < cnt; i += int64_t(gridDim.x) * blockDim.x)
-    dst[i] = float(src[i]);
-}
-
 // dE/dL from a given Z; vectors [j_fp32, M) take FP32 products (nocc <= 128).
 int grad_vectors_z_impl(Context *c, int32_t nocc, const double *corb, const double *p_lt,
                         const double *v, const double *z, double alpha, double beta, double *dl,
@@ -961,21 +985,15 @@ int grad_vectors_z_impl(Context *c, int32_t nocc, const double *corb, const doub
   const int ldc = 16 * ot;
   const double *cb = static_cast<const double *>(c->w->cbank.ptr);
   if (grad_rows_fits(c, nocc, ldc)) {  // one fused launch per precision: W = C Z stays on chip
-    const double *P = nullptr;
-    if ((rc = density_or(c, nocc, corb, p_lt, &P))) return rc;
-    const float *cb32 = nullptr;
-    if (j_fp32 < M) {
-      const int64_t cnt = int64_t(n_pad) * ldc;
-      if ((rc = ensure(c, c->w->gb32, sizeof(float) * size_t(cnt)))) return rc;
-      hipLaunchKernelGGL(k_bank_f32, dim3(unsigned(std::min<int64_t>(ceil_div(cnt, 256), 4096))), dim3(256), 0,
-                         c->stream, cb, static_cast<float *>(c->w->gb32.ptr), cnt);
-      cb32 = static_cast<const float *>(c->w->gb32.ptr);
-    }
+    const double *P = p_lt;
+    if (j_fp32 < M && (rc = density_or(c, nocc, corb, p_lt, &P))) return rc;
+    if (j_fp32 > 0 && (rc = bank_t(c, nocc, ldc, false))) return rc;
+    if (j_fp32 < M && (rc = bank_t(c, nocc, ldc, true))) return rc;
     const int64_t sz = int64_t(nocc) * nocc;
     phase_begin(c);
-    if ((rc = grad_rows(c, nocc, ldc, z, sz, nocc, v, P, alpha, beta, dl, ldd, j_fp32, nullptr)) ||
+    if ((rc = grad_rows(c, nocc, ldc, z, sz, nocc, v, p_lt, alpha, beta, dl, ldd, j_fp32, false)) ||
         (rc = grad_rows(c, nocc, ldc, z + j_fp32 * sz, sz, nocc, v + j_fp32, P, alpha, beta,
-                        dl + j_fp32 * ldd, ldd, M - j_fp32, cb32)))
+                        dl + j_fp32 * ldd, ldd, M - j_fp32, true)))
       return set_error(c, rc, std::string(who) + ": fused gradient launch");
     phase_end(c, MJK_PHASE_BACKWARD);
     return hip_check(c, hipGetLastError(), "grad_vectors_z launch");
