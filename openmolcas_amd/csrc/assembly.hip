@@ -8,15 +8,22 @@
 namespace mjk {
 namespace {
 
-// flt[p] += fj*jlt[p] + fk*klt[p]  (either source may be null)
-__global__ void k_fock_update(double *__restrict__ flt, const double *__restrict__ jlt, double fj,
-                              const double *__restrict__ klt, double fk, int64_t np) {
+// flt[d][p] += fj*jlt[p] + fk*klt[p] for up to kFockSets densities in one launch
+// (either source may be null).  grid = (ceil(np / 256), densities).
+constexpr int kFockSets = 16;
+struct FockSets {
+  double *flt[kFockSets];
+  const double *jlt[kFockSets], *klt[kFockSets];
+  double fj[kFockSets], fk[kFockSets];
+};
+__global__ void k_fock_update(const FockSets s, int64_t np) {
   const int64_t p = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int d = blockIdx.y;
   if (p >= np) return;
-  double v = flt[p];
-  if (jlt) v += fj * jlt[p];
-  if (klt) v += fk * klt[p];
-  flt[p] = v;
+  double v = s.flt[d][p];
+  if (s.jlt[d]) v += s.fj[d] * s.jlt[d][p];
+  if (s.klt[d]) v += s.fk[d] * s.klt[d][p];
+  s.flt[d][p] = v;
 }
 
 constexpr int kRedThreads = 256;
@@ -70,11 +77,18 @@ int fock_update(Context *c, int32_t nd, double *flt, int64_t ldf, const double *
   if (nd < 1) return set_error(c, MJK_ERR_ARG, "fock_update: nd < 1");
   if (ldf < c->np) return set_error(c, MJK_ERR_ARG, "fock_update: ldf < nbas(nbas+1)/2");
   phase_begin(c);
-  for (int d = 0; d < nd; ++d) {
-    const double *js = (jlt && jsrc && jsrc[d] >= 0) ? jlt + jsrc[d] * ldj : nullptr;
-    const double *ks = klt ? klt + d * ldk : nullptr;
-    hipLaunchKernelGGL(k_fock_update, dim3(unsigned(ceil_div(c->np, 256))), dim3(256), 0,
-                       c->stream, flt + d * ldf, js, fj ? fj[d] : 0.0, ks, fk ? fk[d] : 0.0,
+  for (int d0 = 0; d0 < nd; d0 += kFockSets) {
+    const int m = std::min(kFockSets, nd - d0);
+    FockSets s{};
+    for (int i = 0; i < m; ++i) {
+      const int d = d0 + i;
+      s.flt[i] = flt + d * ldf;
+      s.jlt[i] = (jlt && jsrc && jsrc[d] >= 0) ? jlt + jsrc[d] * ldj : nullptr;
+      s.klt[i] = klt ? klt + d * ldk : nullptr;
+      s.fj[i] = fj ? fj[d] : 0.0;
+      s.fk[i] = fk ? fk[d] : 0.0;
+    }
+    hipLaunchKernelGGL(k_fock_update, dim3(unsigned(ceil_div(c->np, 256)), unsigned(m)), dim3(256), 0, c->stream, s,
                        c->np);
   }
   phase_end(c, MJK_PHASE_ASSEMBLY);

@@ -151,15 +151,30 @@ __global__ __launch_bounds__(kThreads) void k_coulomb_j(
             acc[w][d];
 }
 
-// jlt(d*ldj + p) = sum_s jpart[(s*nd + d)*ldl + p], p < np.
-__global__ void k_reduce_j(const double *__restrict__ jpart, int64_t ldl, int64_t np, int nd,
-                           int nsplit, double *__restrict__ jlt, int64_t ldj) {
-  const int64_t p = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int d = blockIdx.y;
-  if (p >= np) return;
+// jlt(d*ldj + p) = sum_s jpart[(s*nd + d)*ldl + p], p < np.  Thread (q, pair)
+// sums every fourth slice from the q-th, eight loads in flight, in a fixed order:
+// one thread per pair took the slices one load after the other (137 of them at
+// n=24: 33 us, now 4).  grid = (ceil(np / 64), nd), block 256.
+__global__ __launch_bounds__(kThreads) void k_reduce_j(const double *__restrict__ jpart, int64_t ldl, int64_t np,
+                                                      int nd, int nsplit, double *__restrict__ jlt, int64_t ldj) {
+  __shared__ double red[3][64];
+  const int cb = threadIdx.x & 63, q = threadIdx.x >> 6, d = blockIdx.y;
+  const int64_t p = int64_t(blockIdx.x) * 64 + cb;
+  const double *__restrict__ src = jpart + d * ldl + min(p, np - 1);
+  const int64_t stride = nd * ldl;
   double s = 0.0;
-  for (int k = 0; k < nsplit; ++k) s += jpart[(int64_t(k) * nd + d) * ldl + p];
-  jlt[d * ldj + p] = s;
+  int k = q;
+  for (; k + 28 < nsplit; k += 32) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = src[(k + 4 * u) * stride];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) s += v[u];
+  }
+  for (; k < nsplit; k += 4) s += src[k * stride];
+  if (q > 0) red[q - 1][cb] = s;
+  __syncthreads();
+  if (q == 0 && p < np) jlt[d * ldj + p] = ((s + red[0][cb]) + red[1][cb]) + red[2][cb];
 }
 
 // Copies nd densities of stride ldd into the zero-padded staging buffer of
@@ -395,12 +410,13 @@ constexpr int kTileVM = 64, kTileVK = 64, kTileU = 4;  // MFMA passes (nd >= 3)
 inline size_t piece(size_t bytes) { return size_t(round_up(int64_t(bytes), 256)); }
 
 // Pass 2 split of the streaming J pass for ndt densities: about 1024
-// workgroups of two segments, 2048 of one.
+// workgroups of two segments, 2048 of one, at least eight vectors each (a slice
+// of one vector costs more to write and reduce than to read).
 void plan_j_stream(const Context *c, int nd, int ndt, CoulombPlan *p) {
   const int64_t M = c->nchol, nseg = c->ldl / kSeg;
   const int64_t nxj = ceil_div(nseg, j_width(ndt));
   int nsplit2 = int(std::min<int64_t>(std::max<int64_t>(ceil_div(2048 / j_width(ndt), nxj), 1), M));
-  p->jchunk = ceil_div(M, nsplit2);
+  p->jchunk = std::max<int64_t>(ceil_div(M, nsplit2), 8);
   p->nsplit2 = int(ceil_div(M, p->jchunk));
   p->bytes_jpart = sizeof(double) * size_t(p->nsplit2) * nd * c->ldl;
 }
@@ -477,7 +493,7 @@ int j_pass(Context *c, Scratch &s, const CoulombPlan &p, int nd, const double *V
   }
   phase_end(c, MJK_PHASE_COULOMB_J);
   phase_begin(c);
-  hipLaunchKernelGGL(k_reduce_j, dim3(unsigned(ceil_div(c->np, 256)), unsigned(nd)), dim3(256), 0,
+  hipLaunchKernelGGL(k_reduce_j, dim3(unsigned(ceil_div(c->np, 64)), unsigned(nd)), dim3(256), 0,
                      c->stream, jpart, c->ldl, c->np, nd, p.nsplit2, jlt, ldj);
   phase_end(c, MJK_PHASE_REDUCE);
   return hip_check(c, hipGetLastError(), "coulomb launch");
@@ -521,7 +537,7 @@ int coulomb_run(Context *c, Scratch &s, int32_t nd, const double *dlt, int64_t l
                        dim3(kThreads), 0, c->stream, c->L, ldl, M, V, nd, p.jchunk, jpart);
     phase_end(c, MJK_PHASE_COULOMB_J);
     phase_begin(c);
-    hipLaunchKernelGGL(k_reduce_j, dim3(unsigned(ceil_div(c->np, 256)), unsigned(nd)), dim3(256), 0,
+    hipLaunchKernelGGL(k_reduce_j, dim3(unsigned(ceil_div(c->np, 64)), unsigned(nd)), dim3(256), 0,
                        c->stream, jpart, ldl, c->np, nd, p.nsplit2, jlt, ldj);
     phase_end(c, MJK_PHASE_REDUCE);
     return hip_check(c, hipGetLastError(), "coulomb launch");

@@ -108,14 +108,29 @@ __device__ inline int64_t xcd_logical(int64_t nblocks) {
 }
 
 // ---- orbital bank --------------------------------------------------------
-// Cb[a*ldc + off + k] = corb[k + a*nocc] for a < n, k < nocc.
+// Orbital sets of one call: set d fills the bank columns off[d] .. of nocc[d]
+// orbitals, element (k, a) at c[d][k + a * nocc[d]].
+struct OrbSets {
+  int n;
+  const double *c[kMaxSets];
+  int nocc[kMaxSets];
+  int off[kMaxSets];
+};
+
+__device__ __forceinline__ double bank_value(const OrbSets &sets, int a, int col, int n) {
+  int d = 0;
+  while (d + 1 < sets.n && col >= sets.off[d + 1]) ++d;
+  const int k = col - sets.off[d];
+  return a < n && k < sets.nocc[d] ? sets.c[d][k + int64_t(a) * sets.nocc[d]] : 0.0;
+}
+
+// Cb[a*ldc + col], every element of the n_pad x ldc bank in one launch (a zero
+// fill and a launch per set before).
 template <typename T>
-__global__ void k_pack_orb(const double *__restrict__ corb, int nocc, int n, int ldc, int off,
-                           T *__restrict__ cb) {
+__global__ void k_pack_orb(const OrbSets sets, int n, int n_pad, int ldc, T *__restrict__ cb) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= int64_t(nocc) * n) return;
-  const int64_t a = i / nocc, k = i % nocc;
-  cb[a * ldc + off + k] = T(corb[i]);
+  if (i >= int64_t(n_pad) * ldc) return;
+  cb[i] = T(bank_value(sets, int(i / ldc), int(i % ldc), n));
 }
 
 // FP32 shadow of the resident vectors for the mixed-precision exchange.
@@ -1196,16 +1211,15 @@ __device__ inline v4f mma_b3(bf16x8 ah, bf16x8 al, bf16x8 bh, bf16x8 bl, v4f acc
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh, acc, 0, 0, 0);
 }
 
-// Transposed split bank: ch/cl[(off + k)*n_pad + a] = hi/lo(corb[k + a*nocc]).
-__global__ void k_pack_orb_b3(const double *__restrict__ corb, int nocc, int n, int n_pad, int off,
-                              __bf16 *__restrict__ ch, __bf16 *__restrict__ cl) {
+// Transposed split bank: ch/cl[col*n_pad + a] = hi/lo of the bank element.
+__global__ void k_pack_orb_b3(const OrbSets sets, int n, int n_pad, int ldc, __bf16 *__restrict__ ch,
+                              __bf16 *__restrict__ cl) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= int64_t(nocc) * n) return;
-  const int64_t a = i / nocc, k = i % nocc;
+  if (i >= int64_t(n_pad) * ldc) return;
   __bf16 h, l;
-  split_bf16(float(corb[i]), h, l);
-  ch[(off + k) * int64_t(n_pad) + a] = h;
-  cl[(off + k) * int64_t(n_pad) + a] = l;
+  split_bf16(float(bank_value(sets, int(i % n_pad), int(i / n_pad), n)), h, l);
+  ch[i] = h;
+  cl[i] = l;
 }
 
 // Half-transform, same work decomposition as k_ht: X[(jr*LDC + k)*n_pad + a].
@@ -1610,9 +1624,23 @@ template <int OT>
 void launch_ht64(Context *c, const double *cb, int64_t j0, int64_t jc, double *X) {
   constexpr int NB = ht64_nb(OT);
   const int64_t nblk = ceil_div(c->n, 16);
-  // fewer blocks per wave while the launch has less than two waves per SIMD
+  // Column blocks per wave of a launch of few rounds of resident workgroups: the
+  // count whose last round wastes least (a wave's time goes with its blocks, plus
+  // about half a block for its share of the bank and the barriers).  n=187
+  // nchol=905 nocc=23: three blocks 84 us (905 workgroups on 768 slots), two 77.
+  constexpr int64_t kPerCu = OT <= 5 ? 3 : 2;
+  const int64_t slots = kPerCu * c->ncu;
   int nb = NB;
-  while (nb > 1 && jc * ceil_div(nblk, nb) < 8 * int64_t(c->ncu)) --nb;
+  double least = 1e300;
+  for (int v = NB; v >= 1; --v) {
+    const int64_t wgs = ceil_div(jc * ceil_div(nblk, v), 4), rounds = ceil_div(wgs, slots);
+    if (v == NB && rounds > 8) break;
+    const double cost = double(rounds) * (v + 0.5);
+    if (cost < least) {
+      least = cost;
+      nb = v;
+    }
+  }
   const int W = int(ceil_div(nblk, nb));
   const int64_t nblocks = ceil_div(jc * W, 4);
   const dim3 grid(unsigned(round_up(nblocks, 8)));
@@ -1739,24 +1767,28 @@ void syrk_launch_b3(Context *c, int tm, int items, const float *X, int ldc, int6
                        c->n_pad, ldc, jn, ntiles, sets, kpart, chunk);
 }
 
+OrbSets orb_sets(int32_t nk, const int32_t *nocc, const double *const *corb, const std::vector<int> &off) {
+  OrbSets s{};
+  s.n = nk;
+  for (int d = 0; d < nk; ++d) {
+    s.c[d] = corb[d];
+    s.nocc[d] = nocc[d];
+    s.off[d] = off[size_t(d)];
+  }
+  return s;
+}
+
 int pack_bank_b3(Context *c, int32_t nk, const int32_t *nocc, const double *const *corb,
                  const std::vector<int> &off, int ldc, DevBuf &buf) {
-  const int n = c->n, n_pad = c->n_pad;
-  const size_t half = sizeof(__bf16) * size_t(ldc) * n_pad;
+  const int64_t half = int64_t(ldc) * c->n_pad;
   int rc;
-  if ((rc = ensure(c, buf, 2 * half))) return rc;
+  if ((rc = ensure(c, buf, 2 * sizeof(__bf16) * size_t(half)))) return rc;
   __bf16 *ch = static_cast<__bf16 *>(buf.ptr);
-  __bf16 *cl = ch + size_t(ldc) * n_pad;
   phase_begin(c);
-  if ((rc = fill_zero(c, ch, 2 * half))) return rc;
-  for (int d = 0; d < nk; ++d) {
-    if (nocc[d] == 0) continue;
-    const int64_t cnt = int64_t(nocc[d]) * n;
-    hipLaunchKernelGGL(k_pack_orb_b3, dim3(unsigned(ceil_div(cnt, 256))), dim3(256), 0, c->stream,
-                       corb[d], nocc[d], n, n_pad, off[size_t(d)], ch, cl);
-  }
+  hipLaunchKernelGGL(k_pack_orb_b3, dim3(unsigned(ceil_div(half, 256))), dim3(256), 0, c->stream,
+                     orb_sets(nk, nocc, corb, off), c->n, c->n_pad, ldc, ch, ch + half);
   phase_end(c, MJK_PHASE_PACK);
-  return MJK_OK;
+  return hip_check(c, hipGetLastError(), "bank launch");
 }
 
 // Layout of the bank for nk sets; returns MJK_OK and ot = 0 when empty.  The
@@ -1788,21 +1820,14 @@ int bank_layout(Context *c, int32_t nk, const int32_t *nocc, std::vector<int> &o
 template <typename T>
 int pack_bank_t(Context *c, int32_t nk, const int32_t *nocc, const double *const *corb,
                 const std::vector<int> &off, int ldc, DevBuf &buf) {
-  const int n = c->n, n_pad = c->n_pad;
-  const size_t bytes = sizeof(T) * size_t(n_pad) * ldc;
+  const int64_t cnt = int64_t(c->n_pad) * ldc;
   int rc;
-  if ((rc = ensure(c, buf, bytes))) return rc;
-  T *cb = static_cast<T *>(buf.ptr);
+  if ((rc = ensure(c, buf, sizeof(T) * size_t(cnt)))) return rc;
   phase_begin(c);
-  if ((rc = fill_zero(c, cb, bytes))) return rc;
-  for (int d = 0; d < nk; ++d) {
-    if (nocc[d] == 0) continue;
-    const int64_t cnt = int64_t(nocc[d]) * n;
-    hipLaunchKernelGGL(k_pack_orb<T>, dim3(unsigned(ceil_div(cnt, 256))), dim3(256), 0, c->stream,
-                       corb[d], nocc[d], n, ldc, off[size_t(d)], cb);
-  }
+  hipLaunchKernelGGL(k_pack_orb<T>, dim3(unsigned(ceil_div(cnt, 256))), dim3(256), 0, c->stream,
+                     orb_sets(nk, nocc, corb, off), c->n, c->n_pad, ldc, static_cast<T *>(buf.ptr));
   phase_end(c, MJK_PHASE_PACK);
-  return MJK_OK;
+  return hip_check(c, hipGetLastError(), "bank launch");
 }
 
 // FP32 copy of L, made once after the vectors change.
