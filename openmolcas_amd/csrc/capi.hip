@@ -7,6 +7,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 
 #include "mjk_internal.h"
 
@@ -151,6 +152,136 @@ void free_buf(DevBuf &b) {
 
 using namespace mjk;
 
+namespace {
+// Pinned host memory of the drop-ins' small transfers: one copy each way instead
+// of one per array (a copy from pageable memory costs 8-15 us of host time,
+// whatever its size).  A buffer is taken for one call and given back when its
+// copies are done; up to kPinnedKept idle ones are kept while any context lives.
+// Limit: above 3 MiB a direction the extra pass over host memory costs what the
+// saved copies gave (CHO_FSCF of 64 vectors, piecewise / staged: 158 / 103 us at
+// n = 131 with two densities, 0.2 MiB; 312 / 291 us at 2.2 MiB; 473 / 478 us at
+// 3.1 MiB; 932 / 992 us at 6.5 MiB).
+constexpr size_t kPinnedMost = size_t(3) << 20;
+constexpr size_t kPinnedLeast = size_t(64) << 10;
+constexpr int kPinnedKept = 4;
+struct Pinned { void *ptr = nullptr; size_t bytes = 0; };
+std::mutex pinned_mu;
+Pinned pinned_idle[kPinnedKept];  // unordered; ptr is null in a free place
+int64_t contexts_alive = 0;
+
+Pinned pinned_take(size_t bytes) {
+  {
+    std::lock_guard<std::mutex> lock(pinned_mu);
+    for (Pinned &i : pinned_idle)
+      if (i.ptr && i.bytes >= bytes) {
+        const Pinned p = i;
+        i = Pinned{};
+        return p;
+      }
+  }
+  Pinned p;
+  p.bytes = kPinnedLeast;
+  while (p.bytes < bytes) p.bytes *= 2;
+  p.bytes = std::min(p.bytes, kPinnedMost);
+  if (hipHostMalloc(&p.ptr, p.bytes, hipHostMallocPortable) != hipSuccess) {
+    (void)hipGetLastError();
+    return Pinned{};  // the copies go piece by piece
+  }
+  return p;
+}
+
+void pinned_give(Pinned p) {
+  {
+    std::lock_guard<std::mutex> lock(pinned_mu);
+    if (contexts_alive > 0) {  // into the place of the smallest; free places have 0 bytes
+      Pinned *s = pinned_idle;
+      for (Pinned &i : pinned_idle)
+        if (i.bytes < s->bytes) s = &i;
+      if (s->bytes < p.bytes) std::swap(*s, p);
+    }
+  }
+  if (p.ptr) (void)hipHostFree(p.ptr);
+}
+
+// +1 / -1 as a context is created / destroyed; the last one frees the idle buffers.
+void pinned_count(int by) {
+  Pinned drop[kPinnedKept];
+  {
+    std::lock_guard<std::mutex> lock(pinned_mu);
+    contexts_alive += by;
+    if (contexts_alive == 0) std::swap(drop, pinned_idle);
+  }
+  for (const Pinned &p : drop)
+    if (p.ptr) (void)hipHostFree(p.ptr);
+}
+
+// Host arrays of one drop-in call to and from consecutive device memory: put()
+// each input, send() once; after the work fetch() the results, which arrive with
+// finish() (the call's synchronisation).  Larger calls copy piece by piece, as
+// the arrays come.
+class HostCopies {
+ public:
+  HostCopies(mjk_context *c, size_t in, size_t out) : c_(c) {  // doubles each way
+    const size_t bytes = sizeof(double) * std::max(in, out);
+    if (bytes <= kPinnedMost) pin_ = pinned_take(bytes);
+    buf_ = static_cast<double *>(pin_.ptr);
+  }
+  ~HostCopies() {
+    if (!buf_) return;
+    if (busy_) (void)hipStreamSynchronize(c_->stream);  // an early return: the copies may be in flight
+    pinned_give(pin_);
+  }
+  int put(double *dst, const double *src, size_t cnt, const char *what) {
+    if (cnt == 0) return MJK_OK;
+    if (!buf_) return hip_check(c_, hipMemcpyAsync(dst, src, sizeof(double) * cnt, hipMemcpyHostToDevice, c_->stream), what);
+    if (!dev_) dev_ = dst;
+    std::memcpy(buf_ + (dst - dev_), src, sizeof(double) * cnt);
+    used_ = std::max(used_, size_t(dst - dev_) + cnt);
+    return MJK_OK;
+  }
+  int send(const char *what) {
+    if (!buf_ || used_ == 0) return MJK_OK;
+    busy_ = true;
+    return hip_check(c_, hipMemcpyAsync(dev_, buf_, sizeof(double) * used_, hipMemcpyHostToDevice, c_->stream), what);
+  }
+  int fetch(double *dst, const double *src, size_t cnt, const char *what) {
+    if (cnt == 0) return MJK_OK;
+    if (!buf_) return hip_check(c_, hipMemcpyAsync(dst, src, sizeof(double) * cnt, hipMemcpyDeviceToHost, c_->stream), what);
+    // a result that follows the one before it on the device joins its copy
+    if (nback_ == 0 || back_[nback_ - 1].src + back_[nback_ - 1].cnt != src) back_[nback_++] = {src, got_, 0};
+    back_[nback_ - 1].cnt += cnt;
+    out_[nout_++] = {dst, got_, cnt};
+    got_ += cnt;
+    return MJK_OK;
+  }
+  int finish(const char *what) {
+    int rc;
+    for (int i = 0; i < nback_; ++i) {
+      busy_ = true;
+      if ((rc = hip_check(c_, hipMemcpyAsync(buf_ + back_[i].at, back_[i].src, sizeof(double) * back_[i].cnt,
+                                             hipMemcpyDeviceToHost, c_->stream), what)))
+        return rc;
+    }
+    if ((rc = hip_check(c_, hipStreamSynchronize(c_->stream), what))) return rc;
+    busy_ = false;
+    for (int i = 0; i < nout_; ++i) std::memcpy(out_[i].dst, buf_ + out_[i].at, sizeof(double) * out_[i].cnt);
+    return MJK_OK;
+  }
+
+ private:
+  struct Copy { const double *src; size_t at, cnt; };
+  struct Out { double *dst; size_t at, cnt; };
+  mjk_context *c_;
+  Pinned pin_;
+  double *buf_ = nullptr, *dev_ = nullptr;
+  size_t used_ = 0, got_ = 0;
+  bool busy_ = false;
+  Copy back_[4];  // at most 4 results a call
+  Out out_[4];
+  int nback_ = 0, nout_ = 0;
+};
+}  // namespace
+
 // LK thresholds of the drop-ins, per density: the basic threshold of
 // Cho_LK_ScreeningThreshold (cho_lk_screeningthreshold.F90:34-39) and
 //   tau  = LKThr / max(1,nOcc_d) * dmpk  (/ MaxRed with Estimate)  (cho_lk_scf.F90:155-165)
@@ -293,6 +424,7 @@ int mjk_create(mjk_context **out, int32_t nbas, int64_t nchol) {
     delete c;
     return rc;
   }
+  pinned_count(1);
   *out = c;
   return MJK_OK;
 }
@@ -309,6 +441,7 @@ int mjk_destroy(mjk_context *c) {
   for (auto e : c->ev_pool) hipEventDestroy(e);
   if (c->own_stream) hipStreamDestroy(c->stream);
   delete c;
+  pinned_count(-1);
   return MJK_OK;
 }
 
@@ -788,26 +921,22 @@ int mjk_cho_fscf(mjk_context *c, int32_t nden, double *const *flt, const int32_t
       return set_error(c, MJK_ERR_ARG, "cho_fscf: null Porb(d)");
     tot += int64_t(nocc[d]) * c->n;
   }
-  // device scratch: D | J | K(nden) | F(nden) | orbitals
-  const size_t need = sizeof(double) * size_t(np * (2 + 2 * nden) + tot);
+  // device scratch: inputs D | F(nden) | orbitals, then J | K(nden)
+  const size_t in = size_t(np * (1 + nden) + tot), need = sizeof(double) * (in + size_t(np * (1 + nden)));
   int rc;
   if ((rc = ensure(c, c->w->misc, need))) return rc;
   double *dD = static_cast<double *>(c->w->misc.ptr);
-  double *dJ = dD + np, *dK = dJ + np, *dF = dK + nden * np, *dC = dF + nden * np;
+  double *dF = dD + np, *dC = dF + nden * np, *dJ = dD + in, *dK = dJ + np;
   const double *cptr[2] = {dC, dC + int64_t(nocc[0]) * c->n};
-  if ((rc = hip_check(c, hipMemcpyAsync(dD, dlt, sizeof(double) * np, hipMemcpyHostToDevice,
-                                        c->stream), "copy DLT")))
-    return rc;
+  HostCopies io(c, in, size_t(np * nden));
+  if ((rc = io.put(dD, dlt, size_t(np), "copy DLT"))) return rc;
   for (int d = 0; d < nden; ++d) {  // FLT(d) and Porb(d) are separate arrays
-    if ((rc = hip_check(c, hipMemcpyAsync(dF + d * np, flt[d], sizeof(double) * np,
-                                          hipMemcpyHostToDevice, c->stream), "copy FLT")))
-      return rc;
+    if ((rc = io.put(dF + d * np, flt[d], size_t(np), "copy FLT"))) return rc;
     if (nocc[d] > 0 &&
-        (rc = hip_check(c, hipMemcpyAsync(const_cast<double *>(cptr[d]), porb[d],
-                                          sizeof(double) * size_t(nocc[d]) * c->n,
-                                          hipMemcpyHostToDevice, c->stream), "copy Porb")))
+        (rc = io.put(const_cast<double *>(cptr[d]), porb[d], size_t(nocc[d]) * c->n, "copy Porb")))
       return rc;
   }
+  if ((rc = io.send("copy DLT, FLT, Porb"))) return rc;
   if (precision == MJK_PREC_FP64) {  // V pass inside the half-transform
     if ((rc = coulomb_exchange(c, dD, np, dJ, np, nden, nocc, cptr, dK, np, nullptr))) return rc;
   } else {
@@ -819,10 +948,8 @@ int mjk_cho_fscf(mjk_context *c, int32_t nden, double *const *flt, const int32_t
   const double fk[2] = {-exfac, -exfac};           // FactXI, cho_fscf.F90:65
   if ((rc = fock_update(c, nden, dF, np, dJ, np, jsrc, fj, dK, np, fk))) return rc;
   for (int d = 0; d < nden; ++d)
-    if ((rc = hip_check(c, hipMemcpyAsync(flt[d], dF + d * np, sizeof(double) * np,
-                                          hipMemcpyDeviceToHost, c->stream), "copy FLT back")))
-      return rc;
-  return hip_check(c, hipStreamSynchronize(c->stream), "cho_fscf sync");
+    if ((rc = io.fetch(flt[d], dF + d * np, size_t(np), "copy FLT back"))) return rc;
+  return io.finish("cho_fscf sync");
 }
 
 int mjk_cho_fscf_sym(mjk_context *c, int32_t nsym, const int32_t *nbas, int32_t nden,
@@ -1024,24 +1151,19 @@ int mjk_cho_lk_scf(mjk_context *c, int32_t nden, double *const *flt, double *con
     for (int64_t k = 0; k < nocc[d]; ++k)
       for (int64_t b = 0; b < n; ++b)
         corb[size_t(o0 + k + nocc[d] * b)] = porb[d][b + n * k];
-  // device scratch: D | J | K(nden) | F(nden) | orbitals
-  const size_t need = sizeof(double) * size_t(np * (2 + 2 * nden) + tot);
+  // device scratch: inputs D | F(nden) | orbitals, then K(nden) | J
+  const size_t in = size_t(np * (1 + nden) + tot), need = sizeof(double) * (in + size_t(np * (1 + nden)));
   int rc;
   if ((rc = ensure(c, c->w->misc, need))) return rc;
   double *dD = static_cast<double *>(c->w->misc.ptr);
-  double *dJ = dD + np, *dK = dJ + np, *dF = dK + nden * np, *dC = dF + nden * np;
-  if ((rc = hip_check(c, hipMemcpyAsync(dD, plt, sizeof(double) * np, hipMemcpyHostToDevice,
-                                        c->stream), "copy PLT")))
-    return rc;
-  for (int d = 0; d < nden; ++d)
-    if ((rc = hip_check(c, hipMemcpyAsync(dF + d * np, flt[d], sizeof(double) * np,
-                                          hipMemcpyHostToDevice, c->stream), "copy FLT")))
-      return rc;
-  if (tot > 0 && (rc = hip_check(c, hipMemcpyAsync(dC, corb.data(), sizeof(double) * tot,
-                                                   hipMemcpyHostToDevice, c->stream),
-                                 "copy Porb")))
-    return rc;
+  double *dF = dD + np, *dC = dF + nden * np, *dK = dD + in, *dJ = dK + nden * np;
   const double *cptr[2] = {dC, dC + int64_t(nocc[0]) * n};
+  std::vector<double> kh;  // K on the host; outlives the copies into it
+  HostCopies io(c, in, size_t(np * nden) * (klt ? 2 : 1));
+  if ((rc = io.put(dD, plt, size_t(np), "copy PLT"))) return rc;
+  for (int d = 0; d < nden; ++d)
+    if ((rc = io.put(dF + d * np, flt[d], size_t(np), "copy FLT"))) return rc;
+  if ((rc = io.put(dC, corb.data(), size_t(tot), "copy Porb")) || (rc = io.send("copy PLT, FLT, Porb"))) return rc;
   if (c->lk_on) {  // the reference's LK screening, FP64
     if (precision != MJK_PREC_FP64)
       return set_error(c, MJK_ERR_ARG, "cho_lk_scf: LK screening computes in FP64 only");
@@ -1062,17 +1184,12 @@ int mjk_cho_lk_scf(mjk_context *c, int32_t nden, double *const *flt, double *con
   const double fk[2] = {-factxi, -factxi};       // -FactXI, cho_lk_scf.F90:803,830
   if ((rc = fock_update(c, nden, dF, np, dJ, np, jsrc, fj, dK, np, fk))) return rc;
   for (int d = 0; d < nden; ++d)
-    if ((rc = hip_check(c, hipMemcpyAsync(flt[d], dF + d * np, sizeof(double) * np,
-                                          hipMemcpyDeviceToHost, c->stream), "copy FLT back")))
-      return rc;
-  std::vector<double> kh;
+    if ((rc = io.fetch(flt[d], dF + d * np, size_t(np), "copy FLT back"))) return rc;
   if (klt) {
     kh.resize(static_cast<size_t>(np * nden));
-    if ((rc = hip_check(c, hipMemcpyAsync(kh.data(), dK, sizeof(double) * np * nden,
-                                          hipMemcpyDeviceToHost, c->stream), "copy K back")))
-      return rc;
+    if ((rc = io.fetch(kh.data(), dK, size_t(np * nden), "copy K back"))) return rc;
   }
-  if ((rc = hip_check(c, hipStreamSynchronize(c->stream), "cho_lk_scf sync"))) return rc;
+  if ((rc = io.finish("cho_lk_scf sync"))) return rc;
   if (klt)
     for (int d = 0; d < nden; ++d)
       for (int64_t p = 0; p < np; ++p)
@@ -1088,17 +1205,14 @@ int mjk_cho_fock_dft_red(mjk_context *c, const double *dlt, double *flt) {
   if ((rc = ensure(c, c->w->misc, sizeof(double) * size_t(2 * np)))) return rc;
   double *dD = static_cast<double *>(c->w->misc.ptr);
   double *dJ = dD + np;
-  if ((rc = hip_check(c, hipMemcpyAsync(dD, dlt, sizeof(double) * np, hipMemcpyHostToDevice,
-                                        c->stream), "copy DLT")))
-    return rc;
+  HostCopies io(c, size_t(np), size_t(np));
+  if ((rc = io.put(dD, dlt, size_t(np), "copy DLT")) || (rc = io.send("copy DLT"))) return rc;
   if ((rc = coulomb(c, 1, dD, np, dJ, np, nullptr))) return rc;
   // FLT is written, not accumulated: the first reduced set's swap_rs2full
   // (add = .false., cho_fock_dft_red.F90:190-191) zeroes all of FLT
   // (swap_rs2full.F90:37-41) and later sets add to it.
-  if ((rc = hip_check(c, hipMemcpyAsync(flt, dJ, sizeof(double) * np, hipMemcpyDeviceToHost,
-                                        c->stream), "copy FLT back")))
-    return rc;
-  return hip_check(c, hipStreamSynchronize(c->stream), "cho_fock_dft_red sync");
+  if ((rc = io.fetch(flt, dJ, size_t(np), "copy FLT back"))) return rc;
+  return io.finish("cho_fock_dft_red sync");
 }
 
 }  // extern "C"
@@ -1129,24 +1243,28 @@ static int fmcscf_core(mjk_context *c, double *const *flt, int32_t nforb, int32_
     return set_error(c, MJK_ERR_ARG, "cho_fmcscf: bad (pw|xy) arguments");
   const int64_t nxy = int64_t(naorb) * (naorb + 1) / 2;
   const int64_t nw = do_puvx ? int64_t(norb) * naorb * nxy : 0;
-  const size_t need = sizeof(double) * size_t(np * 4 * nden + (nk1 + nk2) * n +
-                                              (do_puvx ? naorb * n + n * n + nw : 0));
+  // device scratch: inputs D(nden) | POrb(1..3) | CMO | F(nden), then W (after F:
+  // results come back in one copy) | J(nden) | K(nden)
+  const size_t in = size_t(2 * nden * np + (nk1 + nk2) * n + (do_puvx ? naorb * n + n * n : 0));
+  const size_t need = sizeof(double) * (in + size_t(nw + 2 * nden * np));
   int rc;
   if ((rc = ensure(c, c->w->misc, need))) return rc;
   double *dD = static_cast<double *>(c->w->misc.ptr);
-  double *dJ = dD + nden * np, *dK = dJ + nden * np, *dF = dK + nden * np, *dC1 = dF + nden * np;
-  double *dC2 = dC1 + int64_t(nk1) * n, *dC3 = dC2 + int64_t(nk2) * n;
-  double *dCMO = dC3 + (do_puvx ? int64_t(naorb) * n : 0), *dW = dCMO + (do_puvx ? n * n : 0);
-  auto h2d = [&](void *dst, const void *src, size_t cnt, const char *what) {
-    return hip_check(c, hipMemcpyAsync(dst, src, sizeof(double) * cnt, hipMemcpyHostToDevice,
-                                       c->stream), what);
-  };
+  double *dC1 = dD + nden * np, *dC2 = dC1 + int64_t(nk1) * n, *dC3 = dC2 + int64_t(nk2) * n;
+  double *dCMO = dC3 + (do_puvx ? int64_t(naorb) * n : 0), *dF = dCMO + (do_puvx ? n * n : 0);
+  double *dW = dD + in, *dJ = dW + nw, *dK = dJ + nden * np;
+  HostCopies io(c, in, size_t(nden * np + nw));
   for (int d = 0; d < nden; ++d)  // FI/FA and DI/DA are separate arrays
-    if ((rc = h2d(dD + d * np, dlt[d], size_t(np), "copy DLT")) ||
-        (rc = h2d(dF + d * np, flt[d], size_t(np), "copy FLT")))
+    if ((rc = io.put(dD + d * np, dlt[d], size_t(np), "copy DLT")) ||
+        (rc = io.put(dF + d * np, flt[d], size_t(np), "copy FLT")))
       return rc;
-  if (nk1 > 0 && (rc = h2d(dC1, porb1, size_t(nk1 * n), "copy POrb(1)"))) return rc;
-  if (nk2 > 0 && (rc = h2d(dC2, porb2, size_t(nk2 * n), "copy POrb(2)"))) return rc;
+  if ((rc = io.put(dC1, porb1, size_t(nk1 * n), "copy POrb(1)")) ||
+      (rc = io.put(dC2, porb2, size_t(nk2 * n), "copy POrb(2)")))
+    return rc;
+  if (do_puvx && ((rc = io.put(dC3, porb3, size_t(naorb * n), "copy POrb(3)")) ||
+                  (rc = io.put(dCMO, cmo, size_t(n * n), "copy CMO"))))
+    return rc;
+  if ((rc = io.send("copy DLT, FLT, POrb, CMO"))) return rc;
   if ((rc = coulomb(c, nden, dD, np, dJ, np, nullptr))) return rc;
   const int32_t nocc[2] = {nk1, nk2};
   const double *cptr[2] = {dC1, dC2};
@@ -1161,20 +1279,11 @@ static int fmcscf_core(mjk_context *c, double *const *flt, int32_t nforb, int32_
   const double fj[2] = {1.0, 1.0};        // FactCI, FactCA (cho_fmcscf.F90:71)
   const double fk[2] = {fk_i, fk_a};      // FactXI, FactXA
   if ((rc = fock_update(c, nden, dF, np, dJ, np, jsrc, fj, dK, np, fk))) return rc;
-  if (do_puvx) {
-    if ((rc = h2d(dC3, porb3, size_t(naorb * n), "copy POrb(3)")) ||
-        (rc = h2d(dCMO, cmo, size_t(n * n), "copy CMO")))
-      return rc;
-    if ((rc = mjk_puvx(c, naorb, dC3, dCMO, nfro, norb, dW))) return rc;
-    if ((rc = hip_check(c, hipMemcpyAsync(w_pwxy, dW, sizeof(double) * nw,
-                                          hipMemcpyDeviceToHost, c->stream), "copy W_PWXY")))
-      return rc;
-  }
+  if (do_puvx && (rc = mjk_puvx(c, naorb, dC3, dCMO, nfro, norb, dW))) return rc;
   for (int d = 0; d < nden; ++d)
-    if ((rc = hip_check(c, hipMemcpyAsync(flt[d], dF + d * np, sizeof(double) * np,
-                                          hipMemcpyDeviceToHost, c->stream), "copy FLT back")))
-      return rc;
-  return hip_check(c, hipStreamSynchronize(c->stream), "cho_fmcscf sync");
+    if ((rc = io.fetch(flt[d], dF + d * np, size_t(np), "copy FLT back"))) return rc;
+  if (do_puvx && (rc = io.fetch(w_pwxy, dW, size_t(nw), "copy W_PWXY"))) return rc;
+  return io.finish("cho_fmcscf sync");
 }
 
 namespace {
