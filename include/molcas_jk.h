@@ -93,6 +93,12 @@ int mjk_device_vectors(mjk_context *ctx, double **L, int64_t *ldl);
  * half-transform AO tile (0, 64, 128). */
 int mjk_set_tuning(mjk_context *ctx, int32_t tile_syrk, int32_t split_target, int32_t ht_ta);
 
+/* One-pass Coulomb build: how often a workgroup looks whether the others of its
+ * group have started before the group does without them (default 64, about 1 us
+ * each; 0: at once).  The results are the same bits whatever the value; it bounds
+ * the wait when other streams hold the GPU. */
+int mjk_set_coulomb_looks(mjk_context *ctx, int32_t looks);
+
 /* Times every exchange tiling for these orbital sets and keeps the fastest
  * in the context (best time in *best_ms); klt receives the last K. */
 int mjk_autotune(mjk_context *ctx, int32_t nk, const int32_t *nocc, const double *const *corb,

@@ -4,9 +4,10 @@
 // cho_lk_scf.F90:442-449, cho_fmcscf.F90:261-285):
 //   V_J  = sum_p L^J_p D_p          (D folded: off-diagonal doubled)
 //   J_p  = sum_J L^J_p V_J
-// Both passes stream L once; they are HBM-bound.  L is stored vector-major
+// Bound by HBM.  One or two densities of ordinary sizes read L once for both
+// (k_coulomb_one); otherwise each pass streams L once.  L is stored vector-major
 // (row J holds the packed LT of L^J, stride ldl, a multiple of 512 doubles),
-// so each pass reads whole 4 KiB row segments per workgroup iteration.
+// so whole 4 KiB row segments are read per workgroup iteration.
 #include <mutex>
 #include <string>
 
@@ -177,12 +178,309 @@ __global__ __launch_bounds__(kThreads) void k_reduce_j(const double *__restrict_
   if (q == 0 && p < np) jlt[d * ldj + p] = ((s + red[0][cb]) + red[1][cb]) + red[2][cb];
 }
 
+// ---- one or two densities: both passes in one read of the vectors ----------
+// A group of G workgroups holds one vector at a time in registers, each its slice
+// of the pairs: a workgroup sums its part of V_J, publishes it, and adds V_J L^J to
+// its J once the whole V_J is there.  Its ring of four vectors hides the exchange:
+// while V_J is awaited the next is contracted and the one after is on its way.
+// Bound by HBM (one read of L) once a group has its 48 KiB per step in flight.
+// Measured against the two passes (two reads), us: n=701, 2804 vectors 1735 -> 946
+// (5.8 TB/s), n=512 715 -> 385, n=301 164 -> 96, n=1200 8634 -> 4635; two densities
+// n=701 1761 -> 1134, n=301 172 -> 106.  Rows and ring (rows x vectors of lag):
+// one density, n=512: 8x0 457, 6x1 385, 6x2 387, 5x2 411, 4x3 451 us; two, n=512:
+// 6x0 468, 5x1 440, 4x2 488 us.
+constexpr int kOneWaves = 8, kOneRow = 2 * kWave * kOneWaves;  // streaming waves; doubles per workgroup row
+constexpr int kOneRing = 4;                                    // vectors per workgroup: on its way, contracted, awaited
+constexpr int64_t kOneEmpty = 0x7ff4a5c300f1d2e7;              // "not there yet" (a NaN) in the exchange array
+
+template <int C>
+__device__ inline double dpp_add(double x) {
+  const int2 v = __builtin_bit_cast(int2, x);
+  const int2 y = {__builtin_amdgcn_update_dpp(0, v.x, C, 0xf, 0xf, false),
+                  __builtin_amdgcn_update_dpp(0, v.y, C, 0xf, 0xf, false)};
+  return x + __builtin_bit_cast(double, y);
+}
+
+__device__ inline double lane_value(double x, int lane) {
+  const int2 v = __builtin_bit_cast(int2, x);
+  return __builtin_bit_cast(double, int2{__builtin_amdgcn_readlane(v.x, lane), __builtin_amdgcn_readlane(v.y, lane)});
+}
+
+// Sum over the wave, the same in every lane.
+__device__ inline double wave_sum(double x) {
+  x = dpp_add<0xB1>(x);   // lane ^ 1
+  x = dpp_add<0x4E>(x);   // lane ^ 2
+  x = dpp_add<0x141>(x);  // the other quad of eight lanes
+  x = dpp_add<0x140>(x);  // the other eight of sixteen
+  return (lane_value(x, 0) + lane_value(x, 16)) + (lane_value(x, 32) + lane_value(x, 48));
+}
+
+// LDS written before is seen after; loads from memory stay in flight across it.
+__device__ inline void lds_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// Part of V of one vector that a wave sums: each lane's pairs in rising order, then
+// the wave.
+template <int ROWS>
+__device__ inline double one_dot(const v2d (&x)[ROWS], const v2d *sD, int t) {
+  double a = 0.0;
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    const v2d d = sD[i * (kOneWaves * kWave) + t];
+    a = __builtin_fma(x[i].x, d.x, a);
+    a = __builtin_fma(x[i].y, d.y, a);
+    if (i & 1) asm volatile("" : "+v"(a) : : "memory");  // two rows of D in registers, not all
+  }
+  return wave_sum(a);
+}
+
+// What rows past the end of a slice, and steps past the last vector, read.
+__device__ const v2d one_zeros[kWave] = {};
+
+__device__ inline double sum_waves(const double *s) {
+  return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+}
+
+// Rows of a slice of len doubles that belong to wave w.
+__device__ inline int one_rows(int64_t len, int w) {
+  const int64_t left = len - 2 * kWave * w;
+  return left <= 0 ? 0 : int((left + kOneRow - 1) / kOneRow);
+}
+
+// How the members of a group meet, one per group, zero at the start.
+struct OneGate {
+  int arrived;  // members that have started; kOneApart set: the group works apart
+  int parts, done, sums;  // apart: slices whose parts were begun, ended; slices begun for J
+};
+constexpr int kOneApart = 1 << 30;
+
+// Whether all G members of a group run at the same time, the same answer for each: a
+// member waits for the others for `looks` looks (about 1 us each).
+__device__ inline bool one_together(OneGate *g, int G, int looks) {
+  int v = __hip_atomic_fetch_add(&g->arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+  for (int left = looks;; --left) {
+    if (v & kOneApart) return false;
+    if (v == G) return true;
+    if (left <= 0 && __hip_atomic_compare_exchange_strong(&g->arrived, &v, v | kOneApart, __ATOMIC_RELAXED,
+                                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      return false;
+    __builtin_amdgcn_s_sleep(1);
+    v = __hip_atomic_load(&g->arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+__device__ inline int one_take(int *n) {
+  return __hip_atomic_fetch_add(n, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// grid = ngrp * G; workgroup b belongs to group b / G (workgroups start in this order:
+// with part of the GPU free the first groups are whole).  Group g takes vectors g,
+// g + ngrp, ...  Slice m is pairs [m * slice, (m+1) * slice), slice a multiple of 128
+// and at most ROWS rows of 1024.  D: padded densities (stride ldl).
+// part[(J * G + m) * ND + d]: the exchange, all kOneEmpty at the start (unused for
+// G = 1; G * ND <= 256).
+//
+// Waiting for another member is safe only while it runs, and other streams may hold
+// part of the GPU.  A group whose members have not all started after `looks` looks
+// works apart: whoever of it runs takes slices and sums their parts of every V_J
+// (nothing is waited for), then, all parts being there, takes slices again for J.
+// That is two reads of the vectors, with any number of members, and the same bits.
+// Contexts at once on streams of their own, us, two-pass kernels -> this one: n=301,
+// 1200 vectors, J on four 572 -> 516, J and K on four 2186 -> 1629; n=701, 700 vectors
+// J on two 853 -> 626, on four 1754 -> 1881, J and K on four 9552 -> 7925.  With 4096
+// looks 4 x J at n=900 took 23000; 16 or 8 looks: +2 to +11% at n=301, none gained.
+template <int ND, int ROWS>
+__global__ __launch_bounds__((kOneWaves + 1) * kWave) void k_coulomb_one(
+    const double *__restrict__ L, int64_t ldl, int64_t M, const double *__restrict__ D, int ngrp, int G, int64_t slice,
+    int looks, OneGate *gate, double *part, double *__restrict__ V, double *__restrict__ jpart) {
+  constexpr int R = kOneRing, LAG = R - 3;
+  __shared__ __attribute__((aligned(16))) v2d sD[ND][ROWS * kOneWaves * kWave];
+  __shared__ double sP[R][ND][kOneWaves];
+  __shared__ double sV[2][ND];
+  __shared__ int sTask;  // slice to work on next; < 0: none
+  enum { kTogether, kParts, kSums };
+  const int lane = threadIdx.x & (kWave - 1), w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int grp = blockIdx.x / G;
+  const int T = int((M - grp + ngrp - 1) / ngrp);
+  const int steps = (T + LAG + R - 1) / R * R;
+  int mem = blockIdx.x % G, mode = kTogether;
+
+  for (;;) {
+    const int64_t p0 = min(mem * slice, ldl), len = min(slice, ldl - p0);
+    if (w == kOneWaves) {  // ---- the wave that exchanges V
+      if (mode == kTogether) {
+        const bool one = G == 1 || __builtin_amdgcn_readfirstlane(lane == 0 ? one_together(gate + grp, G, looks) : 0);
+        if (lane == 0) sTask = one ? mem : -1;
+      }
+      lds_barrier();  // D is there
+      lds_barrier();  // parts of the first vector
+      if (mode != kTogether || __builtin_amdgcn_readfirstlane(sTask) >= 0) {
+        for (int s = 0; s < steps; ++s) {
+          double v[ND];
+          if (G > 1 && s < T && lane < ND) {
+            double mine = sum_waves(sP[s % R][lane]);
+            if (__builtin_bit_cast(int64_t, mine) == kOneEmpty) mine = __builtin_nan("");
+            __hip_atomic_store(part + (grp + int64_t(s) * ngrp) * G * ND + mem * ND + lane, mine, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+          }
+          const int64_t J = grp + int64_t(s - LAG) * ngrp;
+          const bool have = mode != kParts && s >= LAG && s - LAG < T;
+#pragma unroll
+          for (int d = 0; d < ND; ++d) v[d] = 0.0;
+          if (have && G == 1) {
+#pragma unroll
+            for (int d = 0; d < ND; ++d) v[d] = sum_waves(sP[(s - LAG) % R][d]);
+          }
+          if (have && G > 1) {
+            const double *row = part + J * G * ND;
+            const int cnt = G * ND;  // <= 256
+            double x[4];
+            for (;;) {  // the others run: their parts come
+              bool ok = true;
+              auto look = [&](int k) {
+                return __hip_atomic_load(row + min(lane + 64 * k, cnt - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              };
+              x[0] = look(0);
+              x[1] = x[2] = x[3] = 0.0;
+              if (cnt > 128) {
+                x[1] = look(1), x[2] = look(2), x[3] = look(3);
+              } else if (cnt > 64) {
+                x[1] = look(1);
+              }
+#pragma unroll
+              for (int k = 0; k < 4; ++k) {
+                ok = ok && __builtin_bit_cast(int64_t, x[k]) != kOneEmpty;
+                if (lane + 64 * k >= cnt) x[k] = 0.0;
+              }
+              if (__all(ok)) break;
+              __builtin_amdgcn_s_sleep(1);
+            }
+            const double y = (x[0] + x[1]) + (x[2] + x[3]);
+            if constexpr (ND == 1) {
+              v[0] = wave_sum(y);
+            } else {  // entry 2m + d: even lanes density 0, odd lanes density 1
+              v[0] = wave_sum(lane & 1 ? 0.0 : y);
+              v[1] = wave_sum(lane & 1 ? y : 0.0);
+            }
+          }
+          if (lane == 0) {
+#pragma unroll
+            for (int d = 0; d < ND; ++d) sV[s & 1][d] = v[d];
+            if (mem == 0 && have) {
+#pragma unroll
+              for (int d = 0; d < ND; ++d) V[J * ND + d] = v[d];
+            }
+          }
+          lds_barrier();
+        }
+      }
+    } else {  // ---- the streaming waves
+      const int t = threadIdx.x;
+      const int nv = __builtin_amdgcn_readfirstlane(one_rows(len, w));
+      using Row = const __attribute__((address_space(1))) v2d *;
+      v2d buf[R][ROWS], acc[ND][ROWS];
+      auto fetch = [&](int s, v2d(&x)[ROWS]) {
+        const uint64_t row = reinterpret_cast<uint64_t>(L + (grp + int64_t(s) * ngrp) * ldl + p0 + 2 * kWave * w);
+        const int have = s < T ? nv : 0;
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i)
+          x[i] = __builtin_nontemporal_load(
+              reinterpret_cast<Row>(i < have ? row + i * (kOneRow * sizeof(double)) : reinterpret_cast<uint64_t>(one_zeros)) + lane);
+      };
+#pragma unroll
+      for (int r = 0; r < R; ++r) fetch(r < 2 ? r : T, buf[r]);
+#pragma unroll
+      for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) {
+          sD[d][i * (kOneWaves * kWave) + t] =
+              reinterpret_cast<Row>(i < nv ? reinterpret_cast<uint64_t>(D + d * ldl + p0 + i * kOneRow + 2 * kWave * w)
+                                           : reinterpret_cast<uint64_t>(one_zeros))[lane];
+          acc[d][i] = v2d{0.0, 0.0};
+        }
+      lds_barrier();
+      auto parts = [&](int s, const v2d(&x)[ROWS]) {
+#pragma unroll
+        for (int d = 0; d < ND; ++d) sP[s % R][d][w] = one_dot<ROWS>(x, sD[d], t);  // the same in every lane
+      };
+      parts(0, buf[0]);
+      lds_barrier();
+      // step s: vector s + 2 on its way, parts of s + 1, V of s - LAG
+      auto step = [&](int s, v2d(&cur)[ROWS], v2d(&nxt)[ROWS], v2d(&far)[ROWS]) {
+        __builtin_amdgcn_sched_barrier(0);  // `far` has been used before it is loaded again
+        fetch(s + 2, far);
+        __builtin_amdgcn_sched_barrier(0);
+        parts(s + 1, nxt);
+        lds_barrier();
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+          const double v = sV[s & 1][d];
+#pragma unroll
+          for (int i = 0; i < ROWS; ++i) {
+            acc[d][i].x = __builtin_fma(cur[i].x, v, acc[d][i].x);
+            acc[d][i].y = __builtin_fma(cur[i].y, v, acc[d][i].y);
+            asm volatile("" : "+v"(acc[d][i]));  // summed here, not where it is next read
+          }
+        }
+      };
+      if (mode != kTogether || __builtin_amdgcn_readfirstlane(sTask) >= 0) {
+        for (int s = 0; s < steps; s += R) {  // steps of zeros at both ends
+#pragma unroll
+          for (int u = 0; u < R; ++u) step(s + u, buf[(u + 3) % R], buf[(u + 1) % R], buf[(u + 2) % R]);
+        }
+        if (mode != kParts) {
+#pragma unroll
+          for (int d = 0; d < ND; ++d)
+#pragma unroll
+            for (int i = 0; i < ROWS; ++i)
+              if (i < nv)
+                *reinterpret_cast<v2d *>(jpart + (int64_t(grp) * ND + d) * ldl + p0 + i * kOneRow + 2 * t) = acc[d][i];
+        }
+      }
+    }
+    // ---- apart: the next slice
+    if (mode == kTogether && __builtin_amdgcn_readfirstlane(sTask) >= 0) return;
+    lds_barrier();  // everybody has read sTask
+    if (w == kOneWaves) {
+      int next = -1, m = mode;
+      if (lane == 0) {
+        OneGate *g = gate + grp;
+        if (m == kParts) one_take(&g->done);
+        if (m != kSums) {
+          m = kParts;
+          next = one_take(&g->parts);
+          if (next >= G) {
+            // slices not done are being worked on, and nothing is waited for there
+            while (__hip_atomic_load(&g->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < G) __builtin_amdgcn_s_sleep(8);
+            m = kSums;
+          }
+        }
+        if (m == kSums) next = one_take(&g->sums);
+        sTask = next < G ? next * 4 + m : -1;
+      }
+    }
+    lds_barrier();
+    const int task = __builtin_amdgcn_readfirstlane(sTask);
+    if (task < 0) return;
+    mem = task >> 2;
+    mode = task & 3;
+    lds_barrier();  // everybody has read sTask
+  }
+}
+
 // Copies nd densities of stride ldd into the zero-padded staging buffer of
-// stride ldl.
+// stride ldl; on the way nempty elements of `part` become kOneEmpty and nzero
+// after them 0.
 __global__ void k_pack_dens(const double *__restrict__ dlt, int64_t ldd, int64_t np,
-                            int64_t ldl, double *__restrict__ out) {
+                            int64_t ldl, double *__restrict__ out, int64_t *__restrict__ part, int64_t nempty,
+                            int64_t nzero) {
   const int64_t p = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   const int d = blockIdx.y;
+  const int64_t threads = int64_t(gridDim.x) * blockDim.x;
+  for (int64_t i = p + d * threads; i < nempty + nzero; i += threads * gridDim.y) part[i] = i < nempty ? kOneEmpty : 0;
   if (p >= ldl) return;
   out[d * ldl + p] = (p < np) ? dlt[d * ldd + p] : 0.0;
 }
@@ -400,6 +698,8 @@ namespace {
 struct CoulombPlan {
   int nd = 0, ndt = 0;
   bool tile = false;                   // nd >= 3: the MFMA passes
+  int group = 0, ngrp = 0;             // one pass: workgroups per group, groups (0: two passes)
+  int64_t slice = 0, nparts = 0;       // one pass: pairs per workgroup; parts of V to exchange
   int nsplit1 = 0, nsplit2 = 0;
   int64_t nblk = 0, pchunk = 0, jchunk = 0;
   size_t bytes_d = 0, bytes_vpart = 0, bytes_v = 0, bytes_jpart = 0;
@@ -421,12 +721,42 @@ void plan_j_stream(const Context *c, int nd, int ndt, CoulombPlan *p) {
   p->bytes_jpart = sizeof(double) * size_t(p->nsplit2) * nd * c->ldl;
 }
 
+// Rows of 1024 pairs per workgroup of the one-pass kernel (register budget: four
+// vectors and the J of each density, three waves per SIMD).
+constexpr int one_rows_max(int nd) { return nd == 1 ? 6 : 5; }
+constexpr int kOneGrid = 256;  // workgroups: one per CU
+
+// The one-pass kernel takes one or two densities from 8192 pairs on (n = 131, 524
+// vectors: 34 us, 38 in two passes; n = 110: 36 against 31, the members' meeting is not
+// hidden) up to 786432, so that there are two groups (n = 1200: 4970 against 8630 us;
+// n = 1300, 200 vectors, one group: 403 against 474 alone but 1006 against 889 on two
+// streams).  Groups: as many as fit, with at least eight vectors each, below which
+// their J costs more to write and reduce than the wait for V (n = 130: 33.8 us with
+// two each, 29.8 with eight), but up to 32 when vectors are few (n = 500, 16 vectors:
+// 36 us in two groups, 28 in eight).
+bool plan_one(const Context *c, int nd, CoulombPlan *p) {
+  const int64_t M = c->nchol, ldl = c->ldl;
+  if (nd > 2 || ldl < 8192) return false;
+  const int64_t gmin = ceil_div(ldl, kOneRow * one_rows_max(nd));
+  if (gmin > kOneGrid / 2 || gmin * nd > 256) return false;
+  const int64_t want = std::max<int64_t>({M / 8, std::min<int64_t>(M / 2, 32), 1});
+  p->ngrp = int(std::min<int64_t>(kOneGrid / gmin, want));
+  p->slice = round_up(ceil_div(ldl, std::min<int64_t>(kOneGrid / p->ngrp, 256 / nd)), 2 * kWave);
+  p->group = int(ceil_div(ldl, p->slice));
+  p->nsplit2 = p->ngrp;
+  p->nparts = p->group > 1 ? M * p->group * nd : 0;
+  p->bytes_vpart = sizeof(double) * size_t(p->nparts) + sizeof(OneGate) * size_t(p->ngrp);
+  p->bytes_jpart = sizeof(double) * size_t(p->ngrp) * nd * ldl;
+  return true;
+}
+
 CoulombPlan plan_coulomb(const Context *c, int nd) {
   CoulombPlan p;
   const int64_t M = c->nchol, ldl = c->ldl;
   p.nd = nd;
   p.bytes_d = sizeof(double) * size_t(nd) * ldl;
   p.bytes_v = sizeof(double) * size_t(M) * nd;
+  if (plan_one(c, nd, &p)) return p;
   if (nd >= 3) {
     p.tile = true;
     p.nblk = ceil_div(M, kTileVM);
@@ -516,8 +846,29 @@ int coulomb_run(Context *c, Scratch &s, int32_t nd, const double *dlt, int64_t l
   else if ((rc = take(c, s, c->w->v, p.bytes_v, &V))) return rc;
   phase_begin(c);
   hipLaunchKernelGGL(k_pack_dens, dim3(unsigned(ceil_div(ldl, 256)), unsigned(nd)), dim3(256), 0,
-                     c->stream, dlt, ldd, c->np, ldl, Dp);
+                     c->stream, dlt, ldd, c->np, ldl, Dp, reinterpret_cast<int64_t *>(vpart),
+                     p.nparts, p.group > 1 ? int64_t(sizeof(OneGate) / 8) * p.ngrp : 0);
   phase_end(c, MJK_PHASE_PACK);
+
+  if (p.group) {
+    double *jpart;
+    if ((rc = take(c, s, c->w->jpart, p.bytes_jpart, &jpart))) return rc;
+    phase_begin(c);
+    const dim3 grid(unsigned(p.ngrp * p.group)), block((kOneWaves + 1) * kWave);
+    OneGate *gate = reinterpret_cast<OneGate *>(vpart + p.nparts);
+    if (nd == 1)
+      hipLaunchKernelGGL((k_coulomb_one<1, one_rows_max(1)>), grid, block, 0, c->stream, c->L, ldl, M, Dp, p.ngrp,
+                         p.group, p.slice, c->coulomb_looks, gate, vpart, V, jpart);
+    else
+      hipLaunchKernelGGL((k_coulomb_one<2, one_rows_max(2)>), grid, block, 0, c->stream, c->L, ldl, M, Dp, p.ngrp,
+                         p.group, p.slice, c->coulomb_looks, gate, vpart, V, jpart);
+    phase_end(c, MJK_PHASE_COULOMB_J);
+    phase_begin(c);
+    hipLaunchKernelGGL(k_reduce_j, dim3(unsigned(ceil_div(c->np, 64)), unsigned(nd)), dim3(256), 0, c->stream, jpart,
+                       ldl, c->np, nd, p.ngrp, jlt, ldj);
+    phase_end(c, MJK_PHASE_REDUCE);
+    return hip_check(c, hipGetLastError(), "coulomb launch");
+  }
 
   if (p.tile) {
     // ---- pass 1: V = L D^T, split over pairs to fill the device

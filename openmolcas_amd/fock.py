@@ -685,6 +685,12 @@ class JKContext:
         self._resident = ("device", t.data_ptr())
         return t
 
+    def set_coulomb_looks(self, looks: int = 64) -> None:
+        """How often a workgroup of the one-pass Coulomb build looks whether the others
+        of its group have started before the group does without them; the results do
+        not depend on it."""
+        self._check(self.lib.mjk_set_coulomb_looks(self._h, int(looks)))
+
     def set_tuning(self, tile_syrk: int = 0, split_target: int = 0, ht_ta: int = 0) -> None:
         self._check(self.lib.mjk_set_tuning(self._h, int(tile_syrk), int(split_target), int(ht_ta)))
 
