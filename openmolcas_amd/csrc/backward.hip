@@ -980,7 +980,7 @@ extern "C" int mjk_grad_vectors(mjk_context *c, int32_t nocc, const double *corb
   for (int64_t ch = 0; ch < nchunk; ++ch) {
     const int64_t j0 = ch * jc, jn = std::min(jc, M - j0);
     phase_begin(c);
-    ht_launch(c, ot, cb, j0, jn, X);  // X[J][k][a] = (C^T L^J)[k][a]
+    ht_launch(c, tot, cb, j0, jn, X);  // X[J][k][a] = (C^T L^J)[k][a]
     phase_end(c, MJK_PHASE_HALF_TRANSFORM);
     phase_begin(c);
     GemmBatch g{};

@@ -390,23 +390,28 @@ __global__ __launch_bounds__(kThreads) void k_ht(
 // stood between the MFMAs).
 constexpr int kHtB = 16;       // contraction rows per chunk
 constexpr int kHtS = 17;       // row stride of a turned block
+constexpr int ht64_ldc(int ot, int tq) { return 16 * (ot + (tq > 0)); }  // bank columns
 
-template <int OT, int NBV, bool FV>
+template <int OT, int TQ, int NBV, bool FV>
 __device__ __forceinline__ void ht64_wave(const double *__restrict__ Lj, int n, int nch, int n_pad,
                                           const double *__restrict__ Cb, int a0, double *__restrict__ xj,
                                           const double *__restrict__ dens, double *__restrict__ vout,
-                                          double (*__restrict__ sC)[kHtB * 16 * OT], double *__restrict__ sT) {
-  constexpr int LDC = 16 * OT;
+                                          double (*__restrict__ sC)[kHtB * ht64_ldc(OT, TQ)], double *__restrict__ sT) {
+  constexpr int LDC = ht64_ldc(OT, TQ);
   constexpr int HP = OT / 2;                 // pairs of orbital tiles; an odd last tile stands alone
   constexpr int NB1 = NBV > 0 ? NBV : 1;
   constexpr int CN = kHtB * LDC / 2 / kThreads;  // 16-byte pieces of a bank chunk per thread ...
   constexpr int CR = kHtB * LDC / 2 % kThreads;  // ... and those of a last, partial round
   const int tid = threadIdx.x, lane = tid & 63, m = lane & 15, g = lane >> 4;
-  v4d acc[OT][NB1];
+  v4d acc[OT > 0 ? OT : 1][NB1];
+  double accq[TQ > 0 ? TQ : 1][NB1];
 #pragma unroll
-  for (int t = 0; t < OT; ++t)
+  for (int j = 0; j < NBV; ++j) {
 #pragma unroll
-    for (int j = 0; j < NBV; ++j) acc[t][j] = v4d{0.0, 0.0, 0.0, 0.0};
+    for (int t = 0; t < OT; ++t) acc[t][j] = v4d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < TQ; ++q) accq[q][j] = 0.0;
+  }
   double vp = 0.0;
   // bank chunk: global -> registers -> LDS, the layout unchanged
   v2d rc[CN + (CR ? 1 : 0)];
@@ -471,6 +476,14 @@ __device__ __forceinline__ void ht64_wave(const double *__restrict__ Lj, int n, 
   auto load_co = [&](int buf, int s) __attribute__((always_inline)) {
     if constexpr (OT % 2 == 1) co = sC[buf][(4 * g + s) * LDC + 16 * (OT - 1) + m];
   };
+  v2d cq = {0.0, 0.0};  // quarter tiles 0 and 1 take alternate columns
+  double ct = 0.0;
+  auto load_cq = [&](int buf, int s) __attribute__((always_inline)) {
+    const double *__restrict__ row = &sC[buf][(4 * g + s) * LDC + 16 * OT];
+    if constexpr (TQ == 1) cq[0] = row[m & 3];
+    if constexpr (TQ >= 2) cq = *reinterpret_cast<const v2d *>(row + 2 * (m & 3));
+    if constexpr (TQ == 3) ct = row[8 + (m & 3)];
+  };
   auto step = [&](int buf, int s, const double(&x)[NB1]) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < HP; ++i) {
@@ -485,12 +498,21 @@ __device__ __forceinline__ void ht64_wave(const double *__restrict__ Lj, int n, 
       for (int j = 0; j < NBV; ++j) acc[OT - 1][j] = F64::mma(co, x[j], acc[OT - 1][j]);
       if (s < 3) load_co(buf, s + 1);
     }
+    if constexpr (TQ > 0) {
+#pragma unroll
+      for (int q = 0; q < TQ; ++q)
+#pragma unroll
+        for (int j = 0; j < NBV; ++j)
+          accq[q][j] = __builtin_amdgcn_mfma_f64_4x4x4f64(q < 2 ? cq[q] : ct, x[j], accq[q][j], 0, 0, 0);
+      if (s < 3) load_cq(buf, s + 1);
+    }
   };
   auto first_c = [&](int buf) __attribute__((always_inline)) {
     if constexpr (NBV > 0) {
 #pragma unroll
       for (int i = 0; i < HP; ++i) load_cp(buf, 0, i);
       load_co(buf, 0);
+      load_cq(buf, 0);
     }
   };
 
@@ -667,19 +689,25 @@ __device__ __forceinline__ void ht64_wave(const double *__restrict__ Lj, int n, 
         const int k = t < 2 * HP ? 32 * (t >> 1) + 2 * row + (t & 1) : 16 * t + row;
         xj[int64_t(k) * n_pad + a] = a < n ? acc[t][j][r] : 0.0;  // clamped columns
       }
+#pragma unroll
+    for (int q = 0; q < TQ; ++q) {
+      const int k = 16 * OT + (TQ == 1 ? g : q < 2 ? 2 * g + q : 8 + g);
+      xj[int64_t(k) * n_pad + a] = a < n ? accq[q][j] : 0.0;
+    }
   }
 }
 
 // grid.x = round_up(ceil(jc * W / 4), 8): four wave items per workgroup, item =
 // J * W + t over the W = ceil(nblk / nb) waves of a vector (nblk = ceil(n / 16)
 // column blocks, nb <= NB of them per wave).
-template <int OT, int NB, bool FV>
+template <int OT, int TQ, int NB, bool FV>
 __global__ __launch_bounds__(kThreads, 2) void k_ht64(const double *__restrict__ L, int64_t ldl, int n, int n_pad,
                                                    const double *__restrict__ Cb, int64_t j0, int64_t jc, int W,
                                                    int nb, int64_t nblocks, double *__restrict__ X,
                                                    const Screen sc, const FuseV fv) {
   static_assert(NB <= 4, "tail widths");
-  __shared__ __attribute__((aligned(16))) double sC[2][kHtB * 16 * OT];
+  constexpr int LDC = ht64_ldc(OT, TQ);
+  __shared__ __attribute__((aligned(16))) double sC[2][kHtB * LDC];
   __shared__ __attribute__((aligned(16))) double sT[4][NB * 16 * kHtS];
   const int64_t lb = xcd_logical(nblocks);
   if (lb < 0) return;
@@ -692,7 +720,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_ht64(const double *__restrict__
   const int a0 = 16 * nb * t;
   int nbv = live ? min(nb, nblk - nb * t) : 0;
   const double *__restrict__ Lj = L + (j0 + J) * ldl;
-  double *__restrict__ xj = X + J * (16 * OT) * int64_t(n_pad);
+  double *__restrict__ xj = X + J * LDC * int64_t(n_pad);
   if (sc.lnorm && live) {  // screened: ||X tile||_F <= ||L^J[:, strips of the tile]||_F max_d ||C_d||_F
     double s2 = 0.0;
     for (int st = a0 / 64; st <= (a0 + 16 * nbv - 1) / 64; ++st) {
@@ -700,7 +728,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_ht64(const double *__restrict__
       s2 += v * v;
     }
     if (sqrt(s2) * sc.cmax[0] < sc.thr_x) {
-      for (int e = threadIdx.x & 63; e < 16 * OT * 16 * nbv; e += 64)
+      for (int e = threadIdx.x & 63; e < LDC * 16 * nbv; e += 64)
         xj[int64_t(e / (16 * nbv)) * n_pad + a0 + e % (16 * nbv)] = 0.0;
       if ((threadIdx.x & 63) == 0) atomicAdd(sc.cnt + 1, 1ull);
       nbv = 0;
@@ -709,11 +737,11 @@ __global__ __launch_bounds__(kThreads, 2) void k_ht64(const double *__restrict__
   double *vout = FV ? fv.vpart + int64_t(t) * fv.m + j0 + J : nullptr;
   // a wave without columns still stages its share of the bank and joins the barriers
   switch (nbv) {
-    case 0: ht64_wave<OT, 0, FV>(Lj, n, nch, n_pad, Cb, a0, xj, fv.p, vout, sC, sT[w]); break;
-    case 1: ht64_wave<OT, 1, FV>(Lj, n, nch, n_pad, Cb, a0, xj, fv.p, vout, sC, sT[w]); break;
-    case 2: if constexpr (NB >= 2) ht64_wave<OT, 2, FV>(Lj, n, nch, n_pad, Cb, a0, xj, fv.p, vout, sC, sT[w]); break;
-    case 3: if constexpr (NB >= 3) ht64_wave<OT, 3, FV>(Lj, n, nch, n_pad, Cb, a0, xj, fv.p, vout, sC, sT[w]); break;
-    default: if constexpr (NB >= 4) ht64_wave<OT, 4, FV>(Lj, n, nch, n_pad, Cb, a0, xj, fv.p, vout, sC, sT[w]); break;
+    case 0: ht64_wave<OT, TQ, 0, FV>(Lj, n, nch, n_pad, Cb, a0, xj, fv.p, vout, sC, sT[w]); break;
+    case 1: ht64_wave<OT, TQ, 1, FV>(Lj, n, nch, n_pad, Cb, a0, xj, fv.p, vout, sC, sT[w]); break;
+    case 2: if constexpr (NB >= 2) ht64_wave<OT, TQ, 2, FV>(Lj, n, nch, n_pad, Cb, a0, xj, fv.p, vout, sC, sT[w]); break;
+    case 3: if constexpr (NB >= 3) ht64_wave<OT, TQ, 3, FV>(Lj, n, nch, n_pad, Cb, a0, xj, fv.p, vout, sC, sT[w]); break;
+    default: if constexpr (NB >= 4) ht64_wave<OT, TQ, 4, FV>(Lj, n, nch, n_pad, Cb, a0, xj, fv.p, vout, sC, sT[w]); break;
   }
 }
 
@@ -1620,15 +1648,15 @@ void launch_ht(Context *c, const float *L, const float *cb, int64_t j0, int64_t 
 // block 2.91; n=1200 nocc=150 43.3 / 44.1 ms), one past that (registers).
 constexpr int ht64_nb(int ot) { return ot == 1 ? 4 : ot == 2 ? 3 : ot <= 10 ? 2 : 1; }
 
-template <int OT>
+template <int OT, int TQ>
 void launch_ht64(Context *c, const double *cb, int64_t j0, int64_t jc, double *X) {
-  constexpr int NB = ht64_nb(OT);
+  constexpr int NB = ht64_nb(OT + (TQ > 0));
   const int64_t nblk = ceil_div(c->n, 16);
   // Column blocks per wave of a launch of few rounds of resident workgroups: the
   // count whose last round wastes least (a wave's time goes with its blocks, plus
   // about half a block for its share of the bank and the barriers).  n=187
   // nchol=905 nocc=23: three blocks 84 us (905 workgroups on 768 slots), two 77.
-  constexpr int64_t kPerCu = OT <= 5 ? 3 : 2;
+  constexpr int64_t kPerCu = OT + (TQ > 0) <= 5 ? 3 : 2;
   const int64_t slots = kPerCu * c->ncu;
   int nb = NB;
   double least = 1e300;
@@ -1646,33 +1674,49 @@ void launch_ht64(Context *c, const double *cb, int64_t j0, int64_t jc, double *X
   const dim3 grid(unsigned(round_up(nblocks, 8)));
   if (c->fv.p) {  // fused Coulomb pass (never together with screening)
     c->fv.ntile = W;
-    hipLaunchKernelGGL((k_ht64<OT, NB, true>), grid, dim3(kThreads), 0, c->stream, c->L, c->ldl, c->n, c->n_pad, cb,
+    hipLaunchKernelGGL((k_ht64<OT, TQ, NB, true>), grid, dim3(kThreads), 0, c->stream, c->L, c->ldl, c->n, c->n_pad, cb,
                        j0, jc, W, nb, nblocks, X, Screen{}, c->fv);
     return;
   }
-  hipLaunchKernelGGL((k_ht64<OT, NB, false>), grid, dim3(kThreads), 0, c->stream, c->L, c->ldl, c->n, c->n_pad, cb,
+  hipLaunchKernelGGL((k_ht64<OT, TQ, NB, false>), grid, dim3(kThreads), 0, c->stream, c->L, c->ldl, c->n, c->n_pad, cb,
                      j0, jc, W, nb, nblocks, X, c->scr, FuseV{});
   if (c->scr.lnorm) c->x_tiles += jc * W;
 }
 
-void ht64_dispatch(Context *c, int ot, const double *cb, int64_t j0, int64_t jn, double *X) {
-  switch (ot) {
-    case 1: launch_ht64<1>(c, cb, j0, jn, X); break;
-    case 2: launch_ht64<2>(c, cb, j0, jn, X); break;
-    case 3: launch_ht64<3>(c, cb, j0, jn, X); break;
-    case 4: launch_ht64<4>(c, cb, j0, jn, X); break;
-    case 5: launch_ht64<5>(c, cb, j0, jn, X); break;
-    case 6: launch_ht64<6>(c, cb, j0, jn, X); break;
-    case 7: launch_ht64<7>(c, cb, j0, jn, X); break;
-    case 8: launch_ht64<8>(c, cb, j0, jn, X); break;
-    case 9: launch_ht64<9>(c, cb, j0, jn, X); break;
-    case 10: launch_ht64<10>(c, cb, j0, jn, X); break;
-    case 11: launch_ht64<11>(c, cb, j0, jn, X); break;
-    case 12: launch_ht64<12>(c, cb, j0, jn, X); break;
-    case 13: launch_ht64<13>(c, cb, j0, jn, X); break;
-    case 14: launch_ht64<14>(c, cb, j0, jn, X); break;
-    case 15: launch_ht64<15>(c, cb, j0, jn, X); break;
-    default: launch_ht64<16>(c, cb, j0, jn, X); break;
+template <int OT>  // full tiles before the last
+void launch_ht64_q(Context *c, int rest, const double *cb, int64_t j0, int64_t jn, double *X) {
+  switch ((rest + 3) / 4) {
+    case 1:
+      return launch_ht64<OT, 1>(c, cb, j0, jn, X);
+    case 2:
+      return launch_ht64<OT, 2>(c, cb, j0, jn, X);
+    case 3:
+      if constexpr (OT < 5) return launch_ht64<OT, 3>(c, cb, j0, jn, X);
+      break;
+    default: break;
+  }
+  launch_ht64<OT + 1, 0>(c, cb, j0, jn, X);
+}
+
+// X^J = C^T L^J of the first tot bank columns (stride 16 ceil(tot / 16)).
+void ht64_dispatch(Context *c, int tot, const double *cb, int64_t j0, int64_t jn, double *X) {
+  switch ((tot - 1) / 16) {
+    case 0: launch_ht64_q<0>(c, tot % 16, cb, j0, jn, X); break;
+    case 1: launch_ht64_q<1>(c, tot % 16, cb, j0, jn, X); break;
+    case 2: launch_ht64_q<2>(c, tot % 16, cb, j0, jn, X); break;
+    case 3: launch_ht64_q<3>(c, tot % 16, cb, j0, jn, X); break;
+    case 4: launch_ht64_q<4>(c, tot % 16, cb, j0, jn, X); break;
+    case 5: launch_ht64_q<5>(c, tot % 16, cb, j0, jn, X); break;
+    case 6: launch_ht64_q<6>(c, tot % 16, cb, j0, jn, X); break;
+    case 7: launch_ht64_q<7>(c, tot % 16, cb, j0, jn, X); break;
+    case 8: launch_ht64_q<8>(c, tot % 16, cb, j0, jn, X); break;
+    case 9: launch_ht64_q<9>(c, tot % 16, cb, j0, jn, X); break;
+    case 10: launch_ht64_q<10>(c, tot % 16, cb, j0, jn, X); break;
+    case 11: launch_ht64_q<11>(c, tot % 16, cb, j0, jn, X); break;
+    case 12: launch_ht64_q<12>(c, tot % 16, cb, j0, jn, X); break;
+    case 13: launch_ht64_q<13>(c, tot % 16, cb, j0, jn, X); break;
+    case 14: launch_ht64_q<14>(c, tot % 16, cb, j0, jn, X); break;
+    default: launch_ht64_q<15>(c, tot % 16, cb, j0, jn, X); break;
   }
 }
 
@@ -2029,7 +2073,7 @@ int exchange_segments(Context *c, int32_t nk, const int32_t *nocc, const double 
       phase_begin(c);
       switch (s.prec) {
         case MJK_PREC_FP64:
-          ht64_dispatch(c, ot, static_cast<const double *>(c->w->cbank.ptr), j0, jn,
+          ht64_dispatch(c, tot, static_cast<const double *>(c->w->cbank.ptr), j0, jn,
                         static_cast<double *>(c->w->x.ptr));
           break;
         case MJK_PREC_FP32:
@@ -2094,8 +2138,8 @@ int pack_bank(Context *c, int32_t nk, const int32_t *nocc, const double *const *
   return pack_bank_t<double>(c, nk, nocc, corb, off, 16 * *ot, c->w->cbank);
 }
 
-void ht_launch(Context *c, int ot, const double *cb, int64_t j0, int64_t jn, double *X) {
-  ht64_dispatch(c, ot, cb, j0, jn, X);
+void ht_launch(Context *c, int tot, const double *cb, int64_t j0, int64_t jn, double *X) {
+  ht64_dispatch(c, tot, cb, j0, jn, X);
 }
 
 int exchange(Context *c, int32_t nk, const int32_t *nocc, const double *const *corb, double *klt,

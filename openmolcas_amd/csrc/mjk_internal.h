@@ -212,9 +212,10 @@ int exchange(Context *c, int32_t nk, const int32_t *nocc, const double *const *c
 // round_up(nocc[d], 4).  tot = sum opad (0: nothing packed).
 int pack_bank(Context *c, int32_t nk, const int32_t *nocc, const double *const *corb,
               std::vector<int> &off, std::vector<int> &opad, int *ot, int *tot);
-// Half-transform of vectors j0..j0+jn-1 against the bank (16*ot columns):
-// X[(jr*16*ot + k)*n_pad + a] = sum_b Cb[b][k] L^{j0+jr}_{ab}.
-void ht_launch(Context *c, int ot, const double *cb, int64_t j0, int64_t jn, double *X);
+// Half-transform of vectors j0..j0+jn-1 against the bank's first tot columns (stride
+// ldc = 16*ceil(tot/16)): X[(jr*ldc + k)*n_pad + a] = sum_b Cb[b][k] L^{j0+jr}_{ab};
+// rows of X past tot hold anything.
+void ht_launch(Context *c, int tot, const double *cb, int64_t j0, int64_t jn, double *X);
 
 // Z[J] = X[J] C for the jn vectors of one half-transform chunk: X holds
 // 16*ot = ldc rows of n_pad per vector, FP64 (x_f32 false) or FP32; C is the

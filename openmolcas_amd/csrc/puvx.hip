@@ -187,7 +187,7 @@ extern "C" int mjk_puvx(mjk_context *c, int32_t naorb, const double *porb3, cons
   for (int64_t ch = 0; ch < nchunk; ++ch) {
     const int64_t j0 = ch * jc, jn = std::min(jc, M - j0);
     phase_begin(c);
-    ht_launch(c, ot, cb, j0, jn, Y);
+    ht_launch(c, tot, cb, j0, jn, Y);
     phase_end(c, MJK_PHASE_HALF_TRANSFORM);
     phase_begin(c);
     if ((rc = z_from_x(c, Y, false, ldc, naorb, jn, z))) return rc;
