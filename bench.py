@@ -519,12 +519,12 @@ def batch_workload(args, dev):
     bw_f = sum(M * ((2.0 if z is not None else 4.0) * n * o * o + 1.0 * n * (n + 1) * o)
                for z, (n, M, o) in zip(batch.Z, shapes))
     ph = {
-        "half_transform": ("k_ht<F64> (X = C^T L with the Coulomb V inside)", "k_ht", ht_f,
+        "half_transform": ("k_ht64 (X = C^T L with the Coulomb V inside)", "k_ht64", ht_f,
                            phases["half_transform"]),
-        "exchange": ("k_syrk<F64> (K = sum X^T X)", "k_syrk", sy_f, phases["exchange"]),
+        "exchange": ("k_syrk64 (K = sum X^T X)", "k_syrk64", sy_f, phases["exchange"]),
         "backward": ("k_grad_rows (dE/dL: W = C Z and the packed W C^T in one launch)", "k_grad_rows",
                      bw_f, phases["backward"]),
-        "zsave": ("k_gemm (Z = X C kept by the forward)", "k_gemm", z_f, phases["zsave"]),
+        "zsave": ("k_zsym (Z = X C kept by the forward)", "k_zsym", z_f, phases["zsave"]),
     }
     name, (label, family, flops, (ms, calls)) = max(ph.items(), key=lambda kv: kv[1][3][0])
     achieved = flops / (ms * 1e-3) / 1e12
@@ -685,9 +685,9 @@ def single_build(args, dev, steps):
     ms_step = 1000.0 * elapsed / steps
 
     # algorithmic work (per build)
-    # the Coulomb passes of their own: V and J (two reads of L), or J alone when
-    # V rides in the half-transform
-    bytes_j = (1.0 if fused else 2.0) * M * npr * 8 + 2.0 * npr * 8 + 2.0 * M * 8
+    # the Coulomb passes of their own: V and J (two reads of L), or one read when V
+    # rides in the half-transform or one kernel does both (no V phase then)
+    bytes_j = (2.0 if phases["coulomb_v"][1] else 1.0) * M * npr * 8 + 2.0 * npr * 8 + 2.0 * M * 8
     flops_ht = 2.0 * M * o * n * n
     flops_syrk = 1.0 * M * o * n * (n + 1)
     peak = PEAK_TFLOPS[args.precision]
@@ -711,13 +711,13 @@ def single_build(args, dev, steps):
     k_tf = (flops_ht + flops_syrk) / (k_ms * 1e-3) / 1e12
     # dominant kernel: the larger of the two exchange kernels by time
     # kernel names as the profiles list them (split-BF16 has kernels of its own)
-    kht, ksy = {"fp64": ("k_ht<F64", "k_syrk<F64"), "fp32": ("k_ht<F32", "k_syrk<F32"),
+    kht, ksy = {"fp64": ("k_ht64", "k_syrk64"), "fp32": ("k_ht<F32", "k_syrk<F32"),
                 "bf16x3": ("k_ht_b3", "k_syrk_b3")}[args.precision]
     if ht_ms * ht_calls >= sy_ms * sy_calls:
         what = "half-transform X = C^T L" + (" with the Coulomb V = L^T D; MFMA flops only" if fused else "")
-        dom = (f"{kht}> ({what})", ht_tf, kht + ("," if "<" in kht else "<"))
+        dom = (f"{kht}{'>' * ('<' in kht)} ({what})", ht_tf, kht)
     else:
-        dom = (f"{ksy}> (K = sum X^T X)", sy_tf, ksy + ("," if "<" in ksy else "<"))
+        dom = (f"{ksy}{'>' * ('<' in ksy)} (K = sum X^T X)", sy_tf, ksy)
     peaks = {name: round(ctx.measure_peak(kind), 2) for name, kind in
              (("mfma_f64_TFs", 0), ("mfma_f32_TFs", 1), ("mfma_bf16_TFs", 2), ("fma_f64_TFs", 3),
               ("copy_TBs", 4))}

@@ -88,9 +88,10 @@ int mjk_create_shared(mjk_context **ctx, int32_t nbas, int64_t nchol, mjk_contex
  * buffer that Cho_X_Init fills (src/cholesky_util/cho_x_init.F90:16-52). */
 int mjk_device_vectors(mjk_context *ctx, double **L, int64_t *ldl);
 
-/* Exchange tiling: SYRK tile (0 automatic, 64, 128), SYRK workgroups per
- * launch at most (0 automatic; whole rounds of two per CU avoid a tail round),
- * half-transform AO tile (0, 64, 128). */
+/* Exchange tiling: SYRK workgroups per launch to aim for (split_target, 0
+ * automatic); in the reduced precisions also the SYRK tile (0 automatic, 64, 128)
+ * and the half-transform's AO tile (0, 64, 128).  The FP64 kernels choose their own
+ * tiles. */
 int mjk_set_tuning(mjk_context *ctx, int32_t tile_syrk, int32_t split_target, int32_t ht_ta);
 
 /* One-pass Coulomb build: how often a workgroup looks whether the others of its

@@ -12,10 +12,11 @@
 // V = sqrt(2) C); the gradient has no counterpart in the reference, which only
 // evaluates the Fock matrix.
 //
-// Kernels: the half-transform X^J = C^T L^J is recomputed chunk by chunk (the
-// chunk size follows the context's X budget); Z = X C, W = C Z and the packed
-// lower triangle of W C^T go through one batched FP64-MFMA GEMM whose epilogue
-// writes the vector gradient directly in packed storage.
+// Kernels: with Z kept by the forward, k_grad_rows forms W = C Z in registers and
+// the packed lower triangle of W C^T in one launch; without it X^J = C^T L^J is
+// recomputed chunk by chunk (the chunk size follows the context's X budget) and
+// Z = X C comes from k_zsym.  Above 128 orbitals W and the packed product go
+// through one batched FP64-MFMA GEMM whose epilogue writes packed storage.
 #include <type_traits>
 
 #include "mjk_internal.h"

@@ -694,6 +694,8 @@ int vector_norms(Context *c, double *w) {
 
 namespace {
 
+constexpr size_t kScratchBytes = size_t(64) << 20;  // the fixed buffer of coulomb_noalloc, below
+
 // Work split and scratch of one Coulomb build (both passes).
 struct CoulombPlan {
   int nd = 0, ndt = 0;
@@ -733,16 +735,22 @@ constexpr int kOneGrid = 256;  // workgroups: one per CU
 // streams).  Groups: as many as fit, with at least eight vectors each, below which
 // their J costs more to write and reduce than the wait for V (n = 130: 33.8 us with
 // two each, 29.8 with eight), but up to 32 when vectors are few (n = 500, 16 vectors:
-// 36 us in two groups, 28 in eight).
+// 36 us in two groups, 28 in eight).  Its scratch stays within the fixed buffer of
+// coulomb_noalloc (tens of thousands of vectors reach it), so that entry takes what
+// the two passes take.
 bool plan_one(const Context *c, int nd, CoulombPlan *p) {
   const int64_t M = c->nchol, ldl = c->ldl;
   if (nd > 2 || ldl < 8192) return false;
   const int64_t gmin = ceil_div(ldl, kOneRow * one_rows_max(nd));
   if (gmin > kOneGrid / 2 || gmin * nd > 256) return false;
   const int64_t want = std::max<int64_t>({M / 8, std::min<int64_t>(M / 2, 32), 1});
-  p->ngrp = int(std::min<int64_t>(kOneGrid / gmin, want));
-  p->slice = round_up(ceil_div(ldl, std::min<int64_t>(kOneGrid / p->ngrp, 256 / nd)), 2 * kWave);
-  p->group = int(ceil_div(ldl, p->slice));
+  const int64_t ngrp = std::min<int64_t>(kOneGrid / gmin, want);
+  const int64_t slice = round_up(ceil_div(ldl, std::min<int64_t>(kOneGrid / ngrp, 256 / nd)), 2 * kWave);
+  const int64_t group = ceil_div(ldl, slice);
+  if ((M * (group + 1) + (ngrp + 1) * ldl) * nd * sizeof(double) > kScratchBytes - 65536) return false;
+  p->ngrp = int(ngrp);
+  p->slice = slice;
+  p->group = int(group);
   p->nsplit2 = p->ngrp;
   p->nparts = p->group > 1 ? M * p->group * nd : 0;
   p->bytes_vpart = sizeof(double) * size_t(p->nparts) + sizeof(OneGate) * size_t(p->ngrp);
@@ -913,7 +921,6 @@ int coulomb_run(Context *c, Scratch &s, int32_t nd, const double *dlt, int64_t l
 // object and held until the process ends.  Host code uses the address that
 // hipGetSymbolAddress returns for the current device, never the array's name
 // (that is a host-side stand-in, not a device address).
-constexpr size_t kScratchBytes = size_t(64) << 20;
 constexpr int kMaxDevices = 64;
 __device__ __align__(256) double scratch[kScratchBytes / sizeof(double)];
 

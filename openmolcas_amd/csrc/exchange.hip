@@ -385,9 +385,16 @@ __global__ __launch_bounds__(kThreads) void k_ht(
 // packed element is read twice, 3.7 TB/s at n=512 nocc=64).  With the V work:
 // n=1200 nchol=6000 nocc=150 55.3 -> 43.3 ms (65 TFLOP/s executed), n=536
 // nchol=2510 nocc=98 3.7 -> 2.8 ms, n=512 nchol=2048 nocc=64 1.40 -> 1.34 ms,
-// n=187 nchol=905 nocc=23 0.116 -> 0.084 ms, against staging square tiles of L
+// n=187 nchol=905 nocc=23 0.116 -> 0.077 ms, against staging square tiles of L
 // in LDS (its transposing stores, their waits and 5 VALU operations per MFMA
 // stood between the MFMAs).
+// TQ: columns past the OT full tiles go in quarters of four, v_mfma_f64_4x4x4 (four
+// 4x4 blocks, one per four AO columns): it takes the same B operand and runs at the
+// same rate (76 TFLOP/s measured), so the bank is padded to 4 columns, not 16.  Lane
+// group g holds row g of a quarter; quarters 0 and 1 take alternate columns of eight
+// (one 16-byte read).  Without the V work, against full tiles only: n=1200 nocc=150
+// 43.3 -> 40.1 ms, n=536 nocc=98 2.81 -> 2.63, n=400 nocc=50 0.78 -> 0.70, n=301
+// nocc=40 0.28 -> 0.25, n=187 nocc=23 0.061 -> 0.053 ms.
 constexpr int kHtB = 16;       // contraction rows per chunk
 constexpr int kHtS = 17;       // row stride of a turned block
 constexpr int ht64_ldc(int ot, int tq) { return 16 * (ot + (tq > 0)); }  // bank columns
@@ -1683,6 +1690,8 @@ void launch_ht64(Context *c, const double *cb, int64_t j0, int64_t jc, double *X
   if (c->scr.lnorm) c->x_tiles += jc * W;
 }
 
+// Three quarters only up to four full tiles: past that they save a quarter of one
+// tile in six or more, less than the variants' place in the library is worth.
 template <int OT>  // full tiles before the last
 void launch_ht64_q(Context *c, int rest, const double *cb, int64_t j0, int64_t jn, double *X) {
   switch ((rest + 3) / 4) {

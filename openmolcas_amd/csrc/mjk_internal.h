@@ -52,15 +52,15 @@ struct Screen {
   unsigned long long *cnt = nullptr;  // [K items skipped, X tiles skipped]
 };
 
-// Coulomb pass V = L^T D fused into the FP64 half-transform (p null = off):
-// workgroup (vector J, AO tile t) adds sum_{a in t} sum_{b >= a} L^J_ba D_ba
-// into vpart[t * m + J], with D the folded density in packed storage, so
+// Coulomb pass V = L^T D fused into the FP64 half-transform (p null = off): the
+// wave of vector J and AO columns t writes sum_{a in t} sum_{b >= a} L^J_ba D_ba
+// to vpart[t * m + J], with D the folded density in packed storage, so
 // sum_t vpart[t * m + J] = sum_{b >= a} L^J_ba D_ba.
 struct FuseV {
   const double *p = nullptr;
   double *vpart = nullptr;
   int64_t m = 0;   // row stride of vpart (vector capacity)
-  int ntile = 0;   // AO tiles per vector of the last launch (set by the launcher)
+  int ntile = 0;   // waves per vector of the last launch (set by the launcher)
 };
 
 // Z^J = C^T L^J C saved by the exchange in progress for the backward (z null =
@@ -149,10 +149,10 @@ struct Context {
   Workspace *w = nullptr;
 
   // tunables (0 = automatic); set by mjk_set_tuning or the autotuner
-  int32_t tile_syrk = 0;     // SYRK tile: 64 or 128
+  int32_t tile_syrk = 0;     // SYRK tile of the reduced precisions: 64 or 128
   int32_t coulomb_looks = 64;  // one-pass J: looks for the other workgroups' start (about 1 us each)
   int32_t split_target = 0;  // SYRK workgroups per launch to aim for
-  int32_t ht_ta = 0;         // half-transform AO tile: 64 or 128
+  int32_t ht_ta = 0;         // half-transform AO tile of the reduced precisions: 64 or 128
 
   // profiling: per-phase accumulated milliseconds and launch counts
   bool profile = false;
