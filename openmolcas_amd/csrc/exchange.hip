@@ -2082,7 +2082,8 @@ int exchange_segments(Context *c, int32_t nk, const int32_t *nocc, const double 
       phase_begin(c);
       switch (s.prec) {
         case MJK_PREC_FP64:
-          ht64_dispatch(c, tot, static_cast<const double *>(c->w->cbank.ptr), j0, jn,
+          // the reduced precisions may round the bank up by a tile: all of it then
+          ht64_dispatch(c, ceil_div(tot, 16) == ot ? tot : ldc, static_cast<const double *>(c->w->cbank.ptr), j0, jn,
                         static_cast<double *>(c->w->x.ptr));
           break;
         case MJK_PREC_FP32:

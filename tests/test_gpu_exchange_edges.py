@@ -52,3 +52,25 @@ def test_exchange_at_tile_edges(gpu, n, M, occ):
     assert np.all(np.abs(V[:, 0] - v) <= vb)
     jb = 2.0 * (npair(n) + M + 16) * U * ((np.abs(L) @ np.abs(dlt)) @ np.abs(L))
     assert np.all(np.abs(J[0] - v @ L) <= jb)
+
+
+@pytest.mark.parametrize("n,M,occ", [(40, 9, [3]), (41, 9, [21]), (60, 7, [38]), (150, 6, [130]), (170, 6, [70, 5, 66]),
+                                     (180, 5, [161]), (210, 5, [120, 9, 14, 4, 6, 13, 11, 5, 10]), (230, 4, [225])])
+@pytest.mark.parametrize("n_fp64", [0, 2, 3])
+def test_fp64_head_and_fp32_tail_share_one_bank(gpu, n, M, occ, n_fp64):
+    """Banks whose FP64 width in quarter tiles is not the reduced precisions' (an even
+    number of tiles past eight).  The tail's rounding: the same sums at u = 2^-24, with
+    three more for the inputs."""
+    L = chol_vectors_np(n, M, seed=n + M)
+    Cs = [orbitals_np(n, o, seed=7 * n + d) for d, o in enumerate(occ)]
+    Lf = lfull(L, n)
+    jk = JKContext(n, M, device=gpu)
+    jk.upload_packed(L)
+    K = jk.exchange_mixed([torch.from_numpy(np.ascontiguousarray(c)) for c in Cs], n_fp64, M).cpu().numpy()
+    jk.close()
+    for d, C in enumerate(Cs):
+        X, A = Lf @ C, np.abs(Lf) @ np.abs(C)
+        ref = sum(x @ x.T for x in X)
+        head, tail = (sum((a @ a.T for a in s), np.zeros((n, n))) for s in (A[:n_fp64], A[n_fp64:]))
+        c = 2.0 * (2 * n + M * C.shape[1] + 19)
+        assert np.all(np.abs(K[d] - pack(ref)) <= pack(c * (U * head + 2.0 ** -24 * tail))), (n, M, occ, n_fp64, d)
