@@ -1917,24 +1917,35 @@ int64_t plan_syrk64(const Context *c, int32_t nk, const int32_t *nocc, const std
   const int64_t slots = 2 * int64_t(c->ncu), steps = jc * work / 4;
   const int64_t rounds = std::min<int64_t>(64, std::max<int64_t>(1, steps * units / (16 * 4 * 160 * slots)));
   const int64_t target = c->split_target ? c->split_target : slots * rounds;
+  // Slices of every set for `aim` workgroups; the number there will be (each XCD's
+  // eighth of a set's two item lists is rounded up).
+  auto slices = [&](int64_t aim) {
+    for (int d = 0; d < nk; ++d) {
+      s.nsf[d] = s.nsd[d] = 0;
+      if (nocc[d] > 0) {
+        const int64_t own = aim * opad[size_t(d)];
+        // at least 4 steps per wave, at most one slice per vector
+        const int64_t most = std::max<int64_t>(1, std::min<int64_t>(jc, jc * opad[size_t(d)] / 64));
+        auto clip = [&](int64_t v) { return int(std::max<int64_t>(1, std::min<int64_t>(v, most))); };
+        s.nsf[d] = clip(own * 16 / (work * units));
+        s.nsd[d] = clip(own * 10 / (work * units));
+      }
+      s.item0[d + 1] = s.item0[d] + int(8 * (ceil_div(s.nsd[d] * T, 8) + ceil_div(s.nsf[d] * nf, 8)));
+    }
+    return int64_t(s.item0[nk]);
+  };
+  // No more than the target: 520 workgroups on 512 slots took a second round
+  // (two or three tiles across: n=187 nocc=23 30.5 -> 22.6 us, n=175 nocc=50 52 -> 37,
+  // n=131 nocc=42 31 -> 26).
+  for (int64_t aim = target; slices(aim) > target && aim > target / 2;) aim -= 8;
   int64_t kb = 0;
   for (int d = 0; d < nk; ++d) {
     s.off[d] = off[size_t(d)];
     s.opad[d] = std::max(opad[size_t(d)], 4);
-    s.nsf[d] = s.nsd[d] = 0;
-    if (nocc[d] > 0) {
-      const int64_t own = target * opad[size_t(d)];
-      // at least 4 steps per wave, at most one slice per vector
-      const int64_t most = std::max<int64_t>(1, std::min<int64_t>(jc, jc * opad[size_t(d)] / 64));
-      auto clip = [&](int64_t v) { return int(std::max<int64_t>(1, std::min<int64_t>(v, most))); };
-      s.nsf[d] = clip(own * 16 / (work * units));
-      s.nsd[d] = clip(own * 10 / (work * units));
-    }
     s.kf[d] = kb;
     kb += s.nsf[d] * nchunk * nf * kSlot64;
     s.kd[d] = kb;
     kb += s.nsd[d] * nchunk * T * kSlot64;
-    s.item0[d + 1] = s.item0[d] + int(8 * (ceil_div(s.nsd[d] * T, 8) + ceil_div(s.nsf[d] * nf, 8)));
   }
   return kb;
 }
