@@ -1665,15 +1665,18 @@ void launch_ht64(Context *c, const double *cb, int64_t j0, int64_t jc, double *X
   // nchol=905 nocc=23: three blocks 84 us (905 workgroups on 768 slots), two 77.
   constexpr int64_t kPerCu = OT + (TQ > 0) <= 5 ? 3 : 2;
   const int64_t slots = kPerCu * c->ncu;
-  int nb = NB;
-  double least = 1e300;
-  for (int v = NB; v >= 1; --v) {
-    const int64_t wgs = ceil_div(jc * ceil_div(nblk, v), 4), rounds = ceil_div(wgs, slots);
-    if (v == NB && rounds > 8) break;
-    const double cost = double(rounds) * (v + 0.5);
-    if (cost < least) {
-      least = cost;
-      nb = v;
+  int nb = c->fv.p ? c->fv.nb : 0;  // V: as the first chunk of this exchange
+  if (!nb) {
+    nb = NB;
+    double least = 1e300;
+    for (int v = NB; v >= 1; --v) {
+      const int64_t wgs = ceil_div(jc * ceil_div(nblk, v), 4), rounds = ceil_div(wgs, slots);
+      if (v == NB && rounds > 8) break;
+      const double cost = double(rounds) * (v + 0.5);
+      if (cost < least) {
+        least = cost;
+        nb = v;
+      }
     }
   }
   const int W = int(ceil_div(nblk, nb));
@@ -1681,6 +1684,7 @@ void launch_ht64(Context *c, const double *cb, int64_t j0, int64_t jc, double *X
   const dim3 grid(unsigned(round_up(nblocks, 8)));
   if (c->fv.p) {  // fused Coulomb pass (never together with screening)
     c->fv.ntile = W;
+    c->fv.nb = nb;
     hipLaunchKernelGGL((k_ht64<OT, TQ, NB, true>), grid, dim3(kThreads), 0, c->stream, c->L, c->ldl, c->n, c->n_pad, cb,
                        j0, jc, W, nb, nblocks, X, Screen{}, c->fv);
     return;

@@ -60,7 +60,9 @@ struct FuseV {
   const double *p = nullptr;
   double *vpart = nullptr;
   int64_t m = 0;   // row stride of vpart (vector capacity)
-  int ntile = 0;   // waves per vector of the last launch (set by the launcher)
+  // waves per vector and 16-column blocks per wave: chosen by the launcher for the first
+  // (largest) chunk and kept for the others, so that every vector has the same parts
+  int ntile = 0, nb = 0;
 };
 
 // Z^J = C^T L^J C saved by the exchange in progress for the backward (z null =
