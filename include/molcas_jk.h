@@ -412,15 +412,19 @@ int mjk_exchange(mjk_context *ctx, int32_t nk, const int32_t *nocc,
 
 /* mjk_coulomb without any allocation, for callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops,
- * harnesses that forbid it).  No counterpart in the reference.  Same kernels
- * and results as mjk_coulomb; every scratch buffer (the padded density, the
+ * harnesses that forbid it).  No counterpart in the reference.  The same
+ * results as mjk_coulomb, bit for bit; one or two densities read the vectors
+ * twice where mjk_coulomb reads them once (n=512, 1000 vectors: 347 against
+ * 195 us), because the scratch is shared and so nothing may be waited for in
+ * it on the device.  Every scratch buffer (the padded density, the
  * partial sums of V and J, and V when v_out is NULL) lives in one fixed
  * 64 MiB device array per GPU, set up with the library and held until the
  * process ends.  Builds that need more scratch than 64 MiB return
  * MJK_ERR_ARG (the scratch grows with nd, nchol and nbas(nbas+1)/2: about
  * nd * nbas(nbas+1)/2 * 8 bytes times the number of vector slices of the J
- * pass).  Calls that overlap on one GPU share the array and race; calls on
- * one context are serialised by its stream. */
+ * pass).  Calls that overlap on one GPU share the array and race: their
+ * results are wrong, but every call ends; calls on one context are serialised
+ * by its stream. */
 int mjk_coulomb_noalloc(mjk_context *ctx, int32_t nd, const double *dlt, int64_t ldd,
                         double *jlt, int64_t ldj, double *v_out);
 

@@ -292,21 +292,24 @@ __device__ inline int one_take(int *n) {
 // 1200 vectors, J on four 572 -> 516, J and K on four 2186 -> 1629; n=701, 700 vectors
 // J on two 853 -> 626, on four 1754 -> 1881, J and K on four 9552 -> 7925.  With 4096
 // looks 4 x J at n=900 took 23000; 16 or 8 looks: +2 to +11% at n=301, none gained.
+//
+// step kParts, then kSums in a second launch: every member does that for its own slice
+// and waits for nobody, whatever other calls write to the exchange and the gates.
+enum OneStep { kTogether, kParts, kSums };
 template <int ND, int ROWS>
 __global__ __launch_bounds__((kOneWaves + 1) * kWave) void k_coulomb_one(
     const double *__restrict__ L, int64_t ldl, int64_t M, const double *__restrict__ D, int ngrp, int G, int64_t slice,
-    int looks, OneGate *gate, double *part, double *__restrict__ V, double *__restrict__ jpart) {
+    int looks, OneStep step_only, OneGate *gate, double *part, double *__restrict__ V, double *__restrict__ jpart) {
   constexpr int R = kOneRing, LAG = R - 3;
   __shared__ __attribute__((aligned(16))) v2d sD[ND][ROWS * kOneWaves * kWave];
   __shared__ double sP[R][ND][kOneWaves];
   __shared__ double sV[2][ND];
   __shared__ int sTask;  // slice to work on next; < 0: none
-  enum { kTogether, kParts, kSums };
   const int lane = threadIdx.x & (kWave - 1), w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int grp = blockIdx.x / G;
   const int T = int((M - grp + ngrp - 1) / ngrp);
   const int steps = (T + LAG + R - 1) / R * R;
-  int mem = blockIdx.x % G, mode = kTogether;
+  int mem = blockIdx.x % G, mode = step_only;
 
   for (;;) {
     const int64_t p0 = min(mem * slice, ldl), len = min(slice, ldl - p0);
@@ -338,7 +341,7 @@ __global__ __launch_bounds__((kOneWaves + 1) * kWave) void k_coulomb_one(
             const double *row = part + J * G * ND;
             const int cnt = G * ND;  // <= 256
             double x[4];
-            for (;;) {  // the others run: their parts come
+            for (;;) {  // the others run: their parts come (kSums alone: they are there)
               bool ok = true;
               auto look = [&](int k) {
                 return __hip_atomic_load(row + min(lane + 64 * k, cnt - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -355,7 +358,7 @@ __global__ __launch_bounds__((kOneWaves + 1) * kWave) void k_coulomb_one(
                 ok = ok && __builtin_bit_cast(int64_t, x[k]) != kOneEmpty;
                 if (lane + 64 * k >= cnt) x[k] = 0.0;
               }
-              if (__all(ok)) break;
+              if (__all(ok) || step_only) break;
               __builtin_amdgcn_s_sleep(1);
             }
             const double y = (x[0] + x[1]) + (x[2] + x[3]);
@@ -441,6 +444,7 @@ __global__ __launch_bounds__((kOneWaves + 1) * kWave) void k_coulomb_one(
         }
       }
     }
+    if (step_only) return;
     // ---- apart: the next slice
     if (mode == kTogether && __builtin_amdgcn_readfirstlane(sTask) >= 0) return;
     lds_barrier();  // everybody has read sTask
@@ -861,16 +865,26 @@ int coulomb_run(Context *c, Scratch &s, int32_t nd, const double *dlt, int64_t l
   if (p.group) {
     double *jpart;
     if ((rc = take(c, s, c->w->jpart, p.bytes_jpart, &jpart))) return rc;
-    phase_begin(c);
     const dim3 grid(unsigned(p.ngrp * p.group)), block((kOneWaves + 1) * kWave);
     OneGate *gate = reinterpret_cast<OneGate *>(vpart + p.nparts);
-    if (nd == 1)
-      hipLaunchKernelGGL((k_coulomb_one<1, one_rows_max(1)>), grid, block, 0, c->stream, c->L, ldl, M, Dp, p.ngrp,
-                         p.group, p.slice, c->coulomb_looks, gate, vpart, V, jpart);
-    else
-      hipLaunchKernelGGL((k_coulomb_one<2, one_rows_max(2)>), grid, block, 0, c->stream, c->L, ldl, M, Dp, p.ngrp,
-                         p.group, p.slice, c->coulomb_looks, gate, vpart, V, jpart);
-    phase_end(c, MJK_PHASE_COULOMB_J);
+    auto one = [&](OneStep step, int phase) {
+      phase_begin(c);
+      if (nd == 1)
+        hipLaunchKernelGGL((k_coulomb_one<1, one_rows_max(1)>), grid, block, 0, c->stream, c->L, ldl, M, Dp, p.ngrp,
+                           p.group, p.slice, c->coulomb_looks, step, gate, vpart, V, jpart);
+      else
+        hipLaunchKernelGGL((k_coulomb_one<2, one_rows_max(2)>), grid, block, 0, c->stream, c->L, ldl, M, Dp, p.ngrp,
+                           p.group, p.slice, c->coulomb_looks, step, gate, vpart, V, jpart);
+      phase_end(c, phase);
+    };
+    // The fixed buffer may be written by an overlapping call, so nothing is waited for
+    // in it: two reads of the vectors, the same bits.
+    if (s.arena && p.group > 1) {
+      one(kParts, MJK_PHASE_COULOMB_V);
+      one(kSums, MJK_PHASE_COULOMB_J);
+    } else {
+      one(kTogether, MJK_PHASE_COULOMB_J);
+    }
     phase_begin(c);
     hipLaunchKernelGGL(k_reduce_j, dim3(unsigned(ceil_div(c->np, 64)), unsigned(nd)), dim3(256), 0, c->stream, jpart,
                        ldl, c->np, nd, p.ngrp, jlt, ldj);
