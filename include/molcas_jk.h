@@ -77,7 +77,8 @@ int mjk_destroy(mjk_context *ctx);
 
 /* As mjk_create, but the new context shares the device workspaces and the
  * stream of `share` (many small systems, one set of scratch buffers; calls on
- * contexts that share must not overlap).  Library-internal design: no
+ * contexts that share must not overlap: on streams of their own they race, and
+ * a Coulomb build may take seconds and give NaN).  Library-internal design: no
  * reference counterpart. */
 int mjk_create_shared(mjk_context **ctx, int32_t nbas, int64_t nchol, mjk_context *share);
 
@@ -100,6 +101,13 @@ int mjk_set_tuning(mjk_context *ctx, int32_t tile_syrk, int32_t split_target, in
  * the wait when other streams hold the GPU. */
 int mjk_set_coulomb_looks(mjk_context *ctx, int32_t looks);
 
+/* One-pass Coulomb build: how often a workgroup looks for a value that another
+ * one that has started owes it (default 2^22, seconds), after which J and V are
+ * NaN.  Such a value comes within milliseconds unless another call writes to the
+ * workspace meanwhile, which the rules of mjk_create_shared and mjk_set_stream
+ * exclude; the limit makes the kernel end all the same. */
+int mjk_set_coulomb_waits(mjk_context *ctx, int32_t looks);
+
 /* Times every exchange tiling for these orbital sets and keeps the fastest
  * in the context (best time in *best_ms); klt receives the last K. */
 int mjk_autotune(mjk_context *ctx, int32_t nk, const int32_t *nocc, const double *const *corb,
@@ -109,8 +117,9 @@ int mjk_autotune(mjk_context *ctx, int32_t nk, const int32_t *nocc, const double
 const char *mjk_last_error(const mjk_context *ctx);
 
 /* Queues all later device work of the context on `hip_stream` (a
- * hipStream_t; NULL = the default stream).  A new context uses a stream of
- * its own.  Library-internal design: no reference counterpart. */
+ * hipStream_t; NULL = the default stream).  Work queued before must have
+ * finished, or the new stream must wait for it: both use the context's
+ * workspaces.  A new context uses a stream of its own.  Library-internal design: no reference counterpart. */
 int mjk_set_stream(mjk_context *ctx, void *hip_stream);
 
 /* Split points of the MJK_PREC_LADDER exchange: vectors [0, j_fp32) in

@@ -41,6 +41,7 @@ SIGNATURES = {
     "mjk_device_vectors": (_c.c_int, [_vp, _c.POINTER(_vp), _c.POINTER(_i64)]),
     "mjk_set_tuning": (_c.c_int, [_vp, _i32, _i32, _i32]),
     "mjk_set_coulomb_looks": (_c.c_int, [_vp, _i32]),
+    "mjk_set_coulomb_waits": (_c.c_int, [_vp, _i32]),
     "mjk_autotune": (_c.c_int, [_vp, _i32, _vp, _vp, _vp, _i64, _i32, _vp]),
     "mjk_set_stream": (_c.c_int, [_vp, _vp]),
     "mjk_set_x_budget": (_c.c_int, [_vp, _i64]),

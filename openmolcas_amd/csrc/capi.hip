@@ -526,6 +526,13 @@ int mjk_set_coulomb_looks(mjk_context *c, int32_t looks) {
   return MJK_OK;
 }
 
+int mjk_set_coulomb_waits(mjk_context *c, int32_t looks) {
+  if (!c) return MJK_ERR_ARG;
+  if (looks < 0) return set_error(c, MJK_ERR_ARG, "set_coulomb_waits: looks < 0");
+  c->coulomb_waits = looks;
+  return MJK_OK;
+}
+
 int mjk_set_reduced_set(mjk_context *c, int32_t jred, int64_t nrs, const int64_t *map) {
   if (!c) return MJK_ERR_ARG;
   if (jred < 0 || jred > 1 << 20 || nrs < 0 || nrs > c->np || (nrs > 0 && !map))

@@ -295,11 +295,16 @@ __device__ inline int one_take(int *n) {
 //
 // step kParts, then kSums in a second launch: every member does that for its own slice
 // and waits for nobody, whatever other calls write to the exchange and the gates.
+//
+// waits: looks (about 1 us each) at what a running member owes, after which V is NaN and
+// nothing more is waited for.  A member answers within milliseconds; only a call that
+// writes to this one's workspace meanwhile (contexts that share one, or one context,
+// on two streams at once) can keep it away for ever.
 enum OneStep { kTogether, kParts, kSums };
 template <int ND, int ROWS>
 __global__ __launch_bounds__((kOneWaves + 1) * kWave) void k_coulomb_one(
     const double *__restrict__ L, int64_t ldl, int64_t M, const double *__restrict__ D, int ngrp, int G, int64_t slice,
-    int looks, OneStep step_only, OneGate *gate, double *part, double *__restrict__ V, double *__restrict__ jpart) {
+    int looks, int waits, OneStep step_only, OneGate *gate, double *part, double *__restrict__ V, double *__restrict__ jpart) {
   constexpr int R = kOneRing, LAG = R - 3;
   __shared__ __attribute__((aligned(16))) v2d sD[ND][ROWS * kOneWaves * kWave];
   __shared__ double sP[R][ND][kOneWaves];
@@ -310,6 +315,7 @@ __global__ __launch_bounds__((kOneWaves + 1) * kWave) void k_coulomb_one(
   const int T = int((M - grp + ngrp - 1) / ngrp);
   const int steps = (T + LAG + R - 1) / R * R;
   int mem = blockIdx.x % G, mode = step_only;
+  if (step_only) waits = 0;
 
   for (;;) {
     const int64_t p0 = min(mem * slice, ldl), len = min(slice, ldl - p0);
@@ -341,7 +347,7 @@ __global__ __launch_bounds__((kOneWaves + 1) * kWave) void k_coulomb_one(
             const double *row = part + J * G * ND;
             const int cnt = G * ND;  // <= 256
             double x[4];
-            for (;;) {  // the others run: their parts come (kSums alone: they are there)
+            for (int left = waits;; --left) {  // the others run: their parts come (kSums alone: they are there)
               bool ok = true;
               auto look = [&](int k) {
                 return __hip_atomic_load(row + min(lane + 64 * k, cnt - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -358,7 +364,11 @@ __global__ __launch_bounds__((kOneWaves + 1) * kWave) void k_coulomb_one(
                 ok = ok && __builtin_bit_cast(int64_t, x[k]) != kOneEmpty;
                 if (lane + 64 * k >= cnt) x[k] = 0.0;
               }
-              if (__all(ok) || step_only) break;
+              if (__all(ok)) break;
+              if (left <= 0) {
+                waits = 0;
+                break;
+              }
               __builtin_amdgcn_s_sleep(1);
             }
             const double y = (x[0] + x[1]) + (x[2] + x[3]);
@@ -458,7 +468,10 @@ __global__ __launch_bounds__((kOneWaves + 1) * kWave) void k_coulomb_one(
           next = one_take(&g->parts);
           if (next >= G) {
             // slices not done are being worked on, and nothing is waited for there
-            while (__hip_atomic_load(&g->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < G) __builtin_amdgcn_s_sleep(8);
+            for (int left = waits; left > 0; --left) {
+              if (__hip_atomic_load(&g->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= G) break;
+              __builtin_amdgcn_s_sleep(8);
+            }
             m = kSums;
           }
         }
@@ -871,10 +884,10 @@ int coulomb_run(Context *c, Scratch &s, int32_t nd, const double *dlt, int64_t l
       phase_begin(c);
       if (nd == 1)
         hipLaunchKernelGGL((k_coulomb_one<1, one_rows_max(1)>), grid, block, 0, c->stream, c->L, ldl, M, Dp, p.ngrp,
-                           p.group, p.slice, c->coulomb_looks, step, gate, vpart, V, jpart);
+                           p.group, p.slice, c->coulomb_looks, c->coulomb_waits, step, gate, vpart, V, jpart);
       else
         hipLaunchKernelGGL((k_coulomb_one<2, one_rows_max(2)>), grid, block, 0, c->stream, c->L, ldl, M, Dp, p.ngrp,
-                           p.group, p.slice, c->coulomb_looks, step, gate, vpart, V, jpart);
+                           p.group, p.slice, c->coulomb_looks, c->coulomb_waits, step, gate, vpart, V, jpart);
       phase_end(c, phase);
     };
     // The fixed buffer may be written by an overlapping call, so nothing is waited for

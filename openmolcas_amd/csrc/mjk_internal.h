@@ -153,6 +153,7 @@ struct Context {
   // tunables (0 = automatic); set by mjk_set_tuning or the autotuner
   int32_t tile_syrk = 0;     // SYRK tile of the reduced precisions: 64 or 128
   int32_t coulomb_looks = 64;  // one-pass J: looks for the other workgroups' start (about 1 us each)
+  int32_t coulomb_waits = 1 << 22;  // and for what those that run owe
   int32_t split_target = 0;  // SYRK workgroups per launch to aim for
   int32_t ht_ta = 0;         // half-transform AO tile of the reduced precisions: 64 or 128
 

@@ -691,6 +691,12 @@ class JKContext:
         not depend on it."""
         self._check(self.lib.mjk_set_coulomb_looks(self._h, int(looks)))
 
+    def set_coulomb_waits(self, looks: int = 1 << 22) -> None:
+        """How often a workgroup of the one-pass Coulomb build looks for a value that a
+        running one owes it before J and V become NaN (only another call on the same
+        workspace at the same time can keep it away)."""
+        self._check(self.lib.mjk_set_coulomb_waits(self._h, int(looks)))
+
     def set_tuning(self, tile_syrk: int = 0, split_target: int = 0, ht_ta: int = 0) -> None:
         self._check(self.lib.mjk_set_tuning(self._h, int(tile_syrk), int(split_target), int(ht_ta)))
 
