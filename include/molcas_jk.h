@@ -92,7 +92,7 @@ int mjk_device_vectors(mjk_context *ctx, double **L, int64_t *ldl);
 /* Exchange tiling: SYRK workgroups per launch to aim for (split_target, 0
  * automatic); in the reduced precisions also the SYRK tile (0 automatic, 64, 128)
  * and the half-transform's AO tile (0, 64, 128).  The FP64 kernels choose their own
- * tiles. */
+ * tiles; these two set what mjk_exchange_screened decides on there. */
 int mjk_set_tuning(mjk_context *ctx, int32_t tile_syrk, int32_t split_target, int32_t ht_ta);
 
 /* One-pass Coulomb build: how often a workgroup looks whether the others of its
@@ -479,15 +479,20 @@ int mjk_exchange_mixed(mjk_context *ctx, int32_t nk, const int32_t *nocc,
  * the device engine (the drop-ins screen the reference's way, see
  * mjk_set_lk_screening): a K tile (TM x TM AOs) of a vector slice
  * is skipped when sum_J ||X^J_A||_F ||X^J_B||_F < tau (an elementwise bound
- * of its contribution), a half-transform tile (one vector, 64 AOs) when
- * ||L^J[:, tile]||_F max_d ||C_d||_F < thr_x.  tau = thr_x = 0 computes
- * everything; precision MJK_PREC_BF16X3 cannot be screened. */
+ * of its contribution), a half-transform tile (one vector; 64 AOs, in FP32 128
+ * up to 96 bank columns) when ||L^J[:, tile]||_F max_d ||C_d||_F < thr_x.
+ * tau = thr_x = 0 computes everything; precision MJK_PREC_BF16X3 cannot be
+ * screened.  TM is 128 from nbas = 385 on, else 64; the slices of a chunk of
+ * vectors share out 1 to 8 rounds of two workgroups per compute unit over the
+ * tiles of nbas rounded up to 128 (mjk_set_tuning changes TM, the target and
+ * the half-transform's tile).  An element of K can miss at most the number of
+ * slices times tau, however the kernels themselves cut the work. */
 int mjk_exchange_screened(mjk_context *ctx, int32_t nk, const int32_t *nocc,
                           const double *const *corb, double *klt, int64_t ldk,
                           int32_t precision, double tau, double thr_x);
 
-/* Work items of the last exchange call: K tiles x slices launched and
- * skipped, half-transform tiles launched and skipped (zero when the call was
+/* Work items of the last exchange call: K tiles x slices tested and
+ * skipped, half-transform tiles tested and skipped (zero when the call was
  * not screened).  Synchronises the context stream.  No counterpart in the
  * reference. */
 int mjk_screening_stats(mjk_context *ctx, int64_t *k_items, int64_t *k_skipped,

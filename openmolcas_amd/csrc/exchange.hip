@@ -87,6 +87,15 @@ struct Syrk64Sets {
   int64_t kf[kMaxSets], kd[kMaxSets];
 };
 
+// K tiles and vector slices that screening decides on (k_keep), `strips` 64-AO strips
+// to a side, ntiles in the lower triangle: set d owns the flags item0[d] + tile *
+// nref[d] + slice.
+struct ScreenSets {
+  int n, strips, ntiles;
+  int nref[kMaxSets];
+  int item0[kMaxSets + 1];
+};
+
 __device__ inline int find_set(const SyrkSets &sets, int b) {
   int d = 0;
   while (d + 1 < sets.n && b >= sets.item0[d + 1]) ++d;
@@ -728,16 +737,17 @@ __global__ __launch_bounds__(kThreads, 2) void k_ht64(const double *__restrict__
   int nbv = live ? min(nb, nblk - nb * t) : 0;
   const double *__restrict__ Lj = L + (j0 + J) * ldl;
   double *__restrict__ xj = X + J * LDC * int64_t(n_pad);
-  if (sc.lnorm && live) {  // screened: ||X tile||_F <= ||L^J[:, strips of the tile]||_F max_d ||C_d||_F
+  if (sc.lnorm && live) {  // screened: ||X tile||_F <= ||L^J[:, tile]||_F max_d ||C_d||_F; the wave lies in one tile
+    const int st0 = a0 / (64 * sc.xw) * sc.xw;
     double s2 = 0.0;
-    for (int st = a0 / 64; st <= (a0 + 16 * nbv - 1) / 64; ++st) {
+    for (int st = st0; st < st0 + sc.xw; ++st) {
       const double v = sc.lnorm[(j0 + J) * sc.nstrip + st];
       s2 += v * v;
     }
     if (sqrt(s2) * sc.cmax[0] < sc.thr_x) {
       for (int e = threadIdx.x & 63; e < LDC * 16 * nbv; e += 64)
         xj[int64_t(e / (16 * nbv)) * n_pad + a0 + e % (16 * nbv)] = 0.0;
-      if ((threadIdx.x & 63) == 0) atomicAdd(sc.cnt + 1, 1ull);
+      if ((threadIdx.x & 63) == 0 && a0 == 64 * st0) atomicAdd(sc.cnt + 1, 1ull);
       nbv = 0;
     }
   }
@@ -981,10 +991,13 @@ __device__ __forceinline__ int slot64_pos(int al, int bl) {
   return 256 * q + 64 * (m >> 2) + 16 * (m & 3) + ((bl >> 1) & 15);
 }
 
-template <bool SH, bool DG>
+// SCR: of the vectors ja .. jz-1 only those whose slice of jref vectors is kept
+// (keep[J / jref]), run by run; with all kept it is the same one run.
+template <bool SH, bool DG, bool SCR>
 __device__ __forceinline__ void syrk64_tile(const double *__restrict__ X, int n_pad, int ldc, int off,
-                                            int q4, int64_t ja, int nst, int A, int B, double *__restrict__ kp,
-                                            double (*__restrict__ red)[4][4][64]) {
+                                            int q4, int64_t ja, int64_t jz, int A, int B, double *__restrict__ kp,
+                                            double (*__restrict__ red)[4][4][64], const uint8_t *__restrict__ keep,
+                                            int64_t jref) {
   constexpr int HA = SH ? 1 : 2, HB = (SH && DG) ? 1 : 2;  // 32-column halves of the two sides
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   v4d acc[2 * HA][2 * HB];
@@ -993,9 +1006,10 @@ __device__ __forceinline__ void syrk64_tile(const double *__restrict__ X, int n_
 #pragma unroll
     for (int j = 0; j < 2 * HB; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
   auto used = [](int i, int j) { return !DG || (i >> 1) > (j >> 1) || ((i >> 1) == (j >> 1) && i >= j); };
-  // steps of this wave and the row pointer of its next load (uniform)
-  const int ns = nst > w ? (nst - w + 3) / 4 : 0;
-  if (ns > 0) {
+  auto run = [&](int64_t ja, int nst) __attribute__((always_inline)) {
+    // steps of this wave and the row pointer of its next load (uniform)
+    const int ns = nst > w ? (nst - w + 3) / 4 : 0;
+    if (ns <= 0) return;
     int kk = w % q4, left = ns;
     const int64_t row4 = 4 * int64_t(n_pad);
     const double *p = X + ((ja + w / q4) * ldc + off) * int64_t(n_pad) + kk * row4;
@@ -1048,6 +1062,19 @@ __device__ __forceinline__ void syrk64_tile(const double *__restrict__ X, int n_
 #pragma unroll
     for (int s = 0; s < kSyrkD - 1; ++s)
       if (t + s < ns) mul(ra[s], rb[s]);
+  };
+  if constexpr (SCR) {
+    for (int64_t j = ja; j < jz;) {
+      int64_t e = (j / jref + 1) * jref;
+      if (keep[j / jref]) {
+        while (e < jz && keep[e / jref]) e += jref;
+        e = min(e, jz);
+        run(j, int(e - j) * q4);
+      }
+      j = e;
+    }
+  } else {
+    run(ja, int(jz > ja ? jz - ja : 0) * q4);  // < 2^29, checked on the host
   }
   // sum of the four waves in wave order: MFMA tiles four at a time through
   // LDS, wave w finishing the w-th of them
@@ -1078,9 +1105,11 @@ __device__ __forceinline__ void syrk64_tile(const double *__restrict__ X, int n_
   }
 }
 
+template <bool SCR>
 __global__ __launch_bounds__(kThreads, 2) void k_syrk64(const double *__restrict__ X, int n, int n_pad,
                                                      int ldc, int64_t jc, int T, const Syrk64Sets sets,
-                                                     double *__restrict__ kpart, int chunk, const Screen sc) {
+                                                     double *__restrict__ kpart, int chunk, const ScreenSets ref,
+                                                     const uint8_t *__restrict__ keep) {
   __shared__ double red[4][4][4][64];
   int set = 0;
   while (set + 1 < sets.n && int(blockIdx.x) >= sets.item0[set + 1]) ++set;
@@ -1114,31 +1143,64 @@ __global__ __launch_bounds__(kThreads, 2) void k_syrk64(const double *__restrict
   const int64_t jper = (jc + ns - 1) / ns;
   const int64_t ja = s * jper, jz = min(jc, ja + jper);
   const int q4 = sets.opad[set] / 4;
-  const int nst = int(jz > ja ? jz - ja : 0) * q4;  // < 2^29, checked on the host
-  if (sc.xn2 && nst > 0) {  // screened: |K_ab| of this slice <= sum_J ||X^J_A||_F ||X^J_B||_F
-    double bound = 0.0;
-    for (int64_t J = ja; J < jz; ++J) {
-      const double *__restrict__ r = sc.xn2 + (int64_t(set) * jc + J) * sc.nstrip;
-      bound += sqrt(r[A] * r[B]);
-    }
-    if (bound < sc.tau) {
+  int64_t jref = 1;
+  if constexpr (SCR) {
+    const int ta = A / ref.strips, tb = B / ref.strips, nref = ref.nref[set];
+    jref = (jc + nref - 1) / nref;
+    keep += ref.item0[set] + (int64_t(ta) * (ta + 1) / 2 + tb) * nref;
+    bool any = false;
+    for (int64_t r = ja / jref; r * jref < jz; ++r) any |= keep[r] != 0;
+    if (!any) {
       for (int e = threadIdx.x; e < kSlot64; e += kThreads) kp[e] = 0.0;
-      if (threadIdx.x == 0) atomicAdd(sc.cnt, 1ull);
       return;
     }
   }
   const bool half = n - A * kT64 <= 32;
   const int off = sets.off[set];
   if (diag) {
-    if (half) syrk64_tile<true, true>(X, n_pad, ldc, off, q4, ja, nst, A, B, kp, red);
-    else syrk64_tile<false, true>(X, n_pad, ldc, off, q4, ja, nst, A, B, kp, red);
+    if (half) syrk64_tile<true, true, SCR>(X, n_pad, ldc, off, q4, ja, jz, A, B, kp, red, keep, jref);
+    else syrk64_tile<false, true, SCR>(X, n_pad, ldc, off, q4, ja, jz, A, B, kp, red, keep, jref);
   } else {
-    if (half) syrk64_tile<true, false>(X, n_pad, ldc, off, q4, ja, nst, A, B, kp, red);
-    else syrk64_tile<false, false>(X, n_pad, ldc, off, q4, ja, nst, A, B, kp, red);
+    if (half) syrk64_tile<true, false, SCR>(X, n_pad, ldc, off, q4, ja, jz, A, B, kp, red, keep, jref);
+    else syrk64_tile<false, false, SCR>(X, n_pad, ldc, off, q4, ja, jz, A, B, kp, red, keep, jref);
   }
 }
 
 // ---- screening norms -------------------------------------------------------
+// keep[item] of the chunk's jn vectors for k_syrk64: a slice's part of a K tile is left
+// out when |K_ab| <= sum_J ||X^J_A||_F ||X^J_B||_F < tau there.  One wave per (set,
+// tile, slice), four per workgroup.
+__global__ __launch_bounds__(kThreads) void k_keep(const double *__restrict__ xn2, int nstrip, int64_t jn,
+                                                  const ScreenSets ref, double tau, uint8_t *__restrict__ keep,
+                                                  unsigned long long *__restrict__ cnt) {
+  const int item = blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (item >= ref.item0[ref.n]) return;
+  int set = 0;
+  while (set + 1 < ref.n && item >= ref.item0[set + 1]) ++set;
+  const int nref = ref.nref[set], t = (item - ref.item0[set]) / nref, s = (item - ref.item0[set]) % nref;
+  int A = int((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
+  while (A * (A + 1) / 2 > t) --A;
+  while ((A + 1) * (A + 2) / 2 <= t) ++A;
+  const int B = t - A * (A + 1) / 2;
+  const int64_t jref = (jn + nref - 1) / nref, ja = s * jref, jz = min(jn, ja + jref);
+  double bound = 0.0;
+  for (int64_t J = ja + lane; J < jz; J += 64) {
+    const double *__restrict__ r = xn2 + (int64_t(set) * jn + J) * nstrip;
+    double a2 = 0.0, b2 = 0.0;
+    for (int st = 0; st < ref.strips; ++st) {
+      a2 += r[A * ref.strips + st];
+      b2 += r[B * ref.strips + st];
+    }
+    bound += sqrt(a2 * b2);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) bound += __shfl_xor(bound, o);
+  if (lane > 0) return;
+  const bool skip = jz > ja && bound < tau;
+  keep[item] = !skip;
+  if (skip) atomicAdd(cnt, 1ull);
+}
+
 __device__ inline double block_sum256(double x, double *red) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
@@ -1670,6 +1732,7 @@ void launch_ht64(Context *c, const double *cb, int64_t j0, int64_t jc, double *X
     nb = NB;
     double least = 1e300;
     for (int v = NB; v >= 1; --v) {
+      if (v == 3 && c->scr.lnorm) continue;  // a screened wave lies in one tile of 64
       const int64_t wgs = ceil_div(jc * ceil_div(nblk, v), 4), rounds = ceil_div(wgs, slots);
       if (v == NB && rounds > 8) break;
       const double cost = double(rounds) * (v + 0.5);
@@ -1691,7 +1754,7 @@ void launch_ht64(Context *c, const double *cb, int64_t j0, int64_t jc, double *X
   }
   hipLaunchKernelGGL((k_ht64<OT, TQ, NB, false>), grid, dim3(kThreads), 0, c->stream, c->L, c->ldl, c->n, c->n_pad, cb,
                      j0, jc, W, nb, nblocks, X, c->scr, FuseV{});
-  if (c->scr.lnorm) c->x_tiles += jc * W;
+  if (c->scr.lnorm) c->x_tiles += jc * ceil_div(c->n, 64 * c->scr.xw);
 }
 
 // Three quarters only up to four full tiles: past that they save a quarter of one
@@ -1765,12 +1828,20 @@ void ht32_dispatch(Context *c, int ot, const float *L, const float *cb, int64_t 
 }
 
 void syrk_launch64(Context *c, const double *X, int ldc, int64_t jn, const Syrk64Sets &sets, double *kpart,
-                   int chunk) {
+                   int chunk, const ScreenSets &ref, uint8_t *keep) {
   const int T = int(ceil_div(c->n, kT64));
-  hipLaunchKernelGGL(k_syrk64, dim3(unsigned(sets.item0[sets.n])), dim3(kThreads), 0, c->stream, X, c->n, c->n_pad,
-                     ldc, jn, T, sets, kpart, chunk, c->scr);
-  if (c->scr.xn2)
-    for (int d = 0; d < sets.n; ++d) c->k_items += int64_t(sets.nsd[d]) * T + int64_t(sets.nsf[d]) * T * (T - 1) / 2;
+  const dim3 grid(unsigned(sets.item0[sets.n]));
+  if (c->scr.xn2) {
+    const int items = ref.item0[ref.n];
+    hipLaunchKernelGGL(k_keep, dim3(unsigned(ceil_div(items, kThreads / 64))), dim3(kThreads), 0, c->stream,
+                       c->scr.xn2, c->scr.nstrip, jn, ref, c->scr.tau, keep, c->scr.cnt);
+    c->k_items += items;
+    hipLaunchKernelGGL((k_syrk64<true>), grid, dim3(kThreads), 0, c->stream, X, c->n, c->n_pad, ldc, jn, T, sets, kpart,
+                       chunk, ref, keep);
+    return;
+  }
+  hipLaunchKernelGGL((k_syrk64<false>), grid, dim3(kThreads), 0, c->stream, X, c->n, c->n_pad, ldc, jn, T, sets, kpart,
+                     chunk, ref, keep);
 }
 
 void syrk_launch32(Context *c, int tm, int items, const float *X, int ldc, int64_t jn, int ntiles,
@@ -2011,8 +2082,6 @@ int exchange_segments(Context *c, int32_t nk, const int32_t *nocc, const double 
   int64_t work = 0;  // contraction rows per vector over all densities
   for (int d = 0; d < nk; ++d)
     if (nocc[d] > 0) work += opad[size_t(d)];
-  Syrk64Sets sets64{};
-  int64_t kb64 = nchunk64 ? plan_syrk64(c, nk, nocc, off, opad, jc, work, nchunk64, &sets64) : 0;
   int tm = c->tile_syrk ? c->tile_syrk : (n_pad >= 512 && n_pad % 128 == 0 ? 128 : 64);
   if (n_pad % tm) tm = 64;
   const int ntile1 = int(ceil_div(n, tm));
@@ -2028,26 +2097,44 @@ int exchange_segments(Context *c, int32_t nk, const int32_t *nocc, const double 
   // still give every item >= 2048 contraction rows; shorter items lose more to
   // their pipeline fill and store-out than finer balancing gains.
   const int64_t slots = 2 * int64_t(c->ncu);
-  int rounds = 1;
-  while (rounds < 8 && jc * work * ntiles >= int64_t(2048) * slots * (2 * rounds)) rounds *= 2;
-  const int target = c->split_target ? c->split_target : int(slots * rounds);
+  auto slices = [&](int d, int64_t tiles) {
+    int rounds = 1;
+    while (rounds < 8 && jc * work * tiles >= int64_t(2048) * slots * (2 * rounds)) rounds *= 2;
+    const int target = c->split_target ? c->split_target : int(slots * rounds);
+    const int64_t want = int64_t(target) * opad[size_t(d)] / (tiles * std::max<int64_t>(work, 1));
+    return nocc[d] > 0 ? int(std::max<int64_t>(1, std::min<int64_t>(want, jc))) : 0;
+  };
+  // What a screened call leaves out at a given tau depends on the tiles and slices that
+  // the bound is tested over.  They are the same in every precision, whatever the
+  // kernels themselves use: TM x TM, slices counted over the tiles of n_pad.  The FP32
+  // kernel, which tests its own slices, scales tau where it has more of them.
+  ScreenSets ref{};
+  ref.n = nk;
+  ref.strips = tm / 64;
+  ref.ntiles = ntiles;
+  double tau32 = tau;
+  const int pad1 = n_pad / tm;
   for (int d = 0; d < nk; ++d) {
-    const int64_t want = int64_t(target) * opad[size_t(d)] /
-                         (int64_t(ntiles) * std::max<int64_t>(work, 1));
-    sets.nsplit[d] = nocc[d] > 0 ? int(std::max<int64_t>(1, std::min<int64_t>(want, jc))) : 0;
+    sets.nsplit[d] = slices(d, ntiles);
     sets.off[d] = off[size_t(d)];
     sets.opad[d] = std::max(opad[size_t(d)], 1);
     sets.kbase[d] = kb;
     kb += int64_t(sets.nsplit[d]) * nchunk * ntiles * tm * tm;
     sets.item0[d + 1] = sets.item0[d] + sets.nsplit[d] * ntiles;
+    ref.nref[d] = slices(d, int64_t(pad1) * (pad1 + 1) / 2);
+    ref.item0[d + 1] = ref.item0[d] + ref.nref[d] * ntiles;
+    if (ref.nref[d] < sets.nsplit[d]) tau32 = std::min(tau32, tau * ref.nref[d] / sets.nsplit[d]);
   }
   const int items = sets.item0[nk];
+  Syrk64Sets sets64{};
+  const int64_t kb64 = nchunk64 ? plan_syrk64(c, nk, nocc, off, opad, jc, work, nchunk64, &sets64) : 0;
   if ((rc = ensure(c, c->w->kpart, sizeof(double) * size_t(std::max<int64_t>(kb64 + kb, 1))))) return rc;
   double *kpart64 = static_cast<double *>(c->w->kpart.ptr), *kpart = kpart64 + kb64;
 
   // ---- screening set-up (norms of L strips, of the orbital sets, counters)
   const bool screen = tau > 0.0 || thr_x > 0.0;
   const int nstrip = n_pad / 64;
+  uint8_t *keep = nullptr;
   c->k_items = c->x_tiles = 0;
   c->scr = Screen{};
   // the screening state must not outlive this call on any return path: other
@@ -2064,6 +2151,7 @@ int exchange_segments(Context *c, int32_t nk, const int32_t *nocc, const double 
       return rc;
     c->scr.cnt = static_cast<unsigned long long *>(c->scount.ptr);
     c->scr.nstrip = nstrip;
+    c->scr.xw = c->ht_ta == 128 && ot <= 6 ? 2 : 1;
     if (thr_x > 0.0) {
       if (!c->lnorm_valid) {
         if ((rc = ensure(c, c->lnorm, sizeof(double) * size_t(c->nchol) * nstrip))) return rc;
@@ -2085,8 +2173,10 @@ int exchange_segments(Context *c, int32_t nk, const int32_t *nocc, const double 
       c->scr.thr_x = thr_x;
     }
     if (tau > 0.0) {
-      if ((rc = ensure(c, c->w->xn2, sizeof(double) * size_t(nk) * jc * nstrip))) return rc;
-      c->scr.tau = tau;
+      const size_t norms = size_t(nk) * jc * nstrip;
+      if ((rc = ensure(c, c->w->xn2, sizeof(double) * norms + size_t(ref.item0[nk])))) return rc;
+      keep = static_cast<uint8_t *>(static_cast<void *>(static_cast<double *>(c->w->xn2.ptr) + norms));
+      c->scr.tau = use[MJK_PREC_FP64] ? tau : tau32;
     }
   }
 
@@ -2134,7 +2224,7 @@ int exchange_segments(Context *c, int32_t nk, const int32_t *nocc, const double 
       phase_begin(c);
       switch (s.prec) {
         case MJK_PREC_FP64:
-          syrk_launch64(c, static_cast<const double *>(c->w->x.ptr), ldc, jn, sets64, kpart64, int(slot64));
+          syrk_launch64(c, static_cast<const double *>(c->w->x.ptr), ldc, jn, sets64, kpart64, int(slot64), ref, keep);
           break;
         case MJK_PREC_FP32:
           syrk_launch32(c, tm, items, static_cast<const float *>(c->w->x.ptr), ldc, jn, ntiles,

@@ -49,6 +49,7 @@ struct Screen {
   const double *xn2 = nullptr;        // [d][J][strip] squared norms of the chunk's X blocks
   double tau = 0.0;                   // K tile threshold
   int nstrip = 0;                     // n_pad / 64
+  int xw = 1;                         // FP64: strips per half-transform tile
   unsigned long long *cnt = nullptr;  // [K items skipped, X tiles skipped]
 };
 
