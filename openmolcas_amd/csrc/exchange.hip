@@ -1983,15 +1983,17 @@ int ensure_l32(Context *c) {
 // per launch: 1024, 4096, 16384, 32768): n=512 nchol=2048 nocc=64 0.58, 0.61,
 // 0.73, 0.95 ms; n=800 nchol=3600 nocc=150 6.5, 6.1, 5.7, 5.8 ms; n=1200
 // nchol=6000 nocc=150 22.9, 21.4, 22.4, 21.5 ms.
+// most: partial tiles (32 KiB) that a launch may take, but at least one round.
 int64_t plan_syrk64(const Context *c, int32_t nk, const int32_t *nocc, const std::vector<int> &off,
-                    const std::vector<int> &opad, int64_t jc, int64_t work, int64_t nchunk, Syrk64Sets *out) {
+                    const std::vector<int> &opad, int64_t jc, int64_t work, int64_t nchunk, int64_t most,
+                    Syrk64Sets *out) {
   Syrk64Sets &s = *out;
   s.n = nk;
   const int64_t T = ceil_div(c->n, kT64), nf = T * (T - 1) / 2;
   const int64_t units = 16 * nf + 10 * T;  // MFMAs of one step over all tiles
   const int64_t slots = 2 * int64_t(c->ncu), steps = jc * work / 4;
   const int64_t rounds = std::min<int64_t>(64, std::max<int64_t>(1, steps * units / (16 * 4 * 160 * slots)));
-  const int64_t target = c->split_target ? c->split_target : slots * rounds;
+  const int64_t target = c->split_target ? c->split_target : std::max(slots, std::min(slots * rounds, most));
   // Slices of every set for `aim` workgroups; the number there will be (each XCD's
   // eighth of a set's two item lists is rounded up).
   auto slices = [&](int64_t aim) {
@@ -2000,8 +2002,8 @@ int64_t plan_syrk64(const Context *c, int32_t nk, const int32_t *nocc, const std
       if (nocc[d] > 0) {
         const int64_t own = aim * opad[size_t(d)];
         // at least 4 steps per wave, at most one slice per vector
-        const int64_t most = std::max<int64_t>(1, std::min<int64_t>(jc, jc * opad[size_t(d)] / 64));
-        auto clip = [&](int64_t v) { return int(std::max<int64_t>(1, std::min<int64_t>(v, most))); };
+        const int64_t fit = std::max<int64_t>(1, std::min<int64_t>(jc, jc * opad[size_t(d)] / 64));
+        auto clip = [&](int64_t v) { return int(std::max<int64_t>(1, std::min<int64_t>(v, fit))); };
         s.nsf[d] = clip(own * 16 / (work * units));
         s.nsd[d] = clip(own * 10 / (work * units));
       }
@@ -2126,9 +2128,24 @@ int exchange_segments(Context *c, int32_t nk, const int32_t *nocc, const double 
     if (ref.nref[d] < sets.nsplit[d]) tau32 = std::min(tau32, tau * ref.nref[d] / sets.nsplit[d]);
   }
   const int items = sets.item0[nk];
+  // Partial tiles of all FP64 chunks together: a sixteenth of the X budget (so that a
+  // smaller budget, which means more chunks, takes less), and less again where the
+  // device has no room for that.
   Syrk64Sets sets64{};
-  const int64_t kb64 = nchunk64 ? plan_syrk64(c, nk, nocc, off, opad, jc, work, nchunk64, &sets64) : 0;
-  if ((rc = ensure(c, c->w->kpart, sizeof(double) * size_t(std::max<int64_t>(kb64 + kb, 1))))) return rc;
+  int64_t kb64 = 0, &most = c->w->kpart_most;
+  for (int64_t tried = -1;; tried = kb64) {
+    const int64_t bytes = std::min(most, c->x_budget / 16);
+    if (nchunk64)
+      kb64 = plan_syrk64(c, nk, nocc, off, opad, jc, work, nchunk64,
+                         bytes / (int64_t(sizeof(double)) * kSlot64 * nchunk64), &sets64);
+    if (kb64 == tried) break;  // no smaller plan
+    if ((rc = ensure(c, c->w->kpart, sizeof(double) * size_t(std::max<int64_t>(kb64 + kb, 1)))) != MJK_ERR_NOMEM) break;
+    most = bytes / 2;
+  }
+  if (rc) {
+    most = INT64_MAX;
+    return rc;
+  }
   double *kpart64 = static_cast<double *>(c->w->kpart.ptr), *kpart = kpart64 + kb64;
 
   // ---- screening set-up (norms of L strips, of the orbital sets, counters)
