@@ -37,6 +37,7 @@
 // {s : MLk(s) >= sqrt(tau)} (CASSCF), which is what the list kernel forms.
 #include <cmath>
 #include <limits>
+#include <utility>
 
 #include "mjk_internal.h"
 
@@ -45,7 +46,6 @@ namespace {
 
 constexpr int kLkBatch = 25;  // Cho_LK_MaxVecPerBatch (src/fock_util/cho_lk_maxvecperbatch.F90:30)
 constexpr int kLkThreads = 256;
-constexpr int kLkGroup = 64;  // most batches that go through the kernels together
 constexpr int kHtCols = 48;   // columns (J, a) of one half-transform wave
 constexpr int kHtPanel = 1024;  // contraction indices b listed at a time
 
@@ -790,27 +790,43 @@ int lk_exchange(Context *c, int32_t nd, const int32_t *nocc, const double *const
   }
   K.last_batches = int64_t(batches.size());
   // Batches that go through the kernels together: as many as 1 GiB of per-batch
-  // buffers holds (X, masks, partial K), up to kLkGroup.
+  // buffers holds (X, masks, partial K), or the X budget if that is less, up to
+  // kLkGroup; half as many, and again, where the device has no room for them.
   const int nt = int(ceil_div(n, 32)), ntile = nt * (nt + 1) / 2;
   const int64_t ld = 64 * int64_t(D.nq);
   const size_t bx = sizeof(double) * size_t(ktot) * kLkBatch * n_pad, bm = 8 * size_t(D.nq) * ns * ns,
                bp = 8 * size_t(D.nq) * nshp, bk = sizeof(double) * 1024 * size_t(nd) * ntile,
                bs = sizeof(double) * size_t(nshp), bf = sizeof(double) * size_t(ns) * ld,
                bw = 8 * size_t(D.nq) * ns;
-  const int ng = int(std::max<size_t>(  // (batch, word) is one grid dimension
-      1, std::min<size_t>({size_t(kLkGroup), batches.size(), (size_t(1) << 30) / (bx + bm + bp + bk + bs + bf + bw),
+  const size_t room = size_t(std::min<int64_t>(int64_t(1) << 30, c->x_budget));
+  int ng = int(std::max<size_t>(  // (batch, word) is one grid dimension
+      1, std::min<size_t>({size_t(K.group_most), batches.size(), room / (bx + bm + bp + bk + bs + bf + bw),
                            size_t(65535 / D.nq)})));
   const size_t flag_bytes = size_t(ld) * ns;
   if ((rc = ensure(c, K.diag, sizeof(double) * size_t(np))) ||
       (rc = ensure(c, K.dh, sizeof(double) * size_t(n) * n)) ||
       (rc = ensure(c, K.ylk, sizeof(double) * size_t(ktot) * n)) ||
-      (rc = ensure(c, K.svshp, bs * ng)) || (rc = ensure(c, K.sumac, sizeof(double) * size_t(ld) * ns)) ||
-      (rc = ensure(c, K.mlk, sizeof(double) * size_t(ld) * ns)) || (rc = ensure(c, K.faa, bf * ng)) ||
-      (rc = ensure(c, K.listed, flag_bytes)) || (rc = ensure(c, K.keep, bw * ng)) ||
-      (rc = ensure(c, K.mask, bm * ng)) || (rc = ensure(c, K.pairs, bp * ng)) ||
-      (rc = ensure(c, K.kacc, bk * ng)) || (rc = ensure(c, K.x, bx * ng)) ||
+      (rc = ensure(c, K.sumac, sizeof(double) * size_t(ld) * ns)) ||
+      (rc = ensure(c, K.mlk, sizeof(double) * size_t(ld) * ns)) || (rc = ensure(c, K.listed, flag_bytes)) ||
       (rc = ensure(c, K.stats, 3 * sizeof(unsigned long long))))
     return rc;
+  const std::pair<DevBuf *, size_t> per_batch[] = {{&K.svshp, bs}, {&K.faa, bf},  {&K.keep, bw}, {&K.mask, bm},
+                                                   {&K.pairs, bp}, {&K.kacc, bk}, {&K.x, bx}};
+  for (;; ng = K.group_most = ng / 2) {
+    for (const auto &b : per_batch)
+      if ((rc = ensure(c, *b.first, b.second * ng))) break;
+    if (!rc) break;
+    if (rc != MJK_ERR_NOMEM || ng == 1) {
+      K.group_most = kLkGroup;
+      return rc;
+    }
+    int rs;
+    if ((rs = hip_check(c, hipStreamSynchronize(c->stream), "LK buffers"))) return rs;
+    for (const auto &b : per_batch) {  // room for the smaller ones
+      if (b.first->ptr) (void)hipFree(b.first->ptr);
+      *b.first = DevBuf{};
+    }
+  }
   double *diag = static_cast<double *>(K.diag.ptr);
   double *sv = static_cast<double *>(K.svshp.ptr), *sumac = static_cast<double *>(K.sumac.ptr);
   double *mlk = static_cast<double *>(K.mlk.ptr), *faa = static_cast<double *>(K.faa.ptr);

@@ -82,6 +82,8 @@ struct ReducedSet {
   std::vector<int32_t> h_map; // host copy (shell-pair occupancy of the LK screening)
 };
 
+constexpr int kLkGroup = 64;  // most batches of vectors that go through the LK kernels together
+
 // State of the reference-form LK screening that the reference keeps in module
 // globals (use Cholesky: nShell, nBasSh, the diagonal CHO_IODIAG reads, MaxRed;
 // Fock_util_global: Estimate, Update) and the device work buffers of one call.
@@ -99,6 +101,7 @@ struct LKState {
   int64_t present_all_version = -1;
   // per call
   DevBuf diag, dh, ylk, svshp, sumac, mlk, listed, keep, mask, pairs, faa, x, kacc, stats;
+  int group_most = kLkGroup;              // batches that the device had room for
   long long last_stats[3] = {0, 0, 0};    // listed shells, half-transformed shell pairs, K blocks
   int64_t last_batches = 0;
   ~LKState() {
