@@ -669,13 +669,13 @@ void launch_v(Context *c, const double *D, int nd, double *vpart, int nsplit, in
                      c->nchol, D, nd, pchunk, vpart);
 }
 
-// Row segments per workgroup of the J pass: two for one or two densities
-// (8 KiB runs per vector row, measured faster), one otherwise (register budget).
-constexpr int j_width(int ndt) { return ndt <= 2 ? 2 : 1; }
+// Row segments per workgroup of the J pass for one or two densities (8 KiB runs per
+// vector row, measured faster than one).
+constexpr int kJWidth = 2;
 
 template <int ND>
 void launch_j(Context *c, const double *V, int nd, double *jpart, int nsplit, int64_t jchunk) {
-  constexpr int W = j_width(ND), U = 4;
+  constexpr int W = kJWidth, U = 4;
   dim3 grid(unsigned(ceil_div(c->ldl / kSeg, W)), unsigned(nsplit));
   hipLaunchKernelGGL((k_coulomb_j<ND, W, U>), grid, dim3(kThreads), 0, c->stream, c->L, c->ldl,
                      c->nchol, V, nd, jchunk, jpart);
@@ -715,7 +715,6 @@ constexpr size_t kScratchBytes = size_t(64) << 20;  // the fixed buffer of coulo
 
 // Work split and scratch of one Coulomb build (both passes).
 struct CoulombPlan {
-  int nd = 0, ndt = 0;
   bool tile = false;                   // nd >= 3: the MFMA passes
   int group = 0, ngrp = 0;             // one pass: workgroups per group, groups (0: two passes)
   int64_t slice = 0, nparts = 0;       // one pass: pairs per workgroup; parts of V to exchange
@@ -728,13 +727,13 @@ constexpr int kTileVM = 64, kTileVK = 64, kTileU = 4;  // MFMA passes (nd >= 3)
 
 inline size_t piece(size_t bytes) { return size_t(round_up(int64_t(bytes), 256)); }
 
-// Pass 2 split of the streaming J pass for ndt densities: about 1024
-// workgroups of two segments, 2048 of one, at least eight vectors each (a slice
-// of one vector costs more to write and reduce than to read).
-void plan_j_stream(const Context *c, int nd, int ndt, CoulombPlan *p) {
+// Pass 2 split of the streaming J pass: about 1024 workgroups of two segments, at
+// least eight vectors each (a slice of one vector costs more to write and reduce than
+// to read).
+void plan_j_stream(const Context *c, int nd, CoulombPlan *p) {
   const int64_t M = c->nchol, nseg = c->ldl / kSeg;
-  const int64_t nxj = ceil_div(nseg, j_width(ndt));
-  int nsplit2 = int(std::min<int64_t>(std::max<int64_t>(ceil_div(2048 / j_width(ndt), nxj), 1), M));
+  const int64_t nxj = ceil_div(nseg, kJWidth);
+  int nsplit2 = int(std::min<int64_t>(std::max<int64_t>(ceil_div(2048 / kJWidth, nxj), 1), M));
   p->jchunk = std::max<int64_t>(ceil_div(M, nsplit2), 8);
   p->nsplit2 = int(ceil_div(M, p->jchunk));
   p->bytes_jpart = sizeof(double) * size_t(p->nsplit2) * nd * c->ldl;
@@ -778,7 +777,6 @@ bool plan_one(const Context *c, int nd, CoulombPlan *p) {
 CoulombPlan plan_coulomb(const Context *c, int nd) {
   CoulombPlan p;
   const int64_t M = c->nchol, ldl = c->ldl;
-  p.nd = nd;
   p.bytes_d = sizeof(double) * size_t(nd) * ldl;
   p.bytes_v = sizeof(double) * size_t(M) * nd;
   if (plan_one(c, nd, &p)) return p;
@@ -796,14 +794,13 @@ CoulombPlan plan_coulomb(const Context *c, int nd) {
     p.nsplit2 = int(ceil_div(M, p.jchunk));
     p.bytes_jpart = sizeof(double) * size_t(p.nsplit2) * nd * ldl;
   } else {
-    p.ndt = nd <= 1 ? 1 : 2;
     const int jb = 8;
     p.nblk = ceil_div(M, jb);
     const int64_t nseg = ldl / kSeg;
     int nsplit1 = int(std::min<int64_t>(std::max<int64_t>(ceil_div(2048, p.nblk), 1), nseg));
     p.pchunk = ceil_div(nseg, nsplit1) * kSeg;
     p.nsplit1 = int(ceil_div(ldl, p.pchunk));
-    plan_j_stream(c, nd, p.ndt, &p);
+    plan_j_stream(c, nd, &p);
   }
   p.bytes_vpart = sizeof(double) * size_t(p.nsplit1) * M * nd;
   return p;
@@ -831,21 +828,15 @@ int take(Context *c, Scratch &s, DevBuf &ws, size_t bytes, double **out) {
   return MJK_OK;
 }
 
-// Pass 2 for one or two densities (ndt = 1, 2) or their padded counts:
-// J = L V, then the fixed-order reduction of the vector slices into jlt.
+// Pass 2 for one or two densities: J = L V, then the fixed-order reduction of the vector slices into jlt.
 int j_pass(Context *c, Scratch &s, const CoulombPlan &p, int nd, const double *V, double *jlt,
            int64_t ldj) {
   int rc;
   double *jpart;
   if ((rc = take(c, s, c->w->jpart, p.bytes_jpart, &jpart))) return rc;
   phase_begin(c);
-  switch (p.ndt) {
-    case 1: launch_j<1>(c, V, nd, jpart, p.nsplit2, p.jchunk); break;
-    case 2: launch_j<2>(c, V, nd, jpart, p.nsplit2, p.jchunk); break;
-    case 4: launch_j<4>(c, V, nd, jpart, p.nsplit2, p.jchunk); break;
-    case 8: launch_j<8>(c, V, nd, jpart, p.nsplit2, p.jchunk); break;
-    default: launch_j<16>(c, V, nd, jpart, p.nsplit2, p.jchunk); break;
-  }
+  if (nd == 1) launch_j<1>(c, V, nd, jpart, p.nsplit2, p.jchunk);
+  else launch_j<2>(c, V, nd, jpart, p.nsplit2, p.jchunk);
   phase_end(c, MJK_PHASE_COULOMB_J);
   phase_begin(c);
   hipLaunchKernelGGL(k_reduce_j, dim3(unsigned(ceil_div(c->np, 64)), unsigned(nd)), dim3(256), 0,
@@ -931,10 +922,8 @@ int coulomb_run(Context *c, Scratch &s, int32_t nd, const double *dlt, int64_t l
 
   // ---- pass 1: V = L^T D
   phase_begin(c);
-  switch (p.ndt) {
-    case 1: launch_v<8, 1>(c, Dp, nd, vpart, p.nsplit1, p.pchunk); break;
-    default: launch_v<8, 2>(c, Dp, nd, vpart, p.nsplit1, p.pchunk); break;
-  }
+  if (nd == 1) launch_v<8, 1>(c, Dp, nd, vpart, p.nsplit1, p.pchunk);
+  else launch_v<8, 2>(c, Dp, nd, vpart, p.nsplit1, p.pchunk);
   phase_end(c, MJK_PHASE_COULOMB_V);
   phase_begin(c);
   hipLaunchKernelGGL(k_reduce_v, dim3(unsigned(ceil_div(M * nd, 256))), dim3(256), 0, c->stream,
@@ -1043,8 +1032,7 @@ int coulomb_exchange_run(Context *c, const double *dlt, int64_t ldd, double *jlt
                      M, 1, ntile, V);
   phase_end(c, MJK_PHASE_REDUCE);
   CoulombPlan p;
-  p.ndt = 1;
-  plan_j_stream(c, 1, 1, &p);
+  plan_j_stream(c, 1, &p);
   Scratch s;  // the context's workspaces
   return j_pass(c, s, p, 1, V, jlt, ldj);
 }

@@ -30,28 +30,11 @@ namespace {
 
 constexpr int kThreads = 256;
 
-// Precision traits of the exchange kernels.  row(lane, r) is the row of the
-// 16x16 result held in register r of `lane` (column = lane % 16); the FP64 and
-// FP32 16x16x4 instructions of gfx950 differ here.  The A operand of lane l is
-// A[l%16][l/16], the B operand B[l/16][l%16], for both.
-struct F64 {
-  typedef double T;
-  typedef v4d Acc;
-  static constexpr bool kFlush = false;  // accumulate in FP64 throughout
-  __device__ static Acc mma(T a, T b, Acc c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  __device__ static int row(int lane, int r) { return 4 * r + (lane >> 4); }
-};
-struct F32 {
-  typedef float T;
-  typedef v4f Acc;
-  static constexpr bool kFlush = true;  // FP32 partial sums folded into FP64
-  __device__ static Acc mma(T a, T b, Acc c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  __device__ static int row(int lane, int r) { return 4 * (lane >> 4) + r; }
-};
+// 16x16x4 products: lane l holds A[l%16][l/16] and B[l/16][l%16].  Register r of the
+// result is row 4 r + l/16 in FP64, row32(l, r) in FP32, column l%16.
+__device__ inline v4d mma64(double a, double b, v4d c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+__device__ inline v4f mma32(float a, float b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+__device__ inline int row32(int lane, int r) { return 4 * (lane >> 4) + r; }
 
 // FP32 SYRK partial sums are folded into FP64 registers every kFlushRows
 // contraction rows, so no FP32 sum runs over more than kFlushRows products.
@@ -157,13 +140,13 @@ __global__ void k_to_f32(const double *__restrict__ src, float *__restrict__ dst
 // (TA/64 MFMA column tiles) and all OT row tiles; each orbital fragment read
 // from LDS feeds the MFMAs of all NJ vectors.  The next b-chunk is fetched
 // into registers while the current one is multiplied out of LDS.
-template <class P, int OT, int TA, int BK, int NJ>
+template <int OT, int TA, int BK, int NJ>
 __global__ __launch_bounds__(kThreads) void k_ht(
-    const typename P::T *__restrict__ L, int64_t ldl, int n, int n_pad,
-    const typename P::T *__restrict__ Cb, int64_t j0, int64_t jc, int ntile_a, int64_t nblocks,
-    typename P::T *__restrict__ X, const Screen sc) {
-  typedef typename P::T T;
-  typedef typename P::Acc Acc;
+    const float *__restrict__ L, int64_t ldl, int n, int n_pad,
+    const float *__restrict__ Cb, int64_t j0, int64_t jc, int ntile_a, int64_t nblocks,
+    float *__restrict__ X, const Screen sc) {
+  typedef float T;
+  typedef v4f Acc;
   constexpr int LDC = 16 * OT;
   // Wave layout.  Narrow banks: wave w owns AO columns w*TA/4 .. (w+1)*TA/4-1
   // and all OT row tiles.  Wide banks (one vector, even OT >= 6, TA = 64): 2 x 2
@@ -344,7 +327,7 @@ __global__ __launch_bounds__(kThreads) void k_ht(
 #pragma unroll
           for (int t = 0; t < OTW; ++t)
 #pragma unroll
-            for (int j = 0; j < NB; ++j) acc[q][t][j] = P::mma(af[qq][t], bf[qq][q][j], acc[q][t][j]);
+            for (int j = 0; j < NB; ++j) acc[q][t][j] = mma32(af[qq][t], bf[qq][q][j], acc[q][t][j]);
       }
       if (c + 1 < nch) stash((c + 1) * BK, cur ^ 1);
       if (c + 2 < nch) fetch((c + 2) * BK);
@@ -362,7 +345,7 @@ __global__ __launch_bounds__(kThreads) void k_ht(
       for (int t = 0; t < OTW; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          xj[int64_t(16 * (t0 + t) + P::row(lane, r)) * n_pad + a] = acc[q][t][j][r];
+          xj[int64_t(16 * (t0 + t) + row32(lane, r)) * n_pad + a] = acc[q][t][j][r];
     }
   }
 }
@@ -506,12 +489,12 @@ __device__ __forceinline__ void ht64_wave(const double *__restrict__ Lj, int n, 
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int j = 0; j < NBV; ++j) acc[2 * i + h][j] = F64::mma(cf[i][h], x[j], acc[2 * i + h][j]);
+        for (int j = 0; j < NBV; ++j) acc[2 * i + h][j] = mma64(cf[i][h], x[j], acc[2 * i + h][j]);
       if (s < 3) load_cp(buf, s + 1, i);
     }
     if constexpr (OT % 2 == 1) {
 #pragma unroll
-      for (int j = 0; j < NBV; ++j) acc[OT - 1][j] = F64::mma(co, x[j], acc[OT - 1][j]);
+      for (int j = 0; j < NBV; ++j) acc[OT - 1][j] = mma64(co, x[j], acc[OT - 1][j]);
       if (s < 3) load_co(buf, s + 1);
     }
     if constexpr (TQ > 0) {
@@ -769,12 +752,12 @@ __global__ __launch_bounds__(kThreads, 2) void k_ht64(const double *__restrict__
 // kpart[(s*ntiles + t)*TM*TM + al*TM + bl] (+)= sum_f X[f][A*TM+al] X[f][B*TM+bl]
 // On diagonal tiles (A == B) only one operand is staged and the MFMA tiles
 // strictly above the diagonal are skipped (those entries are never read).
-template <class P, int TM, int BKF>
+template <int TM, int BKF>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void k_syrk(
-    const typename P::T *__restrict__ X, int n_pad, int ldc, int64_t jc, int ntiles,
+    const float *__restrict__ X, int n_pad, int ldc, int64_t jc, int ntiles,
     const SyrkSets sets, double *__restrict__ kpart_all, int chunk, const Screen sc) {
-  typedef typename P::T T;
-  typedef typename P::Acc Acc;
+  typedef float T;
+  typedef v4f Acc;
   constexpr int WT = TM / 2;
   constexpr int MT = WT / 16;
   constexpr int VW = 16 / int(sizeof(T));  // elements per 16-byte load
@@ -824,30 +807,26 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   }
 
   Acc acc[MT][MT];
-  double accd[P::kFlush ? MT : 1][P::kFlush ? MT : 1][4];
+  double accd[MT][MT][4];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < MT; ++j) acc[i][j] = Acc{0, 0, 0, 0};
-  if constexpr (P::kFlush) {
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) accd[i][j][r] = 0.0;
+  auto flush = [&]() {
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-      for (int j = 0; j < MT; ++j)
+      for (int j = 0; j < MT; ++j) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) accd[i][j][r] = 0.0;
-  }
-  auto flush = [&]() {
-    if constexpr (P::kFlush) {
-#pragma unroll
-      for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < MT; ++j) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) accd[i][j][r] += double(acc[i][j][r]);
-          acc[i][j] = Acc{0, 0, 0, 0};
-        }
-    }
+        for (int r = 0; r < 4; ++r) accd[i][j][r] += double(acc[i][j][r]);
+        acc[i][j] = Acc{0, 0, 0, 0};
+      }
   };
 
   VT ra[PN], rb[PN];
@@ -881,10 +860,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
   // kr + 1 of TM floats, a multiple of 32 apart; column c of row f sits at
   // c ^ 16 (f & 1) so the two rows fall in different bank halves (the 16-byte
   // stores keep their four columns together)
-  auto spos = [](int f, int c) {
-    if constexpr (sizeof(T) == 4) return f * TM + (c ^ ((f & 1) << 4));
-    else return f * TM + c;
-  };
+  auto spos = [](int f, int c) { return f * TM + (c ^ ((f & 1) << 4)); };
   auto stash = [&](int buf) {
 #pragma unroll
     for (int i = 0; i < PN; ++i)
@@ -932,15 +908,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
           for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int j = 0; j < MT; ++j)
-              if (!LO || i >= j) acc[i][j] = P::mma(af[q][i], bf[q][j], acc[i][j]);
+              if (!LO || i >= j) acc[i][j] = mma32(af[q][i], bf[q][j], acc[i][j]);
         }
       };
       if (!diag || wm > wn) steps(std::false_type{});
       else steps(std::true_type{});
     }
-    if constexpr (P::kFlush) {
-      if (((c + 1) * BKF) % kFlushRows == 0) flush();
-    }
+    if (((c + 1) * BKF) % kFlushRows == 0) flush();
     if (c + 1 < nch) stash(cur ^ 1);
     if (c + 2 < nch) fetch((c + 2) * BKF);
     __syncthreads();
@@ -952,12 +926,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) v
     for (int j = 0; j < MT; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int al = wm * WT + i * 16 + P::row(lane, r);
+        const int al = wm * WT + i * 16 + row32(lane, r);
         const int bl = wn * WT + j * 16 + (lane & 15);
-        double v;
-        if constexpr (P::kFlush) v = accd[i][j][r];
-        else v = acc[i][j][r];
-        kp[al * TM + bl] = v;
+        kp[al * TM + bl] = accd[i][j][r];
       }
 }
 
@@ -1044,7 +1015,7 @@ __device__ __forceinline__ void syrk64_tile(const double *__restrict__ X, int n_
             double bv;
             if constexpr (DG) bv = a[j >> 1][j & 1];
             else bv = b[j >> 1][j & 1];
-            acc[i][j] = F64::mma(a[i >> 1][i & 1], bv, acc[i][j]);
+            acc[i][j] = mma64(a[i >> 1][i & 1], bv, acc[i][j]);
           }
     };
 #pragma unroll
@@ -1706,7 +1677,7 @@ void launch_ht(Context *c, const float *L, const float *cb, int64_t j0, int64_t 
   const int ntile_a = c->n_pad / TA;
   const int64_t nblocks = ceil_div(jc, NJ) * ntile_a;
   const int64_t grid = round_up(nblocks, 8);
-  hipLaunchKernelGGL((k_ht<F32, OT, TA, BK, NJ>), dim3(unsigned(grid)), dim3(kThreads), 0,
+  hipLaunchKernelGGL((k_ht<OT, TA, BK, NJ>), dim3(unsigned(grid)), dim3(kThreads), 0,
                      c->stream, L, c->ldl, c->n, c->n_pad, cb, j0, jc, ntile_a, nblocks, X, c->scr);
   if (c->scr.lnorm) c->x_tiles += jc * ntile_a;
 }
@@ -1847,10 +1818,10 @@ void syrk_launch64(Context *c, const double *X, int ldc, int64_t jn, const Syrk6
 void syrk_launch32(Context *c, int tm, int items, const float *X, int ldc, int64_t jn, int ntiles,
                    const SyrkSets &sets, double *kpart, int chunk) {
   if (tm == 128)
-    hipLaunchKernelGGL((k_syrk<F32, 128, 16>), dim3(unsigned(items)), dim3(kThreads), 0, c->stream, X,
+    hipLaunchKernelGGL((k_syrk<128, 16>), dim3(unsigned(items)), dim3(kThreads), 0, c->stream, X,
                        c->n_pad, ldc, jn, ntiles, sets, kpart, chunk, c->scr);
   else
-    hipLaunchKernelGGL((k_syrk<F32, 64, 32>), dim3(unsigned(items)), dim3(kThreads), 0, c->stream, X,
+    hipLaunchKernelGGL((k_syrk<64, 32>), dim3(unsigned(items)), dim3(kThreads), 0, c->stream, X,
                        c->n_pad, ldc, jn, ntiles, sets, kpart, chunk, c->scr);
   if (c->scr.xn2) c->k_items += items;
 }
