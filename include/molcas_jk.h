@@ -423,8 +423,8 @@ int mjk_exchange(mjk_context *ctx, int32_t nk, const int32_t *nocc,
  * device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid it).  No counterpart in the reference.  The same
  * results as mjk_coulomb, bit for bit; one or two densities read the vectors
- * twice where mjk_coulomb reads them once (n=512, 1000 vectors: 347 against
- * 195 us), because the scratch is shared and so nothing may be waited for in
+ * twice where mjk_coulomb reads them once (n=512, 1000 vectors: 326 against
+ * 197 us), because the scratch is shared and so nothing may be waited for in
  * it on the device.  Every scratch buffer (the padded density, the
  * partial sums of V and J, and V when v_out is NULL) lives in one fixed
  * 64 MiB device array per GPU, set up with the library and held until the

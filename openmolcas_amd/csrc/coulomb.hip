@@ -253,9 +253,12 @@ __device__ inline int one_rows(int64_t len, int w) {
 // How the members of a group meet, one per group, zero at the start.
 struct OneGate {
   int arrived;  // members that have started; kOneApart set: the group works apart
-  int parts, done, sums;  // apart: slices whose parts were begun, ended; slices begun for J
+  int parts, done, sums;  // apart: runs of parts begun, ended; slices begun for J
 };
 constexpr int kOneApart = 1 << 30;
+// Apart, a slice's parts go in up to 16 runs of vectors, at least 16 vectors each:
+// whoever finds no more of them waits for the last ones.
+constexpr int kOneRuns = 16, kOneRunLeast = 16;
 
 // Whether all G members of a group run at the same time, the same answer for each: a
 // member waits for the others for `looks` looks (about 1 us each).
@@ -285,15 +288,18 @@ __device__ inline int one_take(int *n) {
 //
 // Waiting for another member is safe only while it runs, and other streams may hold
 // part of the GPU.  A group whose members have not all started after `looks` looks
-// works apart: whoever of it runs takes slices and sums their parts of every V_J
-// (nothing is waited for), then, all parts being there, takes slices again for J.
-// That is two reads of the vectors, with any number of members, and the same bits.
-// Contexts at once on streams of their own, us, two-pass kernels -> this one: n=301,
-// 1200 vectors, J on four 572 -> 516, J and K on four 2186 -> 1629; n=701, 700 vectors
-// J on two 853 -> 626, on four 1754 -> 1881, J and K on four 9552 -> 7925.  With 4096
-// looks 4 x J at n=900 took 23000; 16 or 8 looks: +2 to +11% at n=301, none gained.
+// works apart: whoever of it runs takes runs of vectors of a slice and sums its parts of
+// their V (nothing is waited for), then, all parts being there, takes slices for J.  That
+// is two reads of the vectors, with any number of members, and the same bits.
+// Contexts at once on streams of their own, J alone, us, two-pass kernels -> this one, on
+// two and on four streams: n=301, 1200 vectors 286 -> 172, 584 -> 379; n=512, 1000 668 ->
+// 445, 1329 -> 1305; n=701, 700 876 -> 591, 1721 -> 1712; n=900, 700 1424 -> 1254, 2771 ->
+// 2931; n=1100, 600 1821 -> 1164, 3536 -> 3633.  J and K on four: n=301 2186 -> 1629,
+// n=701 9552 -> 7925.  (Apart, whole slices at a time in the loop that reads once, with two vectors
+// on their way: n=900 on four streams 3574, n=1100 4413.)  With 4096 looks 4 x J at
+// n=900 took 23000; 16 or 8 looks: up to +29% at n=301, none gained.
 //
-// step kParts, then kSums in a second launch: every member does that for its own slice
+// STEP kParts, then kSums in a second launch: every member does that for its own slice
 // and waits for nobody, whatever other calls write to the exchange and the gates.
 //
 // waits: looks (about 1 us each) at what a running member owes, after which V is NaN and
@@ -301,190 +307,321 @@ __device__ inline int one_take(int *n) {
 // writes to this one's workspace meanwhile (contexts that share one, or one context,
 // on two streams at once) can keep it away for ever.
 enum OneStep { kTogether, kParts, kSums };
-template <int ND, int ROWS>
-__global__ __launch_bounds__((kOneWaves + 1) * kWave) void k_coulomb_one(
-    const double *__restrict__ L, int64_t ldl, int64_t M, const double *__restrict__ D, int ngrp, int G, int64_t slice,
-    int looks, int waits, OneStep step_only, OneGate *gate, double *part, double *__restrict__ V, double *__restrict__ jpart) {
-  constexpr int R = kOneRing, LAG = R - 3;
-  __shared__ __attribute__((aligned(16))) v2d sD[ND][ROWS * kOneWaves * kWave];
-  __shared__ double sP[R][ND][kOneWaves];
-  __shared__ double sV[2][ND];
-  __shared__ int sTask;  // slice to work on next; < 0: none
-  const int lane = threadIdx.x & (kWave - 1), w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int grp = blockIdx.x / G;
-  const int T = int((M - grp + ngrp - 1) / ngrp);
-  const int steps = (T + LAG + R - 1) / R * R;
-  int mem = blockIdx.x % G, mode = step_only;
-  if (step_only) waits = 0;
 
-  for (;;) {
-    const int64_t p0 = min(mem * slice, ldl), len = min(slice, ldl - p0);
-    if (w == kOneWaves) {  // ---- the wave that exchanges V
-      if (mode == kTogether) {
-        const bool one = G == 1 || __builtin_amdgcn_readfirstlane(lane == 0 ? one_together(gate + grp, G, looks) : 0);
-        if (lane == 0) sTask = one ? mem : -1;
-      }
-      lds_barrier();  // D is there
-      lds_barrier();  // parts of the first vector
-      if (mode != kTogether || __builtin_amdgcn_readfirstlane(sTask) >= 0) {
-        for (int s = 0; s < steps; ++s) {
-          double v[ND];
-          if (G > 1 && s < T && lane < ND) {
-            double mine = sum_waves(sP[s % R][lane]);
-            if (__builtin_bit_cast(int64_t, mine) == kOneEmpty) mine = __builtin_nan("");
-            __hip_atomic_store(part + (grp + int64_t(s) * ngrp) * G * ND + mem * ND + lane, mine, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-          }
-          const int64_t J = grp + int64_t(s - LAG) * ngrp;
-          const bool have = mode != kParts && s >= LAG && s - LAG < T;
+// The vectors that a workgroup works on: T of its group's from the one with index J0 on.
+struct OneRun {
+  int64_t J0, p0, len;  // first pair and pairs of the slice
+  int ngrp, T;
+};
+
+using OneRow = const __attribute__((address_space(1))) v2d *;
+
+// Rows of this wave of vector s of a run; zeros past its end.
+template <int ROWS>
+__device__ __forceinline__ void one_fetch(const double *__restrict__ L, int64_t ldl, const OneRun &r, int s, int nv, int w,
+                                          int lane, v2d (&x)[ROWS]) {
+  const uint64_t row = reinterpret_cast<uint64_t>(L + (r.J0 + int64_t(s) * r.ngrp) * ldl + r.p0 + 2 * kWave * w);
+  const int have = s < r.T ? nv : 0;
 #pragma unroll
-          for (int d = 0; d < ND; ++d) v[d] = 0.0;
-          if (have && G == 1) {
+  for (int i = 0; i < ROWS; ++i)
+    x[i] = __builtin_nontemporal_load(
+        reinterpret_cast<OneRow>(i < have ? row + i * (kOneRow * sizeof(double)) : reinterpret_cast<uint64_t>(one_zeros)) + lane);
+}
+
+// This wave's rows of D to LDS.
+template <int ND, int ROWS>
+__device__ __forceinline__ void one_dens(const double *__restrict__ D, int64_t ldl, const OneRun &r, int nv, int w, int lane,
+                                         v2d (*sD)[ROWS * kOneWaves * kWave]) {
 #pragma unroll
-            for (int d = 0; d < ND; ++d) v[d] = sum_waves(sP[(s - LAG) % R][d]);
-          }
-          if (have && G > 1) {
-            const double *row = part + J * G * ND;
-            const int cnt = G * ND;  // <= 256
-            double x[4];
-            for (int left = waits;; --left) {  // the others run: their parts come (kSums alone: they are there)
-              bool ok = true;
-              auto look = [&](int k) {
-                return __hip_atomic_load(row + min(lane + 64 * k, cnt - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-              };
-              x[0] = look(0);
-              x[1] = x[2] = x[3] = 0.0;
-              if (cnt > 128) {
-                x[1] = look(1), x[2] = look(2), x[3] = look(3);
-              } else if (cnt > 64) {
-                x[1] = look(1);
-              }
+  for (int d = 0; d < ND; ++d)
 #pragma unroll
-              for (int k = 0; k < 4; ++k) {
-                ok = ok && __builtin_bit_cast(int64_t, x[k]) != kOneEmpty;
-                if (lane + 64 * k >= cnt) x[k] = 0.0;
-              }
-              if (__all(ok)) break;
-              if (left <= 0) {
-                waits = 0;
-                break;
-              }
-              __builtin_amdgcn_s_sleep(1);
-            }
-            const double y = (x[0] + x[1]) + (x[2] + x[3]);
-            if constexpr (ND == 1) {
-              v[0] = wave_sum(y);
-            } else {  // entry 2m + d: even lanes density 0, odd lanes density 1
-              v[0] = wave_sum(lane & 1 ? 0.0 : y);
-              v[1] = wave_sum(lane & 1 ? y : 0.0);
-            }
-          }
-          if (lane == 0) {
+    for (int i = 0; i < ROWS; ++i)
+      sD[d][(i * kOneWaves + w) * kWave + lane] =
+          reinterpret_cast<OneRow>(i < nv ? reinterpret_cast<uint64_t>(D + d * ldl + r.p0 + i * kOneRow + 2 * kWave * w)
+                                          : reinterpret_cast<uint64_t>(one_zeros))[lane];
+}
+
+template <int ND, int ROWS>
+__device__ __forceinline__ void one_add(const v2d (&x)[ROWS], const double *sV, v2d (&acc)[ND][ROWS]) {
 #pragma unroll
-            for (int d = 0; d < ND; ++d) sV[s & 1][d] = v[d];
-            if (mem == 0 && have) {
+  for (int d = 0; d < ND; ++d) {
+    const double v = sV[d];
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+      acc[d][i].x = __builtin_fma(x[i].x, v, acc[d][i].x);
+      acc[d][i].y = __builtin_fma(x[i].y, v, acc[d][i].y);
+      asm volatile("" : "+v"(acc[d][i]));  // summed here, not where it is next read
+    }
+  }
+}
+
+template <int ND, int ROWS>
+__device__ __forceinline__ void one_store(const v2d (&acc)[ND][ROWS], int64_t ldl, int grp, const OneRun &r, int nv, int w,
+                                          int lane, double *__restrict__ jpart) {
+#pragma unroll
+  for (int d = 0; d < ND; ++d)
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i)
+      if (i < nv)
+        *reinterpret_cast<v2d *>(jpart + (int64_t(grp) * ND + d) * ldl + r.p0 + i * kOneRow + 2 * (kWave * w + lane)) = acc[d][i];
+}
+
+// A member's part of V_J(d) to the exchange.
+__device__ __forceinline__ void one_publish(const double *sP, double *part) {
+  double mine = sum_waves(sP);
+  if (__builtin_bit_cast(int64_t, mine) == kOneEmpty) mine = __builtin_nan("");
+  __hip_atomic_store(part, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Parts of V_J of all members (cnt = G ND <= 256 of them), looked for up to `waits` more
+// times; waits becomes 0 when they do not come, and V_J is NaN.
+__device__ __forceinline__ double one_collect(const double *row, int cnt, int lane, int &waits) {
+  double x[4];
+  for (int left = waits;; --left) {
+    bool ok = true;
+    auto look = [&](int k) {
+      return __hip_atomic_load(row + min(lane + 64 * k, cnt - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    x[0] = look(0);
+    x[1] = x[2] = x[3] = 0.0;
+    if (cnt > 128) {
+      x[1] = look(1), x[2] = look(2), x[3] = look(3);
+    } else if (cnt > 64) {
+      x[1] = look(1);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      ok = ok && __builtin_bit_cast(int64_t, x[k]) != kOneEmpty;
+      if (lane + 64 * k >= cnt) x[k] = 0.0;
+    }
+    if (__all(ok)) break;
+    if (left <= 0) {
+      waits = 0;
+      break;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+  return (x[0] + x[1]) + (x[2] + x[3]);
+}
+
+// V_J from the collected parts: entry 2 m + d, even lanes density 0, odd lanes density 1.
+template <int ND>
+__device__ __forceinline__ void one_total(double y, int lane, double (&v)[ND]) {
+  if constexpr (ND == 1) {
+    v[0] = wave_sum(y);
+  } else {
+    v[0] = wave_sum(lane & 1 ? 0.0 : y);
+    v[1] = wave_sum(lane & 1 ? y : 0.0);
+  }
+}
+
+// One slice with nothing to wait for: its parts of V of a run of vectors, or its J with
+// all parts there.  Three vectors on their way while one is worked on and one barrier for
+// four of them, which the one-read loop has no registers and no time for.
+template <int ND, int ROWS, bool SUMS>
+__device__ __forceinline__ void one_slice(const double *__restrict__ L, int64_t ldl, const double *__restrict__ D, int grp,
+                                          int G, int mem, const OneRun &r, int &waits, double *part,
+                                          double *__restrict__ V, double *__restrict__ jpart, int w, int lane,
+                                          v2d (*sD)[ROWS * kOneWaves * kWave], double (*sP)[4][ND][kOneWaves],
+                                          double (*sV)[4][ND]) {
+  const int trips = (r.T + 3) / 4;
+  if (w == kOneWaves) {
+    if constexpr (SUMS) {
+      auto values = [&](int q) {  // V of trip q
+        for (int u = 0; u < 4; ++u) {
+          const int s = 4 * q + u;
+          double v[ND] = {};
+          if (s < r.T) {
+            const int64_t J = r.J0 + int64_t(s) * r.ngrp;
+            one_total<ND>(one_collect(part + J * G * ND, G * ND, lane, waits), lane, v);
+            if (mem == 0 && lane == 0) {
 #pragma unroll
               for (int d = 0; d < ND; ++d) V[J * ND + d] = v[d];
             }
           }
-          lds_barrier();
-        }
-      }
-    } else {  // ---- the streaming waves
-      const int t = threadIdx.x;
-      const int nv = __builtin_amdgcn_readfirstlane(one_rows(len, w));
-      using Row = const __attribute__((address_space(1))) v2d *;
-      v2d buf[R][ROWS], acc[ND][ROWS];
-      auto fetch = [&](int s, v2d(&x)[ROWS]) {
-        const uint64_t row = reinterpret_cast<uint64_t>(L + (grp + int64_t(s) * ngrp) * ldl + p0 + 2 * kWave * w);
-        const int have = s < T ? nv : 0;
+          if (lane == 0) {
 #pragma unroll
-        for (int i = 0; i < ROWS; ++i)
-          x[i] = __builtin_nontemporal_load(
-              reinterpret_cast<Row>(i < have ? row + i * (kOneRow * sizeof(double)) : reinterpret_cast<uint64_t>(one_zeros)) + lane);
-      };
-#pragma unroll
-      for (int r = 0; r < R; ++r) fetch(r < 2 ? r : T, buf[r]);
-#pragma unroll
-      for (int d = 0; d < ND; ++d)
-#pragma unroll
-        for (int i = 0; i < ROWS; ++i) {
-          sD[d][i * (kOneWaves * kWave) + t] =
-              reinterpret_cast<Row>(i < nv ? reinterpret_cast<uint64_t>(D + d * ldl + p0 + i * kOneRow + 2 * kWave * w)
-                                           : reinterpret_cast<uint64_t>(one_zeros))[lane];
-          acc[d][i] = v2d{0.0, 0.0};
-        }
-      lds_barrier();
-      auto parts = [&](int s, const v2d(&x)[ROWS]) {
-#pragma unroll
-        for (int d = 0; d < ND; ++d) sP[s % R][d][w] = one_dot<ROWS>(x, sD[d], t);  // the same in every lane
-      };
-      parts(0, buf[0]);
-      lds_barrier();
-      // step s: vector s + 2 on its way, parts of s + 1, V of s - LAG
-      auto step = [&](int s, v2d(&cur)[ROWS], v2d(&nxt)[ROWS], v2d(&far)[ROWS]) {
-        __builtin_amdgcn_sched_barrier(0);  // `far` has been used before it is loaded again
-        fetch(s + 2, far);
-        __builtin_amdgcn_sched_barrier(0);
-        parts(s + 1, nxt);
-        lds_barrier();
-#pragma unroll
-        for (int d = 0; d < ND; ++d) {
-          const double v = sV[s & 1][d];
-#pragma unroll
-          for (int i = 0; i < ROWS; ++i) {
-            acc[d][i].x = __builtin_fma(cur[i].x, v, acc[d][i].x);
-            acc[d][i].y = __builtin_fma(cur[i].y, v, acc[d][i].y);
-            asm volatile("" : "+v"(acc[d][i]));  // summed here, not where it is next read
+            for (int d = 0; d < ND; ++d) sV[q & 1][u][d] = v[d];
           }
         }
       };
-      if (mode != kTogether || __builtin_amdgcn_readfirstlane(sTask) >= 0) {
-        for (int s = 0; s < steps; s += R) {  // steps of zeros at both ends
-#pragma unroll
-          for (int u = 0; u < R; ++u) step(s + u, buf[(u + 3) % R], buf[(u + 1) % R], buf[(u + 2) % R]);
-        }
-        if (mode != kParts) {
-#pragma unroll
-          for (int d = 0; d < ND; ++d)
-#pragma unroll
-            for (int i = 0; i < ROWS; ++i)
-              if (i < nv)
-                *reinterpret_cast<v2d *>(jpart + (int64_t(grp) * ND + d) * ldl + p0 + i * kOneRow + 2 * t) = acc[d][i];
-        }
+      values(0);
+      lds_barrier();
+      for (int q = 0; q < trips; ++q) {
+        values(q + 1);
+        lds_barrier();
+      }
+    } else {
+      lds_barrier();
+      for (int q = 0; q < trips; ++q) {
+        lds_barrier();
+        const int u = lane / ND, d = lane % ND, s = 4 * q + u;
+        if (lane < 4 * ND && s < r.T)
+          one_publish(sP[q & 1][u][d], part + ((r.J0 + int64_t(s) * r.ngrp) * G + mem) * ND + d);
       }
     }
-    if (step_only) return;
-    // ---- apart: the next slice
-    if (mode == kTogether && __builtin_amdgcn_readfirstlane(sTask) >= 0) return;
-    lds_barrier();  // everybody has read sTask
-    if (w == kOneWaves) {
-      int next = -1, m = mode;
-      if (lane == 0) {
-        OneGate *g = gate + grp;
-        if (m == kParts) one_take(&g->done);
-        if (m != kSums) {
-          m = kParts;
-          next = one_take(&g->parts);
-          if (next >= G) {
-            // slices not done are being worked on, and nothing is waited for there
-            for (int left = waits; left > 0; --left) {
-              if (__hip_atomic_load(&g->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= G) break;
-              __builtin_amdgcn_s_sleep(8);
-            }
-            m = kSums;
+    return;
+  }
+  const int nv = __builtin_amdgcn_readfirstlane(one_rows(r.len, w));
+  v2d buf[4][ROWS], acc[ND][ROWS];
+#pragma unroll
+  for (int u = 0; u < 3; ++u) one_fetch<ROWS>(L, ldl, r, u, nv, w, lane, buf[u]);
+  if constexpr (SUMS) {
+#pragma unroll
+    for (int d = 0; d < ND; ++d)
+#pragma unroll
+      for (int i = 0; i < ROWS; ++i) acc[d][i] = v2d{0.0, 0.0};
+  } else {
+    one_dens<ND, ROWS>(D, ldl, r, nv, w, lane, sD);
+  }
+  lds_barrier();
+  for (int q = 0; q < trips; ++q) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      __builtin_amdgcn_sched_barrier(0);  // the buffer has been used before it is loaded again
+      one_fetch<ROWS>(L, ldl, r, 4 * q + u + 3, nv, w, lane, buf[(u + 3) % 4]);
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (SUMS) {
+        one_add<ND, ROWS>(buf[u], sV[q & 1][u], acc);
+      } else {
+#pragma unroll
+        for (int d = 0; d < ND; ++d) sP[q & 1][u][d][w] = one_dot<ROWS>(buf[u], sD[d], kWave * w + lane);
+      }
+    }
+    lds_barrier();
+  }
+  if constexpr (SUMS) one_store<ND, ROWS>(acc, ldl, grp, r, nv, w, lane, jpart);
+}
+
+template <int ND, int ROWS, OneStep STEP>
+__global__ __launch_bounds__((kOneWaves + 1) * kWave) void k_coulomb_one(
+    const double *__restrict__ L, int64_t ldl, int64_t M, const double *__restrict__ D, int ngrp, int G, int64_t slice,
+    int looks, int waits, OneGate *gate, double *part, double *__restrict__ V, double *__restrict__ jpart) {
+  constexpr int R = kOneRing, LAG = R - 3;
+  __shared__ __attribute__((aligned(16))) v2d sD[ND][ROWS * kOneWaves * kWave];
+  __shared__ double sP[2][4][ND][kOneWaves];
+  __shared__ double sV[2][4][ND];
+  __shared__ int sTask;  // together: whether; apart: what to do next, < 0: nothing
+  const int lane = threadIdx.x & (kWave - 1), w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int grp = blockIdx.x / G, mem = blockIdx.x % G;
+  const int T = int((M - grp + ngrp - 1) / ngrp);  // vectors of the group
+  auto run = [&](int m, int s0, int cnt) {
+    OneRun r;
+    r.J0 = grp + int64_t(s0) * ngrp;
+    r.p0 = min(m * slice, ldl);
+    r.len = min(slice, ldl - r.p0);
+    r.ngrp = ngrp;
+    r.T = cnt;
+    return r;
+  };
+  const OneRun r = run(mem, 0, T);
+  if constexpr (STEP != kTogether) {
+    int none = 0;
+    one_slice<ND, ROWS, STEP == kSums>(L, ldl, D, grp, G, mem, r, none, part, V, jpart, w, lane, sD, sP, sV);
+    return;
+  }
+
+  const int steps = (T + LAG + R - 1) / R * R;
+  if (w == kOneWaves) {  // ---- together: the wave that exchanges V
+    const bool one = G == 1 || __builtin_amdgcn_readfirstlane(lane == 0 ? one_together(gate + grp, G, looks) : 0);
+    if (lane == 0) sTask = one ? 0 : -1;
+    lds_barrier();  // D is there
+    lds_barrier();  // parts of the first vector
+    if (one) {
+      for (int s = 0; s < steps; ++s) {
+        double v[ND] = {};
+        if (G > 1 && s < T && lane < ND)
+          one_publish(sP[0][s % R][lane], part + ((grp + int64_t(s) * ngrp) * G + mem) * ND + lane);
+        const int64_t J = grp + int64_t(s - LAG) * ngrp;
+        const bool have = s >= LAG && s - LAG < T;
+        if (have && G == 1) {
+#pragma unroll
+          for (int d = 0; d < ND; ++d) v[d] = sum_waves(sP[0][(s - LAG) % R][d]);
+        }
+        if (have && G > 1)  // the others run: their parts come
+          one_total<ND>(one_collect(part + J * G * ND, G * ND, lane, waits), lane, v);
+        if (lane == 0) {
+#pragma unroll
+          for (int d = 0; d < ND; ++d) sV[0][s & 1][d] = v[d];
+          if (mem == 0 && have) {
+#pragma unroll
+            for (int d = 0; d < ND; ++d) V[J * ND + d] = v[d];
           }
         }
-        if (m == kSums) next = one_take(&g->sums);
-        sTask = next < G ? next * 4 + m : -1;
+        lds_barrier();
       }
+    }
+  } else {  // ---- together: the streaming waves
+    const int nv = __builtin_amdgcn_readfirstlane(one_rows(r.len, w));
+    v2d buf[R][ROWS], acc[ND][ROWS];
+#pragma unroll
+    for (int u = 0; u < R; ++u) one_fetch<ROWS>(L, ldl, r, u < 2 ? u : T, nv, w, lane, buf[u]);
+    one_dens<ND, ROWS>(D, ldl, r, nv, w, lane, sD);
+#pragma unroll
+    for (int d = 0; d < ND; ++d)
+#pragma unroll
+      for (int i = 0; i < ROWS; ++i) acc[d][i] = v2d{0.0, 0.0};
+    lds_barrier();
+    auto parts = [&](int s, const v2d(&x)[ROWS]) {
+#pragma unroll
+      for (int d = 0; d < ND; ++d) sP[0][s % R][d][w] = one_dot<ROWS>(x, sD[d], kWave * w + lane);  // the same in every lane
+    };
+    parts(0, buf[0]);
+    lds_barrier();
+    // step s: vector s + 2 on its way, parts of s + 1, V of s - LAG
+    auto step = [&](int s, v2d(&cur)[ROWS], v2d(&nxt)[ROWS], v2d(&far)[ROWS]) {
+      __builtin_amdgcn_sched_barrier(0);  // `far` has been used before it is loaded again
+      one_fetch<ROWS>(L, ldl, r, s + 2, nv, w, lane, far);
+      __builtin_amdgcn_sched_barrier(0);
+      parts(s + 1, nxt);
+      lds_barrier();
+      one_add<ND, ROWS>(cur, sV[0][s & 1], acc);
+    };
+    if (__builtin_amdgcn_readfirstlane(sTask) >= 0) {
+      for (int s = 0; s < steps; s += R) {  // steps of zeros at both ends
+#pragma unroll
+        for (int u = 0; u < R; ++u) step(s + u, buf[(u + 3) % R], buf[(u + 1) % R], buf[(u + 2) % R]);
+      }
+      one_store<ND, ROWS>(acc, ldl, grp, r, nv, w, lane, jpart);
+    }
+  }
+  if (__builtin_amdgcn_readfirstlane(sTask) >= 0) return;
+
+  // ---- apart: a run of a slice's parts, or a slice for J, as they come
+  const int runs = max(1, min(kOneRuns, T / kOneRunLeast)), per = (T + runs - 1) / runs;
+  for (int mode = kTogether;;) {
+    lds_barrier();  // everybody has read sTask
+    if (w == kOneWaves && lane == 0) {
+      OneGate *g = gate + grp;
+      int next = 0, m = mode;
+      if (m == kParts) one_take(&g->done);
+      if (m != kSums) {
+        m = kParts;
+        next = one_take(&g->parts);
+        if (next >= G * runs) {
+          // runs not done are being worked on, and nothing is waited for there
+          for (int left = waits; left > 0; --left) {
+            if (__hip_atomic_load(&g->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= G * runs) break;
+            __builtin_amdgcn_s_sleep(8);
+          }
+          m = kSums;
+        }
+      }
+      if (m == kSums) next = one_take(&g->sums);
+      sTask = m == kParts || next < G ? next * 4 + m : -1;
     }
     lds_barrier();
     const int task = __builtin_amdgcn_readfirstlane(sTask);
     if (task < 0) return;
-    mem = task >> 2;
     mode = task & 3;
-    lds_barrier();  // everybody has read sTask
+    const int k = task >> 2;
+    int ln = lane;
+    asm volatile("" : "+v"(ln));  // nothing of the slices is prepared before the loop
+    if (mode == kParts)
+      one_slice<ND, ROWS, false>(L, ldl, D, grp, G, k / runs, run(k / runs, k % runs * per, max(0, min(per, T - k % runs * per))),
+                                 waits, part, V, jpart, w, ln, sD, sP, sV);
+    else
+      one_slice<ND, ROWS, true>(L, ldl, D, grp, G, k, run(k, 0, T), waits, part, V, jpart, w, ln, sD, sP, sV);
   }
 }
 
@@ -871,23 +1008,20 @@ int coulomb_run(Context *c, Scratch &s, int32_t nd, const double *dlt, int64_t l
     if ((rc = take(c, s, c->w->jpart, p.bytes_jpart, &jpart))) return rc;
     const dim3 grid(unsigned(p.ngrp * p.group)), block((kOneWaves + 1) * kWave);
     OneGate *gate = reinterpret_cast<OneGate *>(vpart + p.nparts);
-    auto one = [&](OneStep step, int phase) {
+    auto one = [&](auto kernel, int phase) {
       phase_begin(c);
-      if (nd == 1)
-        hipLaunchKernelGGL((k_coulomb_one<1, one_rows_max(1)>), grid, block, 0, c->stream, c->L, ldl, M, Dp, p.ngrp,
-                           p.group, p.slice, c->coulomb_looks, c->coulomb_waits, step, gate, vpart, V, jpart);
-      else
-        hipLaunchKernelGGL((k_coulomb_one<2, one_rows_max(2)>), grid, block, 0, c->stream, c->L, ldl, M, Dp, p.ngrp,
-                           p.group, p.slice, c->coulomb_looks, c->coulomb_waits, step, gate, vpart, V, jpart);
+      hipLaunchKernelGGL(kernel, grid, block, 0, c->stream, c->L, ldl, M, Dp, p.ngrp, p.group, p.slice, c->coulomb_looks,
+                         c->coulomb_waits, gate, vpart, V, jpart);
       phase_end(c, phase);
     };
+    constexpr int R1 = one_rows_max(1), R2 = one_rows_max(2);
     // The fixed buffer may be written by an overlapping call, so nothing is waited for
     // in it: two reads of the vectors, the same bits.
     if (s.arena && p.group > 1) {
-      one(kParts, MJK_PHASE_COULOMB_V);
-      one(kSums, MJK_PHASE_COULOMB_J);
+      one(nd == 1 ? k_coulomb_one<1, R1, kParts> : k_coulomb_one<2, R2, kParts>, MJK_PHASE_COULOMB_V);
+      one(nd == 1 ? k_coulomb_one<1, R1, kSums> : k_coulomb_one<2, R2, kSums>, MJK_PHASE_COULOMB_J);
     } else {
-      one(kTogether, MJK_PHASE_COULOMB_J);
+      one(nd == 1 ? k_coulomb_one<1, R1, kTogether> : k_coulomb_one<2, R2, kTogether>, MJK_PHASE_COULOMB_J);
     }
     phase_begin(c);
     hipLaunchKernelGGL(k_reduce_j, dim3(unsigned(ceil_div(c->np, 64)), unsigned(nd)), dim3(256), 0, c->stream, jpart,
