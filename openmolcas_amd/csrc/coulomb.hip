@@ -879,7 +879,7 @@ void plan_j_stream(const Context *c, int nd, CoulombPlan *p) {
 // Rows of 1024 pairs per workgroup of the one-pass kernel (register budget: four
 // vectors and the J of each density, three waves per SIMD).
 constexpr int one_rows_max(int nd) { return nd == 1 ? 6 : 5; }
-constexpr int kOneGrid = 256;  // workgroups: one per CU
+constexpr int kOneGrid = 256;  // workgroups at most: one per CU, as many as there are
 
 // The one-pass kernel takes one or two densities from 8192 pairs on (n = 131, 524
 // vectors: 34 us, 38 in two passes; n = 110: 36 against 31, the members' meeting is not
@@ -895,10 +895,11 @@ bool plan_one(const Context *c, int nd, CoulombPlan *p) {
   const int64_t M = c->nchol, ldl = c->ldl;
   if (nd > 2 || ldl < 8192) return false;
   const int64_t gmin = ceil_div(ldl, kOneRow * one_rows_max(nd));
-  if (gmin > kOneGrid / 2 || gmin * nd > 256) return false;
+  const int64_t grid = std::min(kOneGrid, c->ncu);
+  if (gmin > grid / 2 || gmin * nd > 256) return false;
   const int64_t want = std::max<int64_t>({M / 8, std::min<int64_t>(M / 2, 32), 1});
-  const int64_t ngrp = std::min<int64_t>(kOneGrid / gmin, want);
-  const int64_t slice = round_up(ceil_div(ldl, std::min<int64_t>(kOneGrid / ngrp, 256 / nd)), 2 * kWave);
+  const int64_t ngrp = std::min<int64_t>(grid / gmin, want);
+  const int64_t slice = round_up(ceil_div(ldl, std::min<int64_t>(grid / ngrp, 256 / nd)), 2 * kWave);
   const int64_t group = ceil_div(ldl, slice);
   if ((M * (group + 1) + (ngrp + 1) * ldl) * nd * sizeof(double) > kScratchBytes - 65536) return false;
   p->ngrp = int(ngrp);
