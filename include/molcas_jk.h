@@ -130,7 +130,10 @@ int mjk_set_stream(mjk_context *ctx, void *hip_stream);
  * run the ladder. */
 int mjk_set_ladder(mjk_context *ctx, int64_t j_fp32, int64_t j_bf16);
 
-/* Bytes of device memory one chunk of half-transformed vectors may use. */
+/* Bytes of device memory one chunk of half-transformed vectors may use (16 GiB
+ * by default).  The FP64 exchange's partial tiles keep within a sixteenth of it,
+ * the buffers of the batches that LK screening takes together within it and
+ * 1 GiB. */
 int mjk_set_x_budget(mjk_context *ctx, int64_t bytes);
 
 /* ---- vector store (src/cholesky_util vector API) ----------------------- */
@@ -404,8 +407,9 @@ int mjk_cho_lk_casscf_sym(mjk_context *ctx, int32_t nsym, const int32_t *nbas,
 /* ---- device engine (device pointers, asynchronous on the context stream) */
 
 /* Coulomb for nd folded LT densities dlt(d*ldd + p): jlt(d*ldj + p) =
- * sum_J L^J_p V_J(d), V_J(d) = sum_q L^J_q dlt(d,q); two streaming passes over
- * the resident vectors.  v_out (optional, M x nd) receives V.
+ * sum_J L^J_p V_J(d), V_J(d) = sum_q L^J_q dlt(d,q); the resident vectors are
+ * read once for both (one or two densities of 8192 to 786432 pairs) or once
+ * for each.  v_out (optional, M x nd) receives V.
  * Replaces the DGEMV pair of src/fock_util/cho_fscf.F90:208,215. */
 int mjk_coulomb(mjk_context *ctx, int32_t nd, const double *dlt, int64_t ldd,
                 double *jlt, int64_t ldj, double *v_out);
